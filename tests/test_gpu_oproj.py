@@ -85,6 +85,54 @@ def test_o_proj_f16_attention_output(cuda, oracle, B):
     assert err <= TOL
 
 
+@pytest.mark.parametrize("att16", [False, True], ids=["f32att", "f16att"])
+@pytest.mark.parametrize("B,hidden,qdim", [
+    (16, 896, 896), (17, 40, 264), (33, 1000, 4104), (63, 48, 4200),  # rows kernel: 16-token blocks, ragged K, two rounds
+    (65, 300, 72), (250, 1100, 40),       # 64 x 64 tiles, fewer K steps than LDS stages
+    (520, 1540, 360),                     # 64 x 128 tiles (f16 too), partial in both directions
+    (1030, 3100, 136),                    # 128 x 128 (f16) / 64 x 128 (f32) tiles
+    (2050, 3330, 200),                    # 128 x 256 tiles
+    (3600, 4000, 104),                    # 256 x 256 tiles (f16)
+])
+def test_o_proj_tile_edges(cuda, B, hidden, qdim, att16):
+    """Every kernel and tile of the dispatch at sizes that leave partial tiles,
+    partial K steps and a K shorter than the pipeline, against float64.  Bound:
+    qdim products of |w att| accumulate in fp32 (each addition within 2^-24 of
+    the running sum) and the split of f32 att leaves 2^-22 of each product, so
+    the error stays under (qdim 2^-24 + 2^-22) sum |w att| + 2^-23 |x|."""
+    from yllm_amd.attention import o_proj
+
+    g = torch.Generator(device="cuda").manual_seed(B)
+    att = torch.randn(B, qdim, generator=g, device=cuda) * 0.5
+    att = att.half() if att16 else att
+    w = (torch.randn(hidden, qdim, generator=g, device=cuda) * qdim ** -0.5).half()
+    x0 = torch.randn(B, hidden + 8, generator=g, device=cuda)
+    x = x0.clone()
+    o_proj(x[:, :hidden], att, w)
+    want = x0[:, :hidden].double() + att.double() @ w.double().t()
+    bound = (qdim * 2.0 ** -24 + 2.0 ** -22) * (att.double().abs() @ w.double().abs().t()) \
+        + 2.0 ** -23 * want.abs() + 2.0 ** -23 * x0[:, :hidden].double().abs()
+    assert ((x[:, :hidden].double() - want).abs() <= bound).all()
+    assert torch.equal(x[:, hidden:], x0[:, hidden:])
+
+
+@pytest.mark.parametrize("att16", [False, True], ids=["f32att", "f16att"])
+def test_o_proj_rows_too_far_apart_for_a_tile(cuda, att16):
+    """att rows 2^22 elements apart: a tile's 32-bit offsets do not reach, the
+    one-pass kernel takes the tokens eight at a time."""
+    from yllm_amd.attention import o_proj
+
+    B, hidden, qdim, stride = 11, 72, 64, 1 << 22
+    g = torch.Generator(device="cuda").manual_seed(5)
+    att = torch.zeros(B, stride, dtype=torch.float16 if att16 else torch.float32, device=cuda)[:, :qdim]
+    att.copy_(torch.randn(B, qdim, generator=g, device=cuda) * 0.5)
+    w = (torch.randn(hidden, qdim, generator=g, device=cuda) * qdim ** -0.5).half()
+    x = torch.randn(B, hidden, generator=g, device=cuda)
+    want = x.double() + att.double() @ w.double().t()
+    o_proj(x, att, w)
+    assert float((x.double() - want).norm() / want.norm()) <= 1e-6
+
+
 def test_o_proj_strided_rows_and_repeat(cuda, oracle):
     """att and x as slices of wider rows; a second call adds again (x is the
     residual stream, updated in place); a smaller batch after a larger one."""

@@ -11,14 +11,17 @@
 //    inputs each (16-byte weight loads at f16), eight iterations of loads in
 //    flight (all of a 4096-wide row), then a shuffle reduction and the
 //    residual add.
+//  * 9 to kRowsMax tokens with f16 weights (the engine's 64-token prefill calls):
+//    oproj_rows_kernel streams W_o through MFMA, a workgroup per 16 output
+//    rows and its waves splitting the contraction.
 //  * More tokens: oproj_gemm_kernel, an f16 MFMA GEMM with f32 accumulation
-//    and the residual add in its epilogue.  f16 att: one product.  f32 att
-//    with f16 weights: att is split into f16 hi + lo parts (hi = f16(att),
-//    lo = f16(att - hi)) and both products accumulate in the same registers,
-//    which keeps about 22 bits of each activation; attention outputs are
-//    convex combinations of f16 V rows (times a gate <= 1), so |att| <= 65504
-//    and hi never overflows.  f32 weights: the weights are split the same
-//    way and hi.Whi + lo.Whi + hi.Wlo accumulate.
+//    and the residual add in its epilogue.
+// In both MFMA kernels f32 att enters as f16 hi + lo parts (hi = f16(att),
+// lo = f16(att - hi)), split in registers as the fragments are read, and both
+// products accumulate in the same registers, which keeps about 22 bits of
+// each activation; attention outputs are convex combinations of f16 V rows
+// (times a gate <= 1), so |att| <= 65504 and hi never overflows.  f32 weights
+// are split the same way and hi.Whi + lo.Whi + hi.Wlo accumulate.
 #include "common.hpp"
 #include "internal.hpp"
 
@@ -26,7 +29,12 @@
 namespace yhip {
 namespace {
 
-constexpr uint32_t kRows = 2;  // output rows per wave
+constexpr uint32_t kRows = 2;  // output rows per wave of the GEMV
+// Up to this many tokens (f16 weights) the rows kernel, above it the GEMM: at
+// 64 tokens 3584 x 3584 takes 19 us against 32 (f32 att) and 16 against 29
+// (f16), at 96 tokens (two passes over the weights) 38 against 31 and 28
+// against 25.
+constexpr uint32_t kRowsMax = 64;
 
 template <int W_F16, int A_F16, int NB>
 __global__ __launch_bounds__(256) void oproj_gemv_kernel(OProjArgs a)
@@ -110,52 +118,19 @@ __global__ __launch_bounds__(256) void oproj_gemv_kernel(OProjArgs a)
     }
 }
 
-// f32 rows -> f16 hi and lo parts, hi = f16(v), lo = f16(v - hi), each a
-// contiguous [rows][cols] matrix
-__global__ __launch_bounds__(256) void oproj_split_kernel(_Float16* hi, _Float16* lo, const float* src,
-                                                          uint32_t src_stride, uint32_t rows, uint32_t cols)
+constexpr int kBK = 32;  // K per step of the MFMA kernels
+
+// 16-byte chunk swizzle (XOR into the chunk index) of an LDS row of 32 k.
+// Rows of 4 chunks (f16, 64 bytes): 8 consecutive rows hit 8 distinct bank
+// groups (32 banks, b128 reads in groups of 8 lanes), and 16 consecutive rows
+// 16 (64 banks, groups of 16 lanes).  Rows of 8 chunks (f32, 128 bytes): 8
+// consecutive rows hit 8 distinct chunk columns, 16 rows each half of a
+// 256-byte window 8.  Both depend on bits 0..3 of the row only.
+template <bool F32>
+__device__ inline int row_swz(int r)
 {
-    const uint64_t idx = (uint64_t)blockIdx.x * 256u + threadIdx.x;
-    if (idx >= (uint64_t)rows * cols) return;
-    const uint32_t r = (uint32_t)(idx / cols), i = (uint32_t)(idx % cols);
-    const float v = src[(size_t)r * src_stride + i];
-    const _Float16 h = (_Float16)v;
-    hi[idx] = h;
-    lo[idx] = (_Float16)(v - (float)h);
+    return F32 ? (r & 7) ^ ((r >> 3) & 1) : ((r >> 1) ^ (r >> 2)) & 3;
 }
-
-// ---- the GEMM: x[t][o] += sum_k T[t][k] * O[o][k] over nseg K segments ----
-//
-// T (tokens, the MFMA A operand) and O (W_o rows, the B operand) are f16
-// rows with K innermost; segment s multiplies T_s by O_s over k in [0, K)
-// (f32 attention: T_s = hi, lo against O_s = W, W; f32 weights: T_s = hi,
-// lo, hi against O_s = Whi, Whi, Wlo), so the hi + lo products accumulate in
-// registers and x is read and written once.
-//
-// A workgroup (4 waves, 2 x 2) owns BT tokens x BO outputs; a wave owns
-// (TM x 32) x (TN x 32) of them in TM x TN v_mfma_f32_32x32x16_f16
-// accumulators.  K advances 32 at a time through LDS: both tiles go from HBM
-// straight into LDS (buffer loads with the LDS destination, 16 bytes per
-// lane), rows of 64 bytes with XOR-swizzled 16-byte chunks so the fragment
-// reads are free of bank conflicts, in three stages: the tiles of the next
-// two steps load while this step's MFMAs run.  Output: lane l holds output
-// o = l % 32 of its 32 x 32 block and 16 tokens; the residual add is a float
-// atomic add per element at L2 (one add per element, so the result is the
-// load, add and store's), which keeps x's read off the kernel's tail.
-struct GemmArgs {
-    const _Float16* t[3];  // token rows, ld t_ld (elements)
-    const _Float16* o[3];  // output rows (W_o), ld K
-    float* x;
-    uint32_t t_ld, x_stride, N, M, K, nseg;
-};
-
-constexpr int kBK = 32;     // K per step: rows of 4 chunks of 16 bytes
-constexpr int kStages = 3;  // LDS stages: the loads of 2 steps ahead are in flight
-
-// 16-byte chunk swizzle of a 64-byte LDS row: 8 consecutive rows hit 8
-// distinct bank groups (32 banks, b128 reads in groups of 8 lanes), and 16
-// consecutive rows 16 (64 banks, groups of 16 lanes)
-__device__ inline int gemm_swz(int r) { return ((r >> 1) ^ (r >> 2)) & 3; }
 
 // s_waitcnt vmcnt(n), no wait on the other counters
 template <int N>
@@ -171,28 +146,264 @@ __device__ inline f32x16 mfma32(const f16x8& a, const f16x8& b, const f32x16& c)
 }
 
 // one 16-byte HBM -> LDS load per lane (lane i writes at lds + 16 i)
-__device__ inline void gemm_lds_load16(__amdgpu_buffer_rsrc_t r, _Float16* lds, int voff)
+__device__ inline void lds_load16(__amdgpu_buffer_rsrc_t r, char* lds, uint32_t voff, uint32_t soff)
 {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, (int)voff, (int)soff,
+                                             0, 0);
 }
 
-template <int TM, int TN>
-__global__ __launch_bounds__(256, 2) void oproj_gemm_kernel(GemmArgs a)
+__device__ inline __amdgpu_buffer_rsrc_t rsrc_of(const char* p, uint32_t bytes)
 {
-    constexpr int BT = 2 * TM * 32, BO = 2 * TN * 32;  // workgroup tile
-    constexpr int ROWS = BT + BO;                       // LDS rows per stage (128 B each)
-    constexpr int CPR = kBK / 8;                         // chunks per row
-    constexpr int NLD = ROWS * CPR / 256;               // 16-byte loads per thread per step
-    constexpr int NLD_T = BT * CPR / 256;               // of which token rows
-    static_assert(BT * CPR % 256 == 0 && BO * CPR % 256 == 0, "whole load instructions per operand");
-    __shared__ __attribute__((aligned(16))) _Float16 lds[kStages * ROWS * kBK];
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p), 0, (int)bytes, 0x00020000);
+}
+
+constexpr uint32_t kOutside = 0xfffffff0u;  // a buffer offset past every operand: reads zeros
+
+// 8 consecutive k of an operand row as an MFMA fragment: f16 as it is, f32 as
+// hi = f16(v) and lo = f16(v - hi)
+template <bool F32>
+struct Raw {
+    f16x8 h;
+};
+template <>
+struct Raw<true> {
+    f32x4 v[2];
+};
+template <bool F32>
+__device__ inline void split_raw(const Raw<F32>& raw, f16x8& hi, f16x8& lo)
+{
+    if constexpr (F32) {
+        // v - hi is exact, as the multiply-add -1 hi + v too, which takes hi as
+        // f16 and can round to f16 in one instruction; the factor is opaque or
+        // the compiler would turn it back into widen, subtract, convert (4
+        // instead of 2 instructions per element: the rows kernel at 64 tokens
+        // 3584 x 3584 took 20.6 us with that, 18.7 without)
+        float m1 = -1.0f;
+        asm("" : "+s"(m1));
+        typedef float f32x2 __attribute__((ext_vector_type(2)));
+        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+            const f32x2 v = {raw.v[j / 4][j % 4], raw.v[j / 4][j % 4 + 1]};
+            const f16x2 h = __builtin_convertvector(v, f16x2);
+            hi[j] = h[0];
+            hi[j + 1] = h[1];
+            lo[j] = (_Float16)__builtin_fmaf((float)h[0], m1, v[0]);
+            lo[j + 1] = (_Float16)__builtin_fmaf((float)h[1], m1, v[1]);
+        }
+    } else {
+        hi = raw.h;
+    }
+}
+
+// ---- few tokens: x[t][o] += sum_k att[t][k] W[o][k] for at most 16 NT tokens ----
+//
+// Bound by streaming W_o once (3584 x 3584: 25.7 MB, ~5 us) and by the token
+// rows, which every workgroup reads whole from L2 (64 f32 tokens: 0.9 MB per
+// workgroup at 64 bytes per cycle and CU).  A workgroup owns 16 output rows,
+// so hidden / 16 workgroups cover the chip (224 of 256 CUs at 3584), and its 8
+// waves split the contraction: each takes a run of 32-k steps, loads the W
+// fragments of 16 steps into registers at once (all of a 4096-wide row: one
+// HBM round trip) and walks its steps with the token rows coming through its
+// own LDS ring (direct-to-LDS loads, kDep steps deep, no barrier: a wave
+// reads only what it loaded).  Read straight into registers, a token
+// fragment's load instruction would touch 16 rows, a quarter of the lines'
+// rate; through LDS it covers whole 128-byte rows.  The waves' sums meet in LDS in
+// wave order, so the result does not depend on timing.  3584 x 3584, us for 64
+// / 32 / 16 f32 tokens: 18.7 / 14.4 / 12.0; the 64 x 64 GEMM tiles before it
+// (56 workgroups, 224 steps each, and a launch to split att) took 79.
+template <int NT, bool AF32>
+__global__ __launch_bounds__(512, 1) void oproj_rows_kernel(OProjArgs a)
+{
+    constexpr int EB = AF32 ? 4 : 2, CPR = kBK * EB / 16;  // bytes per element, chunks per row of 32 k
+    constexpr int SB = NT * 16 * kBK * EB;                 // bytes of a stage: 16 NT rows
+    constexpr int NLD = SB / 1024;                         // loads per lane and step
+    constexpr int kDep = 8 * 2 * SB > 65536 ? 2 : 4;       // ring depth: at most 128 KB over the 8 waves
+    constexpr int RW = 16;                                 // steps per round
+    __shared__ __attribute__((aligned(16))) char ring[8][kDep][SB];
+    static_assert(sizeof(ring) >= 8 * NT * 1024, "the reduction reuses the ring");
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    const uint32_t o0 = blockIdx.x * 16u, nt = a.B;
+
+    // this thread's part of the output: token 16 (tid / 64) + 4 g + i, row o0 + r16
+    const uint32_t ot = 16u * wave + 4u * g, oo = o0 + r16;
+    float xv[4];
+    if (wave < NT) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            xv[i] = a.x[(size_t)min(ot + i, nt - 1) * a.x_stride + min(oo, a.hidden - 1)];
+    }
+
+    const uint32_t K = a.qdim, ksteps = (K + kBK - 1) / kBK, per = (ksteps + 7) / 8;
+    const uint32_t s0 = wave * per, n = s0 < ksteps ? min(per, ksteps - s0) : 0;
+    // operands of this workgroup: 16 W rows, the tokens' rows
+    const char* wp = reinterpret_cast<const char*>(a.w) + (size_t)o0 * K * 2;
+    const char* tp = reinterpret_cast<const char*>(a.att);
+    const uint32_t wbytes = min(16u, a.hidden - o0) * K * 2u;
+    const uint32_t tbytes = ((nt - 1) * a.att_stride + K) * EB;
+    const uint32_t woff = (r16 * K + 8u * g) * 2u;
+    // load u of a step covers rows 64 u / CPR ..; at 8 rows per load the even and odd loads differ in bit 3 of the
+    // row, hence in the swizzled chunk: tk is that chunk's first k
+    uint32_t tk[2], toff[NLD];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) tk[p] = ((lane % CPR) ^ row_swz<AF32>((64 * p + lane) / CPR & 15)) * (16u / EB);
+#pragma unroll
+    for (int u = 0; u < NLD; ++u) toff[u] = ((64u * u + lane) / CPR * a.att_stride + tk[u & 1]) * EB;
+
+    f32x4 acc[NT];
+#pragma unroll
+    for (int b = 0; b < NT; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    for (uint32_t r0 = 0; r0 < n; r0 += RW) {
+        // step i of the round covers k0 .. k0 + 31; past this wave's steps and past K every load reads zeros
+        auto k0_of = [&](int i) { return (s0 + r0 + i) * kBK; };
+        auto issue = [&](int i) {
+            const bool in = r0 + i < n;
+            const __amdgpu_buffer_rsrc_t rt = rsrc_of(tp, in ? tbytes : 0u);
+            const uint32_t k0 = in ? k0_of(i) : 0u;
+#pragma unroll
+            for (int u = 0; u < NLD; ++u) {
+                lds_load16(rt, ring[wave][i % kDep] + u * 1024, k0 + tk[u & 1] < K ? toff[u] : kOutside, k0 * EB);
+            }
+        };
+        f16x8 w[RW];
+#pragma unroll
+        for (int i = 0; i < RW; ++i) {
+            const bool in = r0 + i < n;
+            const uint32_t k0 = in ? k0_of(i) : 0u;
+            const uint32_t off = k0 + 8u * g < K ? woff : kOutside;
+            // read once per call: non-temporal
+            w[i] = __builtin_bit_cast(f16x8, __builtin_amdgcn_raw_buffer_load_b128(rsrc_of(wp, in ? wbytes : 0u), (int)off,
+                                                                                   (int)(k0 * 2u), 2));
+        }
+#pragma unroll
+        for (int i = 0; i < kDep; ++i) issue(i);
+#pragma unroll
+        for (int i = 0; i < RW; ++i) {
+            if (i % 4 == 0 && r0 + i >= n) break;  // uniform over the wave
+            constexpr int last = RW - 1;
+            // this step's rows have landed; later steps' loads may stay in flight
+            switch (last - i < kDep - 1 ? last - i : kDep - 1) {
+            case 0: wait_vm<0>(); break;
+            case 1: wait_vm<NLD>(); break;
+            case 2: wait_vm<2 * NLD>(); break;
+            default: wait_vm<3 * NLD < 64 ? 3 * NLD : 63>(); break;
+            }
+            asm volatile("" ::: "memory");
+            Raw<AF32> raw[NT];
+#pragma unroll
+            for (int b = 0; b < NT; ++b) {
+                const char* row = ring[wave][i % kDep] + (16 * b + r16) * (kBK * EB);
+                if constexpr (AF32) {
+                    raw[b].v[0] = *reinterpret_cast<const f32x4*>(row + ((2 * g) ^ row_swz<AF32>(r16)) * 16);
+                    raw[b].v[1] = *reinterpret_cast<const f32x4*>(row + ((2 * g + 1) ^ row_swz<AF32>(r16)) * 16);
+                } else {
+                    raw[b].h = *reinterpret_cast<const f16x8*>(row + (g ^ row_swz<AF32>(r16)) * 16);
+                }
+            }
+            if (i + kDep < RW) {
+                __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the reads are done, the stage may be overwritten
+                asm volatile("" ::: "memory");
+                issue(i + kDep);
+            }
+#pragma unroll
+            for (int b = 0; b < NT; ++b) {
+                f16x8 hi, lo;
+                split_raw<AF32>(raw[b], hi, lo);
+                acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, w[i], acc[b], 0, 0, 0);
+                if (AF32) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, w[i], acc[b], 0, 0, 0);
+            }
+        }
+        wait_vm<0>();  // nothing in flight into the ring before it is used again
+    }
+    __syncthreads();
+    f32x4* red = reinterpret_cast<f32x4*>(&ring[0][0][0]);  // [wave][block][lane]
+#pragma unroll
+    for (int b = 0; b < NT; ++b) red[(wave * NT + b) * 64 + lane] = acc[b];
+    __syncthreads();
+    if (wave >= NT) return;
+    f32x4 sum = red[wave * 64 + lane];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) sum += red[(w * NT + wave) * 64 + lane];
+    if (oo < a.hidden) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (ot + i < nt) a.x[(size_t)(ot + i) * a.x_stride + oo] = xv[i] + sum[i];
+    }
+}
+
+// ---- the GEMM: x[t][o] += sum_k T[t][k] * W[o][k] ----
+//
+// T (tokens, the MFMA A operand) and W (W_o rows, the B operand) are f16 or
+// f32 rows with K innermost.  A workgroup (4 waves, WT x WO) owns BT tokens x
+// BO outputs; a wave owns (TM x 32) x (TN x 32) of them in TM x TN
+// v_mfma_f32_32x32x16_f16 accumulators.
+//
+// The bound is the matrix pipe, and next to it the LDS: a 32 x 32 x 16 MFMA
+// takes 32 cycles, in which the four SIMDs can take 4 KB of operands from a
+// 128-byte-per-cycle LDS, tile writes included.  A wave of 128 x 128 (f16, one
+// wave per SIMD) reads 8 fragments for 16 MFMAs and its workgroup writes 32 KB
+// per 128 MFMAs: 0.75 KB per MFMA, where 64 x 128 waves took 1.13 KB, over
+// the limit.  With f32 tokens the hi and lo products share the W fragment: 64
+// x 128 waves read 4 + 4 (f32 fragments are two reads) for 16 MFMAs.
+//
+// K advances 32 at a time through four LDS stages; both tiles go from HBM
+// straight into LDS (16 bytes per lane) in XOR-swizzled rows.  With one wave
+// per SIMD nothing else covers a wave's waits, so the loop is pipelined across
+// the barrier: a step's first half issues its MFMAs while the second half's
+// fragments are read; then the barrier, which says that the stage is read
+// and the next one (loaded three steps ago) has landed; then the second
+// half's MFMAs issue while the next step's first fragments are read and the
+// loads four steps ahead go into the stage just read.  The four stages are
+// separate variables and the loop is unrolled by four, so the compiler sees
+// that loads in flight never alias the reads.  The residual is added with one
+// float atomic add per element at L2 (one add per element, so the result is
+// the load, add and store's), which keeps x's read off the kernel's tail.
+struct GemmArgs {
+    const char* t;  // token rows
+    const char* w;  // W_o rows, ld K
+    float* x;
+    uint32_t t_ld, x_stride, N, M, K;
+};
+
+constexpr int kStages = 4;
+
+// issue order of a half step: each of NRD fragment reads is followed by its
+// share of the NLD tile loads and of the NMF MFMAs
+template <int NRD, int NLD, int NMF, int I>
+__device__ inline void spread()
+{
+    if constexpr (I < NRD) {
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        constexpr int nl = NLD * (I + 1) / NRD - NLD * I / NRD, nm = NMF * (I + 1) / NRD - NMF * I / NRD;
+        if constexpr (nl > 0) __builtin_amdgcn_sched_group_barrier(0x020, nl, 0);
+        if constexpr (nm > 0) __builtin_amdgcn_sched_group_barrier(0x008, nm, 0);
+        spread<NRD, NLD, NMF, I + 1>();
+    }
+}
+
+template <int TM, int TN, int WT, int WO, bool AF32, bool WF32, int WPC>
+__global__ __launch_bounds__(256, WPC) void oproj_gemm_kernel(GemmArgs a)
+{
+    static_assert(WT * WO == 4, "four waves");
+    constexpr int BT = WT * TM * 32, BO = WO * TN * 32;   // workgroup tile
+    constexpr int EA = AF32 ? 4 : 2, EW = WF32 ? 4 : 2;
+    constexpr int RBA = kBK * EA, RBW = kBK * EW;          // row bytes
+    constexpr int CA = RBA / 16, CW = RBW / 16;            // chunks per row
+    constexpr int NLA = BT * CA / 256, NLW = BO * CW / 256;  // loads per thread and step
+    constexpr int NLD = NLA + NLW;
+    constexpr int SB = BT * RBA + BO * RBW;                // stage bytes
+    static_assert(BT * CA % 256 == 0 && BO * CW % 256 == 0, "whole load instructions per operand");
+    __shared__ __attribute__((aligned(16))) char S0[SB], S1[SB], S2[SB], S3[SB];
+    auto stage = [&](int s) -> char* { return s == 0 ? S0 : s == 1 ? S1 : s == 2 ? S2 : S3; };
 
     // the wave index in a scalar register: the LDS destination of a
-    // direct-to-LDS load (M0) must be uniform, and with a per-lane index the
-    // compiler wrapped every such load in a loop over the lanes' values
+    // direct-to-LDS load (M0) must be uniform
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r32 = lane & 31, hh = lane >> 5;
-    const int wt = wave >> 1, wo = wave & 1;
+    const int wt = wave / WO, wo = wave % WO;
     // Tile order: the hardware deals consecutive workgroups to the 8 XCDs in
     // turn; workgroup x takes position (x % 8) * (grid / 8) + x / 8 of the
     // order below, so each XCD works through a contiguous run of it, and the
@@ -206,49 +417,41 @@ __global__ __launch_bounds__(256, 2) void oproj_gemm_kernel(GemmArgs a)
     const uint32_t g_rows = min(4u, n_tt - grp * 4u);
     if (pid >= n_ot * n_tt) return;
     const uint32_t t0 = (grp * 4u + in_g % g_rows) * BT, o0 = (in_g / g_rows) * BO;
-    const uint32_t ksteps = (a.K + kBK - 1) / kBK, nsteps = ksteps * a.nseg;
+    const uint32_t nt = min((uint32_t)BT, a.N - t0), no = min((uint32_t)BO, a.M - o0);
+    const uint32_t K = a.K, nsteps = (K + kBK - 1) / kBK;
 
-    // per load instruction i: the LDS chunk this lane fills and its row / column
-    int goff[NLD];  // byte offset of the chunk within its operand, k0 = 0 (0x80000000: outside)
-
+    // Offsets of this thread's chunks from the tile's first row at k 0; a row
+    // past the tile's last lies past the resource's end and reads zeros.
+    // Load i covers 256 / CA rows, a multiple of 16: the swizzle is the same
+    // for every i.
+    const int ca = (tid % CA) ^ row_swz<AF32>(tid / CA), cw = (tid % CW) ^ row_swz<WF32>(tid / CW);
+    uint32_t ta[NLA], tw[NLW];
 #pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-        const int Lc = 256 * i + 64 * wave + lane;
-        const int R = Lc / CPR, c = (Lc % CPR) ^ gemm_swz(R);
-        if (i < NLD_T) {
-            const uint32_t t = t0 + R;
-            goff[i] = (int)(t * a.t_ld * 2u + c * 16u) | (t < a.N ? 0 : (int)0x80000000);
-        } else {
-            const uint32_t o = o0 + (R - BT);
-            goff[i] = (int)(o * a.K * 2u + c * 16u) | (o < a.M ? 0 : (int)0x80000000);
-        }
-    }
-    auto rsrc = [&](const _Float16* p, uint32_t bytes) {
-        return __builtin_amdgcn_make_buffer_rsrc(const_cast<_Float16*>(p), 0, bytes, 0x00020000);
+    for (int i = 0; i < NLA; ++i) ta[i] = (256 / CA * i + tid / CA) * (a.t_ld * EA) + ca * 16u;
+#pragma unroll
+    for (int i = 0; i < NLW; ++i) tw[i] = (256 / CW * i + tid / CW) * (K * EW) + cw * 16u;
+    const char* tp = a.t + (size_t)t0 * a.t_ld * EA;
+    const char* wp = a.w + (size_t)o0 * K * EW;
+    const uint32_t tbytes = ((nt - 1) * a.t_ld + K) * EA, wbytes = no * K * EW;
+    const uint32_t ka = ca * 16u / EA, kw = cw * 16u / EW;  // k of the chunks within a step
+    // load i of step st into stage s; a step past the last and the chunks past
+    // K of a partial last step read zeros
+    struct Step {
+        __amdgpu_buffer_rsrc_t rt, rw;
+        uint32_t k0, ma, mw;
     };
-    const uint32_t t_bytes = ((a.N - 1) * a.t_ld + a.K) * 2u, o_bytes = a.M * a.K * 2u;
-    // the segments' base addresses as offsets from segment 0's, read once
-    // (indexing a.t[seg] in the loop reads the kernel arguments from memory at
-    // every step and waits for them; a select chain over the pointers went
-    // through scratch memory)
-    const uint64_t tb0 = (uint64_t)a.t[0], ob0 = (uint64_t)a.o[0];
-    const uint64_t td1 = (uint64_t)a.t[1] - tb0, td2 = (uint64_t)a.t[2] - tb0;
-    const uint64_t od1 = (uint64_t)a.o[1] - ob0, od2 = (uint64_t)a.o[2] - ob0;
-    auto issue = [&](_Float16* buf, uint32_t st) {
-        const bool past = st >= nsteps;  // workgroup-uniform
-        const uint32_t seg = past ? 0 : st / ksteps, k0 = past ? 0 : (st % ksteps) * kBK;
-        const uint64_t s1 = seg == 1, s2 = seg == 2;
-        const __amdgpu_buffer_rsrc_t rt = rsrc((const _Float16*)(tb0 + s1 * td1 + s2 * td2), t_bytes);
-        const __amdgpu_buffer_rsrc_t ro = rsrc((const _Float16*)(ob0 + s1 * od1 + s2 * od2), o_bytes);
-#pragma unroll
-        for (int i = 0; i < NLD; ++i) {
-            // a chunk past K (the last step of a K that is no multiple of 64)
-            // reads zeros, not the next row
-            const int Lc = 256 * i + 64 * wave + lane;
-            const int kc = ((Lc % CPR) ^ gemm_swz(Lc / CPR)) * 8;
-            const int off = (past || goff[i] < 0 || k0 + kc >= a.K) ? (int)0x80000000 : goff[i] + (int)k0 * 2;
-            gemm_lds_load16(i < NLD_T ? rt : ro, buf + (256 * i + 64 * wave) * 8, off);
-        }
+    auto step_of = [&](uint32_t st) {
+        const bool in = st < nsteps;  // workgroup-uniform
+        const uint32_t k0 = in ? st * kBK : 0u;
+        return Step{rsrc_of(tp, in ? tbytes : 0u), rsrc_of(wp, in ? wbytes : 0u), k0, k0 + ka < K ? 0u : kOutside,
+                    k0 + kw < K ? 0u : kOutside};
+    };
+    auto issue = [&](const Step& p, int s, int i) {
+        if (i < NLA)
+            lds_load16(p.rt, stage(s) + (256 * i + 64 * wave) * 16, ta[i < NLA ? i : 0] | p.ma, p.k0 * EA);
+        else
+            lds_load16(p.rw, stage(s) + BT * RBA + (256 * (i - NLA) + 64 * wave) * 16, tw[i < NLA ? 0 : i - NLA] | p.mw,
+                       p.k0 * EW);
     };
 
     f32x16 acc[TM][TN];
@@ -259,99 +462,137 @@ __global__ __launch_bounds__(256, 2) void oproj_gemm_kernel(GemmArgs a)
 #pragma unroll
             for (int i = 0; i < 16; ++i) acc[m][n][i] = 0.0f;
 
-    // MFMA fragments: row row0 + r32 of a stage, 16-byte chunk (2 kk + hh) ^
-    // swz(r32) (row0 is a multiple of 32, so the swizzle is r32's).  The
-    // lane's part of the address goes through an opaque move each step, so
-    // the compiler keeps one base per k chunk instead of hoisting an address
-    // per fragment out of the loop.
-    auto compute = [&](uint32_t stage) {
-        int lane_row;
-        asm volatile("v_mov_b32 %0, %1" : "=v"(lane_row) : "v"(r32 * kBK * 2 + (int)(stage * ROWS * kBK * 2)));
-        const int sw = gemm_swz(r32);
-        const char* base = reinterpret_cast<const char*>(lds) + lane_row;
-        constexpr int KK = kBK / 16;
-        f16x8 ft[2][TM], fo[2][TN];
-        auto load = [&](int kk) {
-            const char* b = base + (((2 * kk + hh) ^ sw) << 4);
-#pragma unroll
-            for (int n = 0; n < TN; ++n)
-                fo[kk & 1][n] = *reinterpret_cast<const f16x8*>(b + (BT + (wo * TN + n) * 32) * kBK * 2);
-#pragma unroll
-            for (int m = 0; m < TM; ++m)
-                ft[kk & 1][m] = *reinterpret_cast<const f16x8*>(b + ((wt * TM + m) * 32) * kBK * 2);
-        };
-        load(0);
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk) {
-            if (kk + 1 < KK) load(kk + 1);  // in flight under this k chunk's MFMAs
-#pragma unroll
-            for (int m = 0; m < TM; ++m)
-#pragma unroll
-                for (int n = 0; n < TN; ++n) acc[m][n] = mfma32(ft[kk & 1][m], fo[kk & 1][n], acc[m][n]);
+    // fragments of half kk of a stage: row r32 of each 32-row block, k 16 kk + 8 hh ..
+    struct Frags {
+        Raw<AF32> t[TM];
+        Raw<WF32> w[TN];
+    };
+    // (each address is one offset from its stage: through a chain of them the
+    // compiler loses track of the variable and waits for every load in flight)
+    const int swa = row_swz<AF32>(r32 & 15), sww = row_swz<WF32>(r32 & 15);
+    const int ra = (wt * TM * 32 + r32) * RBA, rw = BT * RBA + (wo * TN * 32 + r32) * RBW;
+    auto read_row = [&](auto& f, int s, int off, int kk, int swz) {
+        if constexpr (sizeof(f) == 32) {
+            f.v[0] = *reinterpret_cast<const f32x4*>(stage(s) + (off + (((4 * kk + 2 * hh) ^ swz) << 4)));
+            f.v[1] = *reinterpret_cast<const f32x4*>(stage(s) + (off + (((4 * kk + 2 * hh + 1) ^ swz) << 4)));
+        } else {
+            f.h = *reinterpret_cast<const f16x8*>(stage(s) + (off + (((2 * kk + hh) ^ swz) << 4)));
         }
     };
-
-    // Steps 0..kStages-2 load ahead; step st waits for its own tiles (the
-    // loads of the kStages-2 later steps may stay in flight: a count, issued
-    // in order, of NLD loads per step, every one of them issued -- past the
-    // end they read zeros), then, after the barrier that orders the last
-    // reads of stage (st-1) % kStages before it, loads step st+kStages-1 there.
+    auto read = [&](Frags& f, int s, int kk) {
 #pragma unroll
-    for (int s = 0; s < kStages - 1; ++s) issue(lds + s * ROWS * kBK, s);
-    for (uint32_t st = 0; st < nsteps; ++st) {
-        wait_vm<(kStages - 2) * NLD>();
-        lds_barrier();
-        issue(lds + ((st + kStages - 1) % kStages) * ROWS * kBK, st + kStages - 1);
-        compute(st % kStages);
+        for (int n = 0; n < TN; ++n) read_row(f.w[n], s, rw + n * 32 * RBW, kk, sww);
+#pragma unroll
+        for (int m = 0; m < TM; ++m) read_row(f.t[m], s, ra + m * 32 * RBA, kk, swa);
+    };
+    auto mma = [&](const Frags& f) {
+        f16x8 wh[TN], wl[WF32 ? TN : 1];
+#pragma unroll
+        for (int n = 0; n < TN; ++n) split_raw<WF32>(f.w[n], wh[n], wl[WF32 ? n : 0]);
+#pragma unroll
+        for (int m = 0; m < TM; ++m) {
+            f16x8 hi, lo;
+            split_raw<AF32>(f.t[m], hi, lo);
+#pragma unroll
+            for (int n = 0; n < TN; ++n) acc[m][n] = mfma32(hi, wh[n], acc[m][n]);
+            if constexpr (AF32) {
+#pragma unroll
+                for (int n = 0; n < TN; ++n) acc[m][n] = mfma32(lo, wh[n], acc[m][n]);
+            }
+            if constexpr (WF32) {
+#pragma unroll
+                for (int n = 0; n < TN; ++n) acc[m][n] = mfma32(hi, wl[n], acc[m][n]);
+            }
+        }
+    };
+    constexpr int NMF = TM * TN * (1 + AF32 + WF32);              // MFMAs per half step
+    constexpr int NRD = TM * (AF32 ? 2 : 1) + TN * (WF32 ? 2 : 1);  // fragment reads per half step
+
+    Frags f0, f1;
+#pragma unroll
+    for (int s = 0; s < kStages; ++s) {
+        const Step p = step_of(s);
+#pragma unroll
+        for (int i = 0; i < NLD; ++i) issue(p, s, i);
+    }
+    wait_vm<(kStages - 1) * NLD>();
+    lds_barrier();
+    read(f0, 0, 0);
+    for (uint32_t st = 0; st < nsteps; st += kStages) {
+#pragma unroll
+        for (int s = 0; s < kStages; ++s) {  // step st + s; past the last its operands are zeros
+            read(f1, s, 1);
+            mma(f0);
+            spread<NRD, 0, NMF, 0>();
+            __builtin_amdgcn_sched_barrier(0);
+            wait_vm<(kStages - 2) * NLD>();  // step st + s + 1 has landed
+            lds_barrier();                   // for every wave, and every wave has read stage s
+            const Step p = step_of(st + s + kStages);
+            read(f0, (s + 1) % kStages, 0);
+#pragma unroll
+            for (int i = 0; i < NLD; ++i) issue(p, s, i);
+            mma(f1);
+            spread<NRD, NLD, NMF, 0>();
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     wait_vm<0>();  // the loads past the end land before the workgroup ends
 
     // x[t][o] += acc with float atomics at L2 (each element receives one
     // add: the result equals a load, add and store), no load of x on the way
+    float* xp = a.x + (size_t)t0 * a.x_stride + o0;
+    const uint32_t tb = wt * TM * 32 + 4 * hh, ob = wo * TN * 32 + r32;
+    const bool whole = nt == (uint32_t)BT && no == (uint32_t)BO;  // workgroup-uniform
 #pragma unroll
     for (int m = 0; m < TM; ++m)
 #pragma unroll
-        for (int n = 0; n < TN; ++n) {
-            const uint32_t o = o0 + (wo * TN + n) * 32 + r32;
+        for (int i = 0; i < 16; ++i) {
+            const uint32_t t = tb + 32 * m + 8 * (i / 4) + i % 4;
+            float* row = xp + (size_t)t * a.x_stride + ob;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const uint32_t t = t0 + (wt * TM + m) * 32 + 8 * (i / 4) + 4 * hh + (i % 4);
-                if (t < a.N && o < a.M) unsafeAtomicAdd(a.x + (size_t)t * a.x_stride + o, acc[m][n][i]);
-            }
+            for (int n = 0; n < TN; ++n)
+                if (whole || (t < nt && ob + 32u * n < no)) unsafeAtomicAdd(row + 32 * n, acc[m][n][i]);
         }
 }
 
-template <int TM, int TN>
+template <int TM, int TN, int WT, int WO, bool AF32, bool WF32, int WPC>
 hipError_t launch_gemm_tiles(const GemmArgs& a, hipStream_t st)
 {
-    constexpr uint32_t BT = 2 * TM * 32, BO = 2 * TN * 32;
+    constexpr uint32_t BT = WT * TM * 32, BO = WO * TN * 32;
     const uint32_t tiles = ((a.N + BT - 1) / BT) * ((a.M + BO - 1) / BO);
-    hipLaunchKernelGGL((oproj_gemm_kernel<TM, TN>), dim3((tiles + 7) / 8 * 8), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((oproj_gemm_kernel<TM, TN, WT, WO, AF32, WF32, WPC>), dim3((tiles + 7) / 8 * 8), dim3(256), 0,
+                       st, a);
     return hipGetLastError();
 }
 
-// Tile choice: 128 x 256 workgroup tiles for large batches, two workgroups
-// per CU (MFMA-bound; one workgroup's barrier wait is covered by the other's
-// MFMAs: 8192 x 4096 x 4096 ran 787 TFLOP/s against 771 for 256 x 256 tiles
-// at one workgroup per CU); 64 x 64 for small ones (the engine's chunks of
-// up to 64 tokens: the weights are read once and the launch is
-// bandwidth-bound, so more, smaller workgroups stream them).  Token rows are
-// launched in pieces whose byte offsets stay below 2 GiB.
-hipError_t launch_gemm(GemmArgs a, hipStream_t st)
+// Tile choice: the largest tile of which there are enough for three quarters
+// of the CUs.  A larger tile moves fewer LDS and L2 bytes per MFMA, but one
+// workgroup per CU cannot fill a chip of which it leaves a quarter idle.
+// f16 att, 4096 x 4096, us with 256 x 256 / 128 x 256 / 128 x 128 / 64 x 128 /
+// 64 x 64 tiles: 8192 tokens 320 / 359 / 372, 2048 tokens 108 / 96 / 104, 1024
+// 96 / 72 / 55 / 73 / 85, 512 - / 66 / 47 / 43 / 47, 256 - / - / 44 / 39 / 29.
+// f32 att, 3584 x 3584, 128 x 256 / 64 x 128 / 64 x 64: 2048 tokens 118 / 147,
+// 1024 90 / 76 / 99, 512 85 / 45 / 55, 256 (4096 x 4096) - / 44 / 39.
+hipError_t launch_gemm(const GemmArgs& a, bool af32, bool wf32, hipStream_t st)
 {
-    const uint64_t row_bytes = (uint64_t)a.t_ld * 2;
-    uint64_t per = ((1ull << 31) - 1 - (uint64_t)a.K * 2) / row_bytes;
-    per = per / 256 * 256;
-    const uint32_t N = a.N;
-    for (uint32_t n0 = 0; n0 < N; n0 += (uint32_t)per) {
-        GemmArgs b = a;
-        b.N = (uint32_t)(N - n0 < per ? N - n0 : per);
-        for (uint32_t s = 0; s < a.nseg; ++s) b.t[s] = a.t[s] + (size_t)n0 * a.t_ld;
-        b.x = a.x + (size_t)n0 * a.x_stride;
-        const hipError_t e = b.N > 128 ? launch_gemm_tiles<2, 4>(b, st) : launch_gemm_tiles<1, 1>(b, st);
-        if (e != hipSuccess) return e;
+    const uint64_t enough = (uint64_t)n_cus() * 3 / 4;
+    auto fits = [&](uint32_t bt, uint32_t bo) {
+        return (uint64_t)((a.N + bt - 1) / bt) * ((a.M + bo - 1) / bo) >= enough;
+    };
+    if (wf32) {
+        if (fits(128, 128)) return launch_gemm_tiles<2, 2, 2, 2, true, true, 1>(a, st);
+        return launch_gemm_tiles<1, 1, 2, 2, true, true, 2>(a, st);
     }
-    return hipSuccess;
+    if (af32) {
+        if (fits(128, 256)) return launch_gemm_tiles<2, 4, 2, 2, true, false, 1>(a, st);
+        if (fits(64, 128)) return launch_gemm_tiles<1, 2, 2, 2, true, false, 2>(a, st);
+        return launch_gemm_tiles<1, 1, 2, 2, true, false, 2>(a, st);
+    }
+    if (fits(256, 256)) return launch_gemm_tiles<4, 4, 2, 2, false, false, 1>(a, st);
+    if (fits(128, 256)) return launch_gemm_tiles<2, 4, 2, 2, false, false, 1>(a, st);
+    if (fits(128, 128)) return launch_gemm_tiles<2, 2, 2, 2, false, false, 2>(a, st);
+    if (fits(64, 128)) return launch_gemm_tiles<1, 2, 2, 2, false, false, 2>(a, st);
+    return launch_gemm_tiles<1, 1, 2, 2, false, false, 2>(a, st);
 }
 
 template <int W_F16, int A_F16>
@@ -370,6 +611,19 @@ hipError_t launch_gemv(const OProjArgs& a, hipStream_t st)
     return hipGetLastError();
 }
 
+template <bool AF32>
+hipError_t launch_rows(const OProjArgs& a, hipStream_t st)
+{
+    const uint32_t gx = (a.hidden + 15) / 16;
+    if (a.B <= 16)
+        hipLaunchKernelGGL((oproj_rows_kernel<1, AF32>), dim3(gx), dim3(512), 0, st, a);
+    else if (a.B <= 32)
+        hipLaunchKernelGGL((oproj_rows_kernel<2, AF32>), dim3(gx), dim3(512), 0, st, a);
+    else
+        hipLaunchKernelGGL((oproj_rows_kernel<4, AF32>), dim3(gx), dim3(512), 0, st, a);
+    return hipGetLastError();
+}
+
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
 }  // namespace
@@ -377,7 +631,7 @@ size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 size_t oproj_workspace(uint32_t B, uint32_t qdim, uint32_t w_f16, uint32_t att_f16, uint32_t hidden)
 {
     if (B <= kGemvRows || att_f16) return 0;
-    // f32 att as f16 hi and lo matrices; f32 weights as f16 hi and lo too
+    // What callers have had to bring for f32 operands (once their f16 parts); no kernel uses it any more.
     return 2 * align256((size_t)B * qdim * 2) + (w_f16 ? 0 : 2 * align256((size_t)hidden * qdim * 2));
 }
 
@@ -391,52 +645,36 @@ const char* launch_oproj(const OProjArgs& a, void* ws, size_t ws_bytes, hipStrea
             e = a.att_f16 ? launch_gemv<0, 1>(a, st) : launch_gemv<0, 0>(a, st);
         return e == hipSuccess ? nullptr : hipGetErrorString(e);
     }
+    (void)ws;
     (void)ws_bytes;
-    GemmArgs g = {};
-    g.x = a.x;
-    g.x_stride = a.x_stride;
-    g.N = a.B;
-    g.M = a.hidden;
-    g.K = a.qdim;
-    const _Float16* w16 = reinterpret_cast<const _Float16*>(a.w);
-    if (a.att_f16) {  // f16 weights and f16 activations: one segment
-        g.nseg = 1;
-        g.t[0] = reinterpret_cast<const _Float16*>(a.att);
-        g.t_ld = a.att_stride;
-        g.o[0] = w16;
-        const hipError_t e = launch_gemm(g, st);
-        return e == hipSuccess ? nullptr : hipGetErrorString(e);
+    // the MFMA kernels address a tile's rows with 32-bit byte offsets; rows too
+    // long for that go through the one-pass kernel, eight tokens at a time
+    const uint64_t row = 4ull * (a.att_stride > a.qdim ? a.att_stride : a.qdim);
+    if (256u * row >= 0xf0000000ull) {
+        for (uint32_t b0 = 0; b0 < a.B; b0 += kGemvRows) {
+            OProjArgs p = a;
+            p.B = a.B - b0 < kGemvRows ? a.B - b0 : kGemvRows;
+            p.x = a.x + (size_t)b0 * a.x_stride;
+            p.att = reinterpret_cast<const char*>(a.att) + (size_t)b0 * a.att_stride * (a.att_f16 ? 2 : 4);
+            if (const char* msg = launch_oproj(p, nullptr, 0, st)) return msg;
+        }
+        return nullptr;
     }
-    // f32 activations (and f32 weights): f16 hi / lo parts in the workspace
-    const size_t tpart = align256((size_t)a.B * a.qdim * 2);
-    _Float16* thi = reinterpret_cast<_Float16*>(ws);
-    _Float16* tlo = reinterpret_cast<_Float16*>(reinterpret_cast<char*>(ws) + tpart);
-    const uint64_t n = (uint64_t)a.B * a.qdim;
-    hipLaunchKernelGGL(oproj_split_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st, thi, tlo,
-                       reinterpret_cast<const float*>(a.att), a.att_stride, a.B, a.qdim);
-    g.t_ld = a.qdim;
-    if (a.w_f16) {
-        g.nseg = 2;
-        g.t[0] = thi;  // hi . W
-        g.t[1] = tlo;  // lo . W
-        g.o[0] = g.o[1] = w16;
+    hipError_t e;
+    if (a.w_f16 && a.B <= kRowsMax) {
+        e = a.att_f16 ? launch_rows<false>(a, st) : launch_rows<true>(a, st);
     } else {
-        const size_t wpart = align256((size_t)a.hidden * a.qdim * 2);
-        _Float16* whi = reinterpret_cast<_Float16*>(reinterpret_cast<char*>(ws) + 2 * tpart);
-        _Float16* wlo = reinterpret_cast<_Float16*>(reinterpret_cast<char*>(ws) + 2 * tpart + wpart);
-        const uint64_t nw = (uint64_t)a.hidden * a.qdim;
-        hipLaunchKernelGGL(oproj_split_kernel, dim3((uint32_t)((nw + 255) / 256)), dim3(256), 0, st, whi, wlo,
-                           reinterpret_cast<const float*>(a.w), a.qdim, a.hidden, a.qdim);
-        g.nseg = 3;  // hi.Whi + lo.Whi + hi.Wlo (the lo.lo term is below f32 rounding)
-        g.t[0] = thi;
-        g.t[1] = tlo;
-        g.t[2] = thi;
-        g.o[0] = whi;
-        g.o[1] = whi;
-        g.o[2] = wlo;
+        GemmArgs g = {};
+        g.t = reinterpret_cast<const char*>(a.att);
+        g.w = reinterpret_cast<const char*>(a.w);
+        g.x = a.x;
+        g.t_ld = a.att_stride;
+        g.x_stride = a.x_stride;
+        g.N = a.B;
+        g.M = a.hidden;
+        g.K = a.qdim;
+        e = launch_gemm(g, !a.att_f16, !a.w_f16, st);
     }
-    hipError_t e = hipGetLastError();
-    if (e == hipSuccess) e = launch_gemm(g, st);
     return e == hipSuccess ? nullptr : hipGetErrorString(e);
 }
 
