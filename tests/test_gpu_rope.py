@@ -117,6 +117,44 @@ def test_rope_kv_store_matches_oracle(cuda, oracle, kind, nh, nkv, d, n_rot, the
     assert (K[:, outside, :] == SENTINEL).all() and (V[:, :, outside] == SENTINEL).all()
 
 
+@pytest.mark.parametrize("kind,nh,nkv,d,n_rot,ps,B", [
+    (1, 5, 3, 64, 0, 61, 128),     # the last scatter size
+    (2, 7, 1, 128, 0, 61, 129),    # the first with V tile blocks, three of them for 129 rows
+    (3, 3, 1, 256, 64, 64, 129),
+    (2, 9, 3, 64, 0, 7, 1400),     # an odd number of passes, several per wave
+    (1, 29, 4, 128, 0, 1, 1100),   # 33 passes in waves of 8
+    (3, 16, 2, 256, 64, 0, 2500),  # 18 passes in waves of 4
+])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_rope_v_tiles_and_pass_split(cuda, oracle, kind, nh, nkv, d, n_rot, ps, B, aligned):
+    """Around the change from scattered V to tile blocks and over the splits of
+    a token's heads, with a V cache that takes 16-byte stores and one that does
+    not; bounds as in test_rope_kv_store_matches_oracle."""
+    from yllm_amd.attention import LayerKV, rope_kv_store
+
+    x, q, k, v = fused_rows(1500 + B, B, nh, nkv, d)
+    pos = np.arange(ps, ps + B)
+    th = np.float32(1e6)
+    cache = sentinel_cache(cuda, nkv, d, ps + B + 70)
+    if not aligned:
+        buf = torch.full((cache.v.numel() + 8,), SENTINEL, dtype=torch.int16, device=cuda).view(torch.float16)
+        cache = LayerKV(cache.k, buf[2:2 + cache.v.numel()].view(cache.v.shape))
+        assert cache.v.data_ptr() % 16 == 4
+    xt = torch.from_numpy(x).to(cuda)
+    qd, kvd = nh * d, nkv * d
+    got_q = rope_kv_store(cache, xt[:, :qd], xt[:, qd:qd + kvd], xt[:, qd + kvd:], ps, nh, kind, float(th),
+                          n_rot=n_rot).cpu().numpy()
+    assert np.abs(got_q - oracle.rope(q, pos, d, th, kind, n_rot)).max() <= 4e-6 * max(1.0, float(np.abs(q).max()))
+    K, V = cache_bits(cache)
+    check_k(K, oracle.f32_to_f16(oracle.rope(k, pos, d, th, kind, n_rot)), pos, nkv, d,
+            max(1.0, float(np.abs(k).max())))
+    got_v = V[:, :, ps:ps + B].transpose(2, 0, 1).reshape(B, kvd)
+    assert np.array_equal(got_v, oracle.f32_to_f16(np.ascontiguousarray(v)))
+    outside = np.ones(K.shape[1], bool)
+    outside[ps:ps + B] = False
+    assert (K[:, outside, :] == SENTINEL).all() and (V[:, :, outside] == SENTINEL).all()
+
+
 @pytest.mark.parametrize("odt", [torch.float16, torch.bfloat16])
 def test_rope_q_out_dtypes(cuda, oracle, odt):
     from yllm_amd.attention import round_bf16, rope_kv_store

@@ -25,11 +25,11 @@
 //    pair is two adjacent elements.  q goes to
 //    q_out (f32 / f16 / bf16); k is rounded with the reference f32->f16
 //    rounding (platform.c:340-379) into the token's K row of each kv head.
-//    For a few tokens (decode) the same wave also writes the token's V
+//    Up to kScatterRows tokens the same waves also write the token's V
 //    elements into the tiles.
-//  * V tile blocks (more than kScatterRows tokens): 64 tokens x 64 channels
-//    staged in LDS, read along source rows and written along tile rows,
-//    rounded the same way.
+//  * V tile blocks (more than kScatterRows tokens): 64 positions x 64 channels
+//    through LDS, read along source rows and written along tile rows, rounded
+//    the same way.
 #include "common.hpp"
 #include "internal.hpp"
 
@@ -38,7 +38,11 @@
 namespace yhip {
 namespace {
 
-constexpr uint32_t kScatterRows = 16;  // up to this many tokens the rotation waves write V too
+// Up to this many tokens the rotation waves write V too, one pass each, with
+// no tile blocks (a memory round trip through LDS and a barrier): 28 / 4 heads
+// of 128, us with / without tile blocks: 17 tokens 5.4 / 3.3, 64 tokens 5.5 /
+// 3.8, 128 tokens 5.5 / 4.7, 256 tokens 5.7 / 5.4 (32 / 8 heads 6.2 / 6.8).
+constexpr uint32_t kScatterRows = 128;
 
 __device__ inline uint16_t bf16_bits(float x)
 {
@@ -75,24 +79,51 @@ __device__ inline void store_q_pair(void* out, size_t o, uint32_t e0, uint32_t e
     }
 }
 
+// V tile block vb: 64 destination positions, aligned to 64 so that 8 positions
+// never straddle a tile, times 64 channels (of one kv head: D is a multiple of
+// 64).  Each thread's eight 8-byte loads go out together, from clamped, valid
+// rows: one row per trip of a loop with the load under its bounds test was a
+// memory round trip per trip, which launches of up to 700 tokens waited for
+// (28 / 4 heads of 128, 300 tokens: 9.4 us, now 5.8).  The tile is stored transposed in LDS; 8 positions of one channel leave as one
+// 16-byte store where all of them are stored rows and the cache allows it.
 template <int D>
 __device__ void v_tile_block(const RopeArgs& a, uint32_t vb)
 {
-    __shared__ uint16_t tile[64][66];
-    const uint32_t kv_dim = a.n_kv * D;
-    const uint32_t ntx = (kv_dim + 63u) / 64u;
-    const uint32_t j0 = (vb % ntx) * 64u, b0 = (vb / ntx) * 64u;
-    const uint32_t tx = threadIdx.x & 63u, ty = threadIdx.x >> 6;
-    for (uint32_t r = ty; r < 64u; r += 4u) {
-        const uint32_t b = b0 + r, j = j0 + tx;
-        if (b < a.B && j < kv_dim) tile[r][tx] = f32_to_f16_ref(__builtin_nontemporal_load(a.v + (size_t)b * a.v_stride + j));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    constexpr uint32_t TP = 66;  // halfs per channel: even, so words stay aligned; 33 words spread the banks
+    __shared__ __attribute__((aligned(16))) uint16_t tile[64 * TP];
+    const uint32_t ntx = a.n_kv * D / 64u;
+    const uint32_t j0 = (vb % ntx) * 64u, p0 = (a.pos_start & ~63u) + (vb / ntx) * 64u;
+    const uint32_t end = a.pos_start + a.B;
+    const uint32_t c2 = (threadIdx.x & 31u) * 2u, r0 = threadIdx.x >> 5;  // channels c2, c2 + 1; rows r0, r0 + 8, ...
+    f32x2 x[8];
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) {
+        const uint32_t pos = min(max(p0 + r0 + 8u * u, a.pos_start), end - 1u);
+        x[u] = __builtin_nontemporal_load(
+            reinterpret_cast<const f32x2*>(a.v + (size_t)(pos - a.pos_start) * a.v_stride + j0 + c2));
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) {
+        tile[c2 * TP + r0 + 8u * u] = f32_to_f16_ref(x[u][0]);
+        tile[(c2 + 1) * TP + r0 + 8u * u] = f32_to_f16_ref(x[u][1]);
     }
     __syncthreads();
-    for (uint32_t r = ty; r < 64u; r += 4u) {
-        const uint32_t j = j0 + r, b = b0 + tx;
-        if (b < a.B && j < kv_dim) {
-            const uint32_t h = j / D, d = j - h * D;
-            a.vc[v_index(h, a.pos_start + b, d, D, a.kv_stride)] = tile[tx][r];
+    const uint32_t h = j0 / D, d0 = j0 - h * D;
+    const bool wide = ((uintptr_t)a.vc & 15u) == 0;
+#pragma unroll
+    for (uint32_t it = 0; it < 2; ++it) {
+        const uint32_t g = threadIdx.x + 256u * it, dl = g >> 3, q0 = (g & 7u) * 8u, pos0 = p0 + q0;
+        u32x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) w[e] = *reinterpret_cast<const uint32_t*>(&tile[dl * TP + q0 + 2 * e]);
+        uint16_t* dst = a.vc + v_index(h, pos0, d0 + dl, D, a.kv_stride);
+        if (wide && pos0 >= a.pos_start && pos0 + 8u <= end) {
+            *reinterpret_cast<u32x4*>(dst) = w;
+        } else {
+#pragma unroll
+            for (uint32_t e = 0; e < 8; ++e)
+                if (pos0 + e >= a.pos_start && pos0 + e < end) dst[e] = (uint16_t)(w[e / 2] >> (16 * (e & 1u)));
         }
     }
 }
@@ -239,19 +270,28 @@ hipError_t launch_kind(const RopeArgs& a, dim3 grid, hipStream_t st)
 
 hipError_t launch_rope_kv(RopeArgs a, hipStream_t st)
 {
-    // waves per token: one (all heads share the token's sines and cosines)
-    // unless there are too few tokens to give the chip about 1024 waves;
-    // then the heads are split over up to one wave per pass
+    // Passes (of hpi heads) per wave.  A wave reuses its token's sines and
+    // cosines over all its passes and issues four passes' loads together, so
+    // it takes a multiple of four; few waves with many passes leave too few
+    // bytes in flight and drain unevenly.  So about 8192 waves, four to twelve
+    // passes each (four at d 256, where a pass is two pairs per lane).  us at
+    // 32 / 8 heads of 128 with 1 / 4 / 8 / 12 / 20 / 40 passes: 64 tokens 5.0 /
+    // 5.0 / 5.5 / 6.0 / 7.8 / 11.7, 700 tokens 15.4 / 9.7 / 10.1 / 10.3 / 12.5 /
+    // 18.6, 8191 tokens 129 / 67.5 / 58.5 / 58.9 / 60.4 / 68.8 (all heads in one
+    // wave: before); 16 / 2 heads of 256 at 8191 (18 passes) 77 / 60.4 / 63.3 /
+    // 68.3 / 82.  Up to kScatterRows tokens, which write V too, one pass.
     const uint32_t hpi = a.D >= 128 ? 1u : 64u / (a.D / 2);
     const uint32_t active = a.q_out ? a.n_heads + a.n_kv : a.n_kv;
     const uint32_t passes = (active + hpi - 1) / hpi;
-    uint32_t groups = a.B >= 1024u ? 1u : (1024u + a.B - 1) / a.B;
-    groups = groups < passes ? groups : passes;
-    const uint32_t per = (passes + groups - 1) / groups;  // passes per wave
+    const uint32_t cap = a.D > 128 ? 4u : 12u;
+    const uint64_t share = ((uint64_t)a.B * passes + 32767u) / 32768u * 4u;
+    const uint32_t per0 = a.B <= kScatterRows ? 1u : share < cap ? (uint32_t)share : cap;
+    const uint32_t groups = (passes + per0 - 1) / per0;
+    const uint32_t per = (passes + groups - 1) / groups;  // passes per wave, evenly
     a.heads_per_wave = per * hpi;
     a.groups = (passes + per - 1) / per;
     a.rope_blocks = (uint32_t)(((uint64_t)a.B * a.groups + 3u) / 4u);
-    a.v_blocks = a.B > kScatterRows ? ((a.n_kv * a.D + 63u) / 64u) * ((a.B + 63u) / 64u) : 0u;
+    a.v_blocks = a.B > kScatterRows ? a.n_kv * a.D / 64u * (((a.pos_start & 63u) + a.B + 63u) / 64u) : 0u;
     const dim3 grid(a.rope_blocks + a.v_blocks);
     switch (a.kind) {
     case kRopeNone: return launch_kind<kRopeNone>(a, grid, st);
