@@ -597,3 +597,40 @@ def test_prefill_chunked_prompt_equals_single_launch(cuda, oracle):
     for t in (0, 63, 64, 1000, 1983, 1984, 2047):
         want = oracle.decode(q[t], kc[: t + 1], vc[: t + 1], t, nh, nkv, hd)
         assert rel_l2(chunked[t], want) <= TOL
+
+
+def test_workspace_given_short_or_misaligned(cuda):
+    """A caller's workspace that is too short is replaced (as without one), one
+    that is long enough but misaligned stays refused, and the operators queue
+    on torch's current stream."""
+    from yllm_amd._lib import YhipError, current_stream
+    from yllm_amd.attention import (LayerKV, attn_decode, attn_prefill, decode_workspace_bytes, kv_store,
+                                    o_proj, o_proj_workspace_bytes, prefill_workspace_bytes)
+
+    g = torch.Generator(device="cuda").manual_seed(77)
+    nh, nkv, d, L = 8, 2, 128, 3000
+    cache = LayerKV.empty(nkv, d, L, device=cuda)
+    kv_store(cache, torch.randn(L, nkv * d, generator=g, device=cuda).half(),
+             torch.randn(L, nkv * d, generator=g, device=cuda).half(), 0)
+    q = torch.randn(nh * d, generator=g, device=cuda)
+    qb = torch.randn(20, nh * d, generator=g, device=cuda)
+    att = torch.randn(20, nh * d, generator=g, device=cuda)
+    w = torch.randn(64, nh * d, generator=g, device=cuda)
+    calls = [
+        (decode_workspace_bytes(1, L, L, nh, nkv, d), lambda ws: attn_decode(q, cache, L - 1, nh, workspace=ws)),
+        (prefill_workspace_bytes(20, L, nh, nkv, d), lambda ws: attn_prefill(qb, cache, L - 20, nh, workspace=ws)),
+        (o_proj_workspace_bytes(20, 64, nh * d, torch.float32),
+         lambda ws: o_proj(torch.zeros(20, 64, device=cuda), att, w, workspace=ws)),
+    ]
+    for i, (need, call) in enumerate(calls):
+        assert need > 0
+        want = call(None)
+        for n in (0, need - 1, need, need + 4096):
+            assert torch.equal(call(torch.empty(n, dtype=torch.uint8, device=cuda)), want)
+        if i > 0:  # the decode takes any alignment
+            with pytest.raises(YhipError):
+                call(torch.empty(need + 4096, dtype=torch.uint8, device=cuda)[4:])
+    side = torch.cuda.Stream()
+    assert current_stream() == torch.cuda.current_stream().cuda_stream
+    with torch.cuda.stream(side):
+        assert current_stream() == side.cuda_stream

@@ -22,7 +22,8 @@ from dataclasses import dataclass
 import numpy as np
 import torch
 
-from ._lib import BF16, F16, F32, YhipError, check, lib
+from ._lib import BF16, ENOSPC, F16, F32, YhipError, check, lib
+from ._lib import current_stream as _stream
 
 _DT = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 
@@ -34,21 +35,14 @@ def _dtype_code(t: torch.Tensor) -> int:
         raise YhipError(-22, f"unsupported dtype {t.dtype}") from None
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
-
-
 def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
 def _need_gpu(*ts: torch.Tensor | None) -> None:
     for t in ts:
-        if t is not None:
-            if not t.is_cuda:
-                raise YhipError(-22, "tensor must be on the GPU")
-            if not t.is_contiguous():
-                raise YhipError(-22, "tensor must be contiguous")
+        if t is not None and not (t.is_cuda and t.is_contiguous()):
+            raise YhipError(-22, "tensor must be contiguous" if t.is_cuda else "tensor must be on the GPU")
 
 
 def round_up(x: int, m: int) -> int:
@@ -170,13 +164,11 @@ def o_proj(x: torch.Tensor, att: torch.Tensor, w: torch.Tensor, workspace: torch
     if not w.is_contiguous() or w.dim() != 2 or w.shape[1] != att.shape[1] or w.shape[0] != x.shape[1]:
         raise YhipError(-22, f"o_proj: w {tuple(w.shape)} does not match att {tuple(att.shape)} / x {tuple(x.shape)}")
     B, hidden, qdim = x.shape[0], w.shape[0], w.shape[1]
-    need = o_proj_workspace_bytes(B, hidden, qdim, w.dtype, att.dtype)
-    ws = _workspace(need, x.device, workspace)
     xs = x.stride(0) if B > 1 else hidden
     ats = att.stride(0) if B > 1 else qdim
-    check(lib().yhip_o_proj(_ptr(x), xs, _ptr(att), _dtype_code(att), ats, _ptr(w), _dtype_code(w), B, hidden,
-                            qdim, _ptr(ws),
-                            ws.numel() * ws.element_size() if ws is not None else 0, _stream()))
+    args = (x.data_ptr(), xs, att.data_ptr(), _dtype_code(att), ats, w.data_ptr(), _dtype_code(w), B, hidden, qdim)
+    _with_workspace(lib().yhip_o_proj, args, workspace,
+                    lambda: o_proj_workspace_bytes(B, hidden, qdim, w.dtype, att.dtype), x.device)
     return x
 
 
@@ -215,6 +207,22 @@ def _workspace(nbytes: int, device: torch.device, ws: torch.Tensor | None) -> to
     return decode_workspace(nbytes, device)
 
 
+def _with_workspace(fn, args: tuple, workspace: torch.Tensor | None, need, device: torch.device) -> None:
+    """fn(*args, workspace, its bytes, stream).  A caller's workspace is tried
+    as it is, which spares the separate planning call: the library refuses one
+    that is too short before it launches anything, and then, as without one,
+    `need()` bytes are allocated."""
+    if workspace is not None and workspace.numel():
+        have = workspace.numel() * workspace.element_size()
+        rc = fn(*args, workspace.data_ptr(), have, _stream())
+        if rc != ENOSPC or have >= need():
+            check(rc)
+            return
+    nbytes = need()
+    ws = _workspace(nbytes, device, None)
+    check(fn(*args, _ptr(ws), nbytes, _stream()))
+
+
 def attn_decode(q: torch.Tensor, cache: LayerKV, pos: int, n_heads: int, gate: torch.Tensor | None = None,
                 out: torch.Tensor | None = None, workspace: torch.Tensor | None = None) -> torch.Tensor:
     """One query token at position pos over keys 0..pos. q: f32 [n_heads*head_dim]."""
@@ -224,10 +232,11 @@ def attn_decode(q: torch.Tensor, cache: LayerKV, pos: int, n_heads: int, gate: t
         raise YhipError(-22, "attn_decode: q must be f32 [n_heads*head_dim]")
     if out is None:
         out = torch.empty(n_heads * d, dtype=torch.float32, device=q.device)
-    nbytes = decode_workspace_bytes(1, pos + 1, pos + 1, n_heads, cache.n_kv, d)
-    ws = _workspace(nbytes, q.device, workspace)
-    check(lib().yhip_attn_decode(_ptr(out), _ptr(q), _ptr(cache.k), _ptr(cache.v), pos, n_heads, cache.n_kv,
-                                 d, cache.kv_stride, _ptr(gate), _ptr(ws), nbytes, _stream()))
+    fn, n_kv = lib().yhip_attn_decode, cache.n_kv
+    args = (out.data_ptr(), q.data_ptr(), cache.k.data_ptr(), cache.v.data_ptr(), pos, n_heads, n_kv, d,
+            cache.kv_stride, _ptr(gate))
+    _with_workspace(fn, args, workspace, lambda: decode_workspace_bytes(1, pos + 1, pos + 1, n_heads, n_kv, d),
+                    q.device)
     return out
 
 
@@ -245,11 +254,11 @@ def attn_decode_rope(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, cache: L
         raise YhipError(-22, "attn_decode_rope: q, k, v must be the token's f32 rows")
     if out is None:
         out = torch.empty(n_heads * d, dtype=torch.float32, device=q.device)
-    nbytes = decode_workspace_bytes(1, pos + 1, pos + 1, n_heads, cache.n_kv, d)
-    ws = _workspace(nbytes, q.device, workspace)
-    check(lib().yhip_attn_decode_rope(_ptr(out), _ptr(q), _ptr(k), _ptr(v), _ptr(cache.k), _ptr(cache.v), pos,
-                                      n_heads, cache.n_kv, d, cache.kv_stride, rope, n_rot, theta, _ptr(gate),
-                                      _ptr(ws), nbytes, _stream()))
+    fn, n_kv = lib().yhip_attn_decode_rope, cache.n_kv
+    args = (out.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), cache.k.data_ptr(), cache.v.data_ptr(), pos,
+            n_heads, n_kv, d, cache.kv_stride, rope, n_rot, theta, _ptr(gate))
+    _with_workspace(fn, args, workspace, lambda: decode_workspace_bytes(1, pos + 1, pos + 1, n_heads, n_kv, d),
+                    q.device)
     return out
 
 
@@ -323,15 +332,14 @@ def attn_prefill(q: torch.Tensor, cache: LayerKV, pos_start: int, n_heads: int,
         out = torch.empty((B, n_heads * d), dtype=out_dtype, device=q.device)
     if out.shape[0] != B or out.shape[1] != n_heads * d:
         raise YhipError(-22, "attn_prefill: out must be [B, n_heads*head_dim]")
-    nbytes = prefill_workspace_bytes(B, pos_start + B, n_heads, cache.n_kv, d)
-    ws = _workspace(nbytes, q.device, workspace)
+    n_kv = cache.n_kv
     qs = q.stride(0) if B > 1 else q.shape[1]
     os_ = out.stride(0) if B > 1 else out.shape[1]
     gs = (gate.stride(0) if B > 1 else gate.shape[1]) if gate is not None else 0
-    check(lib().yhip_attn_prefill(_ptr(out), _dtype_code(out), os_, _ptr(q), _dtype_code(q), qs, _ptr(cache.k),
-                                  _ptr(cache.v), pos_start, B, n_heads, cache.n_kv, d, cache.kv_stride, _ptr(gate),
-                                  gs, _ptr(ws), ws.numel() * ws.element_size() if ws is not None else 0,
-                                  _stream()))
+    args = (out.data_ptr(), _dtype_code(out), os_, q.data_ptr(), _dtype_code(q), qs, cache.k.data_ptr(),
+            cache.v.data_ptr(), pos_start, B, n_heads, n_kv, d, cache.kv_stride, _ptr(gate), gs)
+    _with_workspace(lib().yhip_attn_prefill, args, workspace,
+                    lambda: prefill_workspace_bytes(B, pos_start + B, n_heads, n_kv, d), q.device)
     return out
 
 

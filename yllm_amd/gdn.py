@@ -24,17 +24,15 @@ from __future__ import annotations
 import torch
 
 from ._lib import F16, F32, YhipError, check, lib
+from ._lib import current_stream as _stream
 
 L2_EPS = 1e-6  # the qwen35 GDN l2norm epsilon (engine.c:826-827 passes the model's norm eps)
 
 
-def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
-
-
 def _f32_gpu(*ts: torch.Tensor) -> None:
+    f32 = torch.float32
     for t in ts:
-        if not t.is_cuda or t.dtype != torch.float32:
+        if t.dtype is not f32 or not t.is_cuda:
             raise YhipError(-22, "GDN tensors must be fp32 on the GPU")
 
 
@@ -203,21 +201,24 @@ def gdn_decode(S: torch.Tensor, conv_in: torch.Tensor, conv_out: torch.Tensor, q
     token); qkv [conv_dim] = q | k | v; z [n_v*d]; alpha, beta_raw, dt_bias,
     ssm_a [n_v]; conv_w [conv_dim, kwidth]; norm_w [d] fp32 or f16.
     Returns y [n_v*d]."""
-    _f32_gpu(S, conv_in, conv_out, qkv, z, alpha, beta_raw, conv_w, dt_bias, ssm_a)
-    n_v, d = S.shape[0], S.shape[1]
-    kwidth, conv_dim = conv_in.shape
-    if S.shape != (n_v, d, d) or not S.is_contiguous() or conv_out.shape != conv_in.shape:
-        raise YhipError(-22, "gdn_decode: S must be contiguous [n_v, d, d]; conv_in / conv_out [kwidth, conv_dim]")
-    if conv_dim != (2 * n_k + n_v) * d or conv_w.shape != (conv_dim, kwidth):
-        raise YhipError(-22, "gdn_decode: conv_dim must be (2*n_k + n_v)*d and conv_w [conv_dim, kwidth]")
-    for t in (conv_in, conv_out, qkv, z, alpha, beta_raw, conv_w, dt_bias, ssm_a, norm_w):
+    f32 = torch.float32
+    for t in (S, conv_in, conv_out, qkv, z, alpha, beta_raw, conv_w, dt_bias, ssm_a):
+        if t.dtype is not f32 or not t.is_cuda:
+            raise YhipError(-22, "GDN tensors must be fp32 on the GPU")
         if not t.is_contiguous():
             raise YhipError(-22, "gdn_decode: tensors must be contiguous")
-    if qkv.numel() < conv_dim or z.numel() < n_v * d or min(alpha.numel(), beta_raw.numel(), dt_bias.numel(),
-                                                            ssm_a.numel()) < n_v or norm_w.numel() != d:
+    shape = S.shape
+    n_v, d = shape[0], shape[1]
+    kwidth, conv_dim = conv_in.shape
+    if shape != (n_v, d, d) or conv_out.shape != conv_in.shape:
+        raise YhipError(-22, "gdn_decode: S must be [n_v, d, d]; conv_in / conv_out [kwidth, conv_dim]")
+    if conv_dim != (2 * n_k + n_v) * d or conv_w.shape != (conv_dim, kwidth):
+        raise YhipError(-22, "gdn_decode: conv_dim must be (2*n_k + n_v)*d and conv_w [conv_dim, kwidth]")
+    if (qkv.numel() < conv_dim or z.numel() < n_v * d or alpha.numel() < n_v or beta_raw.numel() < n_v
+            or dt_bias.numel() < n_v or ssm_a.numel() < n_v or norm_w.numel() != d):
         raise YhipError(-22, "gdn_decode: input sizes do not match the heads")
-    if not norm_w.is_cuda or norm_w.dtype not in (torch.float32, torch.float16):
-        raise YhipError(-22, "gdn_decode: norm_w must be fp32 or f16 on the GPU")
+    if not norm_w.is_cuda or norm_w.dtype not in (torch.float32, torch.float16) or not norm_w.is_contiguous():
+        raise YhipError(-22, "gdn_decode: norm_w must be contiguous, fp32 or f16 on the GPU")
     if y is None:
         y = torch.empty(n_v * d, dtype=torch.float32, device=S.device)
     _f32_gpu(y)
