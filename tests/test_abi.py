@@ -282,3 +282,28 @@ def test_decode_rope_rejects_bad_args(hiplib):
     # 32k keys split: a workspace is needed
     big = [P, P, P, P, P, P, 32767, 32, 8, 128, 32768, 1, 0, F(1e4), None, None, 0, None]
     assert hiplib.yhip_attn_decode_rope(*big) == -28 and "workspace" in _err(hiplib)
+
+
+def test_prefill_plan_fits_its_workspace(hiplib):
+    """The workspace of yhip_attn_prefill_workspace serves every call it
+    promises to: no shape's plan asks for more.  (Without a GPU a call that
+    passes its checks ends at the launch, so nothing is dereferenced.)"""
+    import torch
+
+    if torch.cuda.is_available():
+        pytest.skip("a GPU would run the launch")
+    p, n = 1 << 20, 0
+    for nh, nkv, d in ((14, 2, 64), (28, 4, 128), (32, 8, 128), (16, 2, 256), (6, 3, 256), (5, 5, 64)):
+        row = nh * d
+        for B in (1, 2, 33, 64, 100, 127, 128, 200, 333, 700, 1000, 1800):
+            for end in (B, B + 1, B + 100, B + 700, B + 2000, 8000, 40000):
+                if end < B:
+                    continue
+                ws = hiplib.yhip_attn_prefill_workspace(B, end, nh, nkv, d)
+                for start in {0, (end - B) // 3, end - B}:
+                    for dt in (0, 1, 2):
+                        rc = hiplib.yhip_attn_prefill(p, 1, row, p, dt, row, p, p, start, B, nh, nkv, d, 65536, None, 0,
+                                                      p, ws, None)
+                        assert rc == -5, (nh, nkv, d, B, end, start, dt, rc, hiplib.yhip_last_error())
+                        n += 1
+    assert n > 1000

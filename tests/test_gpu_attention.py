@@ -634,3 +634,64 @@ def test_workspace_given_short_or_misaligned(cuda):
     assert current_stream() == torch.cuda.current_stream().cuda_stream
     with torch.cuda.stream(side):
         assert current_stream() == side.cuda_stream
+
+
+def _prefill_f64(q, cache, start, nh, gate=None):
+    """Causal attention of rows q over the cache in float64 (torch, per head)."""
+    nkv, stride, d = cache.k.shape
+    T, n = q.shape[0], start + q.shape[0]
+    K = cache.k[:, :n].double()
+    V = cache.v.view(nkv, stride // 32, d, 32).permute(0, 1, 3, 2).reshape(nkv, stride, d)[:, :n].double()
+    past = torch.arange(n, device=q.device)[None, :] > torch.arange(start, n, device=q.device)[:, None]
+    out = torch.empty(T, nh * d, dtype=torch.float64, device=q.device)
+    for h in range(nh):
+        s = q[:, h * d:(h + 1) * d].double() @ K[h * nkv // nh].t() / d ** 0.5
+        out[:, h * d:(h + 1) * d] = s.masked_fill(past, float("-inf")).softmax(-1) @ V[h * nkv // nh]
+    return out if gate is None else out * gate.double().sigmoid()
+
+
+@pytest.mark.parametrize("nh,nkv,d,T,start,qdt,odt,gated", [
+    # head_dim 256, 16-bit queries: whole query blocks over all keys (256 items and more)
+    (64, 4, 256, 513, 0, "bf16", "bf16", True),     # one query in the last block, two items per workgroup
+    (64, 8, 256, 600, 5, "f16", "f32", False),      # query blocks that straddle tiles, a partial last tile
+    (96, 6, 256, 385, 64, "bf16", "f16", True),     # kv heads that are no divisor of 8
+    (128, 8, 256, 257, 127, "f16", "f32", True),
+    # the same kernel in the split mode: packed rows, several splits, splits past a row block's keys
+    (16, 2, 256, 33, 900, "bf16", "f32", True),
+    (16, 2, 256, 100, 3001, "f16", "f32", False),
+    (16, 2, 256, 130, 700, "bf16", "bf16", True),
+    (6, 3, 256, 300, 1500, "f16", "f32", True),
+    (16, 2, 256, 1000, 0, "bf16", "f32", False),    # unsplit, fewer items than CUs
+    # short walks, which keep the pair kernel
+    (16, 2, 256, 64, 0, "bf16", "f32", True),
+    (16, 2, 256, 33, 100, "f16", "f32", True),
+    # tile groups that do not fill the XCDs evenly, the plan's unsplit and split choices
+    (14, 2, 64, 1500, 0, "f16", "f32", False),
+    (14, 2, 64, 700, 3000, "f32", "f32", False),
+    (28, 4, 128, 700, 0, "f32", "f32", False),
+    (15, 3, 128, 140, 900, "bf16", "f32", False),
+    (5, 5, 64, 70, 800, "f16", "f32", True),
+])
+def test_prefill_plan_and_halves_edges(cuda, nh, nkv, d, T, start, qdt, odt, gated):
+    """Where the head_dim 256 kernel and the split plan change: against
+    float64, max relative L2 1e-3 (f16 probabilities, 2^-11 each) and 3e-3 per
+    row, bf16 outputs plus their 2^-8 rounding; V past the last key is NaN."""
+    from yllm_amd.attention import LayerKV, attn_prefill, kv_store
+
+    dt = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}
+    g = torch.Generator(device="cuda").manual_seed(T + start)
+    n = start + T
+    cache = LayerKV.empty(nkv, d, n + 64, device=cuda)
+    cache.k.fill_(float("nan"))
+    cache.v.fill_(float("nan"))
+    kv_store(cache, torch.randn(n, nkv * d, generator=g, device=cuda).half(),
+             torch.randn(n, nkv * d, generator=g, device=cuda).half(), 0)
+    q = (torch.randn(T, nh * d, generator=g, device=cuda) * 1.5).to(dt[qdt])
+    gate = torch.randn(T, nh * d + 5, generator=g, device=cuda)[:, 3:-2] if gated else None  # rows are float-aligned only
+    got = attn_prefill(q, cache, start, nh, out_dtype=dt[odt], gate=gate).double()
+    want = _prefill_f64(q, cache, start, nh, gate)
+    add = 2.0 ** -8 if odt == "bf16" else 0.0
+    err = float((got - want).norm() / want.norm())
+    rows = float(((got - want).norm(dim=1) / want.norm(dim=1)).max())
+    print(f"prefill {nh}/{nkv} d={d} {T}@{start} {qdt}->{odt}: rel_l2 {err:.2e}, worst row {rows:.2e}")
+    assert err <= 1e-3 + add and rows <= 3e-3 + add

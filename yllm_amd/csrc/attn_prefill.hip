@@ -262,6 +262,77 @@ __device__ inline void item_keys(const PrefillArgs& a, const PItem& I, uint32_t&
     }
 }
 
+// Item `it` of this workgroup in the plain mode; false past the last.
+__device__ inline bool plain_item(const PrefillArgs& a, uint32_t nqb, uint32_t it, PItem& I)
+{
+    I.split = 0;
+    if (a.xcd_map) {
+        // Consecutive workgroups go to the 8 XCDs in turn.  XCD x serves
+        // kv head x % n_kv, so the query heads that read one kv head
+        // share an L2 and its K/V tiles are fetched from HBM once per XCD
+        // group, not once per XCD; the XCD's own workgroups take its items.
+        const uint32_t x = blockIdx.x % 8u, j = blockIdx.x / 8u, W = gridDim.x / 8u;
+        const uint32_t slot = it * W + ((it & 1u) ? W - 1u - j : j);
+        if (slot >= nqb * a.n_heads / 8u) return false;
+        const uint32_t per = 8u / a.n_kv, G = a.n_heads / a.n_kv;
+        const uint32_t g = x % a.n_kv, i = slot * per + x / a.n_kv;
+        I.qb = nqb - 1 - i / G;
+        I.h = g * G + i % G;
+    } else {
+        const uint32_t W = gridDim.x;
+        const uint32_t slot = it * W + ((it & 1u) ? W - 1u - blockIdx.x : blockIdx.x);
+        if (slot >= nqb * a.n_heads) return false;
+        I.qb = nqb - 1 - slot / a.n_heads;
+        I.h = slot % a.n_heads;
+    }
+    I.kvh = I.h * a.n_kv / a.n_heads;  // engine.c:537
+    return true;
+}
+
+// The split mode's item of this workgroup; false where the grid has none.  The
+// items of a (kv head, split) tile group read the same K/V tiles, so they should
+// share an XCD's L2 (consecutive workgroups go to the 8 XCDs in turn).  With a
+// multiple of 8 groups XCD x serves groups x, x+8, ...  Otherwise whole groups
+// would leave XCDs idle (2 kv heads without a split: six of eight; 1800 tokens
+// of 16 / 2 heads of 256 took 195 us), so each XCD takes an eighth of the items
+// in group order; within a group the order deals the row blocks out evenly, so
+// that every run of it holds heavy and light ones.
+__device__ inline bool split_item(const PrefillArgs& a, PItem& I)
+{
+    const uint32_t x = blockIdx.x % 8u, j = blockIdx.x / 8u;
+    const uint32_t ipg = a.n_rb * (a.pack ? 1u : a.gmax), groups = a.n_kv * a.n_split;
+    uint32_t tg, w;
+    if (groups % 8u == 0) {
+        tg = (j / ipg) * 8u + x;
+        w = j % ipg;
+    } else {
+        const uint32_t per = gridDim.x / 8u, i = x * per + j;
+        if (i >= groups * ipg) return false;
+        tg = i / ipg;
+        w = i - tg * ipg;
+        if (!a.pack) {
+            // position w of the group's order: the items 0 mod 8 first, then 1 mod 8, ... (packed rows walk the
+            // same keys)
+            const uint32_t len = ipg / 8u, rem = ipg % 8u;
+            const bool lead = w < rem * (len + 1u);  // the first `rem` residues have one item more
+            const uint32_t r1 = lead ? w : w - rem * (len + 1u), l1 = lead ? len + 1u : len, q = r1 / l1;
+            w = (lead ? 0u : rem) + q + 8u * (r1 - q * l1);
+        }
+    }
+    if (tg >= groups) return false;
+    I.kvh = tg % a.n_kv;
+    I.split = tg / a.n_kv;
+    const uint32_t h0 = head0(a, I.kvh), h1 = head0(a, I.kvh + 1);
+    if (a.pack) {
+        I.qb = w;
+        I.h = h0;
+        return w * BM < (h1 - h0) * a.B;
+    }
+    I.qb = a.n_rb - 1 - w / a.gmax;  // heaviest first
+    I.h = h0 + w % a.gmax;
+    return I.h < h1;
+}
+
 // SPLIT: the split mode (one item per workgroup, packed rows, a key range
 // per split); a separate instantiation keeps the plain mode's registers.
 // QS: fp32 queries as f16 hi + lo parts, two score MFMAs per k-chunk (32 more
@@ -336,50 +407,8 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
     const uint32_t nqb = (a.B + BM - 1) / BM;
     // item `it` of this workgroup; false past the last
     auto item_of = [&](uint32_t it, PItem& I) -> bool {
-        if (SPLIT) {
-            // one item per workgroup.  The items of a (kv head, split) tile
-            // group read the same K/V tiles: XCD x serves tile groups x, x+8,
-            // ... (consecutive workgroups go to the 8 XCDs in turn), so they
-            // share its L2.
-            if (it > 0) return false;
-            const uint32_t x = blockIdx.x % 8u, j = blockIdx.x / 8u;
-            const uint32_t ipg = a.n_rb * (a.pack ? 1u : a.gmax);
-            const uint32_t tg = (j / ipg) * 8u + x, w = j % ipg;
-            if (tg >= a.n_kv * a.n_split) return false;
-            I.kvh = tg % a.n_kv;
-            I.split = tg / a.n_kv;
-            const uint32_t h0 = head0(a, I.kvh), h1 = head0(a, I.kvh + 1);
-            if (a.pack) {
-                I.qb = w;
-                I.h = h0;
-                return w * BM < (h1 - h0) * a.B;
-            }
-            I.qb = a.n_rb - 1 - w / a.gmax;  // heaviest first
-            I.h = h0 + w % a.gmax;
-            return I.h < h1;
-        }
-        I.split = 0;
-        if (a.xcd_map) {
-            // Consecutive workgroups go to the 8 XCDs in turn.  XCD x serves
-            // kv head x % n_kv, so the query heads that read one kv head
-            // share an L2 and its K/V tiles are fetched from HBM once per XCD
-            // group, not once per XCD; the XCD's own workgroups take its items.
-            const uint32_t x = blockIdx.x % 8u, j = blockIdx.x / 8u, W = gridDim.x / 8u;
-            const uint32_t slot = it * W + ((it & 1u) ? W - 1u - j : j);
-            if (slot >= nqb * a.n_heads / 8u) return false;
-            const uint32_t per = 8u / a.n_kv, G = a.n_heads / a.n_kv;
-            const uint32_t g = x % a.n_kv, i = slot * per + x / a.n_kv;
-            I.qb = nqb - 1 - i / G;
-            I.h = g * G + i % G;
-        } else {
-            const uint32_t W = gridDim.x;
-            const uint32_t slot = it * W + ((it & 1u) ? W - 1u - blockIdx.x : blockIdx.x);
-            if (slot >= nqb * a.n_heads) return false;
-            I.qb = nqb - 1 - slot / a.n_heads;
-            I.h = slot % a.n_heads;
-        }
-        I.kvh = I.h * a.n_kv / a.n_heads;  // engine.c:537
-        return true;
+        if (SPLIT) return it == 0 && split_item(a, I);  // one item per workgroup
+        return plain_item(a, nqb, it, I);
     };
     // An item's first loads are issued during the previous item: its
     // group's first K, V and second K tiles in the previous item's last key
@@ -922,6 +951,394 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
     }  // items
 }
 
+// head_dim 256, 16-bit queries.  Bound by the LDS: 128 bytes per
+// cycle and CU against 4 KB of operands per 32-cycle MFMA slot of the four
+// SIMDs.  A workgroup is 8 waves over 128 queries, one per CU, and two waves
+// share 32 queries (a wave with all 256 dimensions of O and Q would be alone on
+// its SIMD).  The pair splits the scores by keys and the output by dimensions:
+// of a 64-key tile each wave forms the scores of 32 keys over all 256
+// dimensions (Q in 64 registers), turns them into probabilities, hands the
+// 2 KB of f16 probabilities to its partner through LDS and accumulates its
+// half of the dimensions of O over all 64 keys.  Split by dimensions on both
+// sides (prefill_kernel's pair mode, which keeps f32 queries), the waves exchange fp32 partial scores and both form every
+// probability: 1.75 KB of LDS traffic per MFMA against 1.38, and twice the exp2.
+// 4096 tokens, 16 / 2 heads, bf16, gated: 215 -> 166 us (825 TFLOP/s), ungated
+// 188 -> 153.
+//
+// Step t starts with the raw scores of tile t in registers and their maxima
+// in LDS.  The next tile's score MFMAs begin; the pair's common maximum is
+// formed (lazily, as in prefill_kernel); the 16 probabilities of a lane go
+// between the rest of the score MFMAs and then to LDS; the output MFMAs of the
+// wave's own 32 keys follow; a barrier; those of the partner's keys, under
+// which the next tile's maximum is formed; a barrier.  K is loaded two tiles
+// ahead, V one, straight into LDS, and an item's first tiles and queries during
+// the previous item's last step.
+template <int D, bool SPLIT>
+__global__ __launch_bounds__(512) void prefill_halves_kernel(PrefillArgs a)
+{
+    static_assert(D == 256, "two waves of 128 output dimensions");
+    constexpr int BN = 64, DH = D / 2;
+    constexpr int NKK = D / 16, NDB = DH / 32;
+    constexpr int KCH = D / 8, VCH = BN / 8;
+    constexpr int CH = BN * D / (8 * 512);  // 16-byte chunks per thread per tile (K and V each)
+        constexpr float kSlack = 8.0f;
+    __shared__ __attribute__((aligned(16))) _Float16 Kl0[BN * D], Kl1[BN * D], Vl0[D * BN], Vl1[D * BN];
+    __shared__ f16x8 Pl[8][2][64];  // each wave's probabilities: k-slot, lane
+    __shared__ float Ml[8][64];     // each wave's tile maxima, then its row sums
+
+    const uint32_t nqb = (a.B + BM - 1) / BM;
+    PItem cur;
+    if (SPLIT ? !split_item(a, cur) : !plain_item(a, nqb, 0, cur)) return;  // uniform over the workgroup
+    for (uint32_t it = 0;; ++it) {
+        int tid;  // opaque per item, as in prefill_kernel
+        asm volatile("v_mov_b32 %0, %1" : "=v"(tid) : "v"((int)threadIdx.x));
+        const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+        const int qw = wave >> 1, hf = wave & 1;
+        const int r32 = lane & 31, hh = lane >> 5;
+        PItem nxt{};
+        const bool has_next = !SPLIT && plain_item(a, nqb, it + 1, nxt);
+
+        auto kbuf = [&](int par) { return par == 0 ? &Kl0[0] : &Kl1[0]; };
+        auto vbuf = [&](int par) { return par == 0 ? &Vl0[0] : &Vl1[0]; };
+        // chunk 512 i + tid of a tile: K LDS row R = 16 i + tid / KCH, V LDS row d = 64 i + tid / VCH; the swizzles
+        // and the row permutation are the same for every i
+        const int kgo = (lds_row_of_key(tid / KCH) * D + ((tid % KCH) ^ chunk_swz<KCH>(tid / KCH)) * 8) * 2;
+        const int vch = (tid % VCH) ^ chunk_swz<VCH>(tid / VCH);
+        const int vgo = (vch >> 2) * (D * (int)kVTile * 2) + tid / VCH * ((int)kVTile * 2) + (vch & 3) * 16;
+        // tile kt of kv head kv, counted from position p0 (a multiple of 64: 64 rows of K and two V tiles of 32
+        // positions are the same number of elements)
+        const uint32_t head_bytes = a.kv_stride * D * 2;
+        auto dma_k = [&](uint32_t kv, uint32_t p0, int par, uint32_t kt) {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<uint16_t*>(a.kc + k_index(kv, p0, 0, D, a.kv_stride)), 0, head_bytes - p0 * D * 2, 0x00020000);
+#pragma unroll
+            for (int i = 0; i < CH; ++i)
+                lds_load16(r, kbuf(par) + (512 * i + 64 * wave) * 8, kgo, kt * BN * D * 2 + i * (16 * D * 2));
+        };
+        auto dma_v = [&](uint32_t kv, uint32_t p0, int par, uint32_t kt) {
+            const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(
+                const_cast<uint16_t*>(a.vc + v_index(kv, p0, 0, D, a.kv_stride)), 0, head_bytes - p0 * D * 2, 0x00020000);
+#pragma unroll
+            for (int i = 0; i < CH; ++i)
+                lds_load16(r, vbuf(par) + (512 * i + 64 * wave) * 8, vgo, kt * BN * D * 2 + i * (64 * (int)kVTile * 2));
+        };
+        auto dma_done = [] { __builtin_amdgcn_s_waitcnt(0x0f70); };  // vmcnt(0)
+        // an item's tiles: how many, from position p0 on, and its last key (split_tiles counts 32 keys, an even
+        // number of them)
+        auto tiles_of = [&](const PItem& I, uint32_t& kmax, uint32_t& p0) -> uint32_t {
+            kmax = a.pos_start + ((SPLIT && a.pack) ? a.B - 1 : min(a.B, I.qb * BM + BM) - 1);
+            const uint32_t all = kmax / BN + 1, per = (a.split_tiles + 1) / 2;
+            p0 = 0;
+            if (!SPLIT) return all;
+            p0 = I.split * per * BN;
+            // a row block without keys in this split walks one tile, keys of later rows, with every wave idle
+            return max(min(all - min(all, I.split * per), per), 1u);
+        };
+        // the item's first K tiles; those of V follow into buffer 0
+        auto issue_k = [&](const PItem& I) {
+            uint32_t km, p0;
+            const uint32_t n = tiles_of(I, km, p0);
+            dma_k(I.kvh, p0, 0, 0);
+            if (n > 1) dma_k(I.kvh, p0, 1, 1);
+        };
+        const uint32_t kvh = cur.kvh;
+        uint32_t kmax, p0;
+        const uint32_t ntiles = tiles_of(cur, kmax, p0);
+        if (it == 0) {
+            issue_k(cur);
+            dma_v(kvh, p0, 0, 0);
+        }
+        f16x8 qf[NKK];  // loaded by each item itself: prefetched, they held 64 registers over the epilogue and spilled
+        {
+            const PRow rw = row_of<SPLIT>(a, cur, qw * 32 + r32);
+            const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + (size_t)rw.b * a.q_stride + (size_t)rw.h * D + hh * 8;
+#pragma unroll
+            for (int kk = 0; kk < NKK; ++kk) qf[kk] = *reinterpret_cast<const f16x8*>(qp + kk * 16);
+        }
+
+        // positions relative to p0 from here on (negative: before this split's keys)
+        uint32_t wfirst, wlast;
+        const bool wave_active = wave_span<SPLIT>(a, cur, qw, wfirst, wlast);
+        const int base = (int)(a.pos_start - p0);
+        const int wpos_first = __builtin_amdgcn_readfirstlane(base + (int)wfirst), wpos_last = base + (int)wlast;
+        const int my_pos = base + (int)row_of<SPLIT>(a, cur, qw * 32 + r32).b;
+        // the pair's tiles
+        const uint32_t wsteps = __builtin_amdgcn_readfirstlane(
+            wave_active && wpos_last >= 0 ? min((uint32_t)wpos_last / BN + 1, ntiles) : 0);
+
+        // Fragment offsets.  K row r32 + 32 hf, chunk (2 kk + hh) ^ swz: the swizzle changes the chunk's low four bits
+        // only, so k-chunks kk and kk + 8 share an offset up to a constant.  V row DH hf + 32 b + r32, chunk
+        // (4 kh + 2 s + hh) ^ swz for k-slot s of key half kh.
+        const int krow = (r32 + 32 * hf) * D, vrow = (DH * hf + r32) * BN;
+        int ko[8], vo[2][2];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ko[j] = krow + (((2 * j + hh) ^ chunk_swz<KCH>(r32)) << 3);
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            vo[0][s] = vrow + (((4 * hf + 2 * s + hh) ^ chunk_swz<VCH>(r32)) << 3);        // the wave's own half
+            vo[1][s] = vrow + (((4 * (hf ^ 1) + 2 * s + hh) ^ chunk_swz<VCH>(r32)) << 3);  // its partner's
+        }
+        auto read_k = [&](int par, int kk) {
+            return *reinterpret_cast<const f16x8*>(kbuf(par) + (ko[kk & 7] + (kk >> 3) * 128));
+        };
+        auto read_v = [&](int par, int b, int other, int s) {
+            return *reinterpret_cast<const f16x8*>(vbuf(par) + (vo[other][s] + 32 * b * BN));
+        };
+        // keys past kmax in the item's last tile were never stored: their P is 0, their V must be finite
+        auto zero_v_tail = [&](int par) {
+            const uint32_t valid = kmax - p0 - (ntiles - 1) * BN + 1;
+            _Float16* vb = vbuf(par);
+            for (int idx = tid; idx < D * VCH; idx += 512) {
+                const int d = idx / VCH, c = idx % VCH;
+                if ((uint32_t)(8 * c + 7) < valid) continue;
+                f16x8* ch = reinterpret_cast<f16x8*>(vb + (d * BN + ((c ^ chunk_swz<VCH>(d)) << 3)));
+                f16x8 v = *ch;
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if ((uint32_t)(8 * c + e) >= valid) v[e] = (_Float16)0.0f;
+                *ch = v;
+            }
+        };
+
+        float m = -1e30f, l = 0.0f, mx = 0.0f;
+        f32x16 o[NDB];
+#pragma unroll
+        for (int b = 0; b < NDB; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[b][i] = 0.0f;
+
+        // mask the wave's keys of tile st past the lanes' positions, form their maximum and publish it
+        auto tile_max = [&](f32x16& S, uint32_t st) {
+            const int k0 = (int)st * BN + 32 * hf;
+            if (k0 + 31 > wpos_first) {
+                const int rel = my_pos - k0 - 8 * hh;  // element i is key 8 hh + key_of_acc(i, 0) of the half
+#pragma unroll
+                for (int i = 0; i < 16; ++i)
+                    if (key_of_acc(i, 0) > rel) S[i] = -INFINITY;
+            }
+            mx = S[0];
+#pragma unroll
+            for (int i = 1; i < 16; ++i) mx = fmaxf(mx, S[i]);
+            mx = max_xor32(mx);
+            Ml[wave][lane] = mx;
+        };
+        auto rescale = [&](float other) {
+            const float t = fmaxf(mx, other) * a.c;
+            if (__ballot(t > m + kSlack)) {  // wave-uniform, and the same for both waves of the pair
+                const float mn = t > m + kSlack ? t : m;
+                const float alpha = fast_exp2(m - mn);
+                m = mn;
+                l *= alpha;
+#pragma unroll
+                for (int b = 0; b < NDB; ++b) o[b] *= alpha;
+            }
+        };
+        auto prob = [&](const f32x16& S, f16x8 (&pf)[2], int i) {
+            const float p = fast_exp2(fmaf(S[i], a.c, -m));
+            l += p;
+            pf[i >> 3][i & 7] = (_Float16)p;
+        };
+        // O^T += V^T P^T over the wave's own or its partner's keys of the tile in V buffer par
+        auto pv = [&](const f16x8 (&pf)[2], int par, int other) {
+            constexpr int NM = 2 * NDB;  // MFMA n: k-slot n / NDB, block n % NDB
+            f16x8 vf[3];
+            vf[0] = read_v(par, 0, other, 0);
+            vf[1] = read_v(par, 1, other, 0);
+#pragma unroll
+            for (int n = 0; n < NM; ++n) {
+                if (n + 2 < NM) vf[(n + 2) % 3] = read_v(par, (n + 2) % NDB, other, (n + 2) / NDB);
+                o[n % NDB] = mfma32(vf[n % 3], pf[n / NDB], o[n % NDB]);
+            }
+        };
+
+        // prologue: the item's first loads are in flight
+        dma_done();
+        if (a.q_dtype == kBF16) {
+#pragma unroll
+            for (int kk = 0; kk < NKK; ++kk) {
+                const u32x4 w = __builtin_bit_cast(u32x4, qf[kk]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    qf[kk][2 * j] = (_Float16)__builtin_bit_cast(float, w[j] << 16);
+                    qf[kk][2 * j + 1] = (_Float16)__builtin_bit_cast(float, w[j] & 0xffff0000u);
+                }
+            }
+        }
+        lds_barrier();
+        f32x16 Sa, Sb;
+        if (wsteps > 0) {
+#pragma unroll
+            for (int kk = 0; kk < NKK; ++kk) Sa = mfma32(read_k(0, kk), qf[kk], kk == 0 ? f32x16{} : Sa);
+            tile_max(Sa, 0);
+        }
+        lds_barrier();
+
+        // step st < ntiles - 1 (ph = st % 2): K(st + 2) replaces K(st), read by the previous step's scores, and
+        // V(st + 1) V(st - 1)
+        auto step = [&](int ph, uint32_t st, f32x16& Scur, f32x16& Snext) {
+            if (st + 2 < ntiles) dma_k(kvh, p0, ph, st + 2);
+            dma_v(kvh, p0, ph ^ 1, st + 1);
+            // opaque each step, or the compiler keeps a second set of offsets for the other buffers (and spills)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(ko[j]));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(vo[j >> 1][j & 1]));
+            f16x8 pf[2];
+            if (st < wsteps) {
+                const float other = Ml[wave ^ 1][lane];
+                f16x8 kf[3];
+                kf[0] = read_k(ph ^ 1, 0);
+                kf[1] = read_k(ph ^ 1, 1);
+                constexpr int NF = 4;  // score MFMAs ahead of the maximum
+#pragma unroll
+                for (int n = 0; n < NF; ++n) {
+                    kf[(n + 2) % 3] = read_k(ph ^ 1, n + 2);
+                    Snext = mfma32(kf[n % 3], qf[n], n == 0 ? f32x16{} : Snext);
+                }
+                rescale(other);
+#pragma unroll
+                for (int n = NF; n < NKK; ++n) {
+                    if (n + 2 < NKK) kf[(n + 2) % 3] = read_k(ph ^ 1, n + 2);
+                    Snext = mfma32(kf[n % 3], qf[n], Snext);
+#pragma unroll
+                    for (int i = 16 * (n - NF) / (NKK - NF); i < 16 * (n - NF + 1) / (NKK - NF); ++i) prob(Scur, pf, i);
+                }
+                Pl[wave][0][lane] = pf[0];
+                Pl[wave][1][lane] = pf[1];
+                pv(pf, ph, 0);
+            }
+            lds_barrier();  // the pair's probabilities are in LDS
+            if (st < wsteps) {
+                f16x8 po[2];
+                po[0] = Pl[wave ^ 1][0][lane];
+                po[1] = Pl[wave ^ 1][1][lane];
+                pv(po, ph, 1);
+                tile_max(Snext, st + 1);
+            }
+            dma_done();
+            lds_barrier();
+        };
+        // the item's last tile: no scores follow, so both K buffers are free and the next item's first loads go out
+        auto last = [&](int ph, uint32_t st, f32x16& Scur) {
+            if (has_next) {
+                issue_k(nxt);
+                if (ph == 1) dma_v(nxt.kvh, 0, 0, 0);
+            }
+            if (p0 / BN + ntiles == kmax / BN + 1 && (kmax + 1) % BN != 0) {  // uniform
+                zero_v_tail(ph);
+                lds_barrier();
+            }
+            f16x8 pf[2];
+            if (st < wsteps) {
+                rescale(Ml[wave ^ 1][lane]);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) prob(Scur, pf, i);
+                Pl[wave][0][lane] = pf[0];
+                Pl[wave][1][lane] = pf[1];
+                pv(pf, ph, 0);
+            }
+            lds_barrier();
+            if (st < wsteps) {
+                f16x8 po[2];
+                po[0] = Pl[wave ^ 1][0][lane];
+                po[1] = Pl[wave ^ 1][1][lane];
+                pv(po, ph, 1);
+            }
+            l = sum_xor32(l);
+            Ml[wave][lane] = l;  // read for the last time before the barrier above
+            lds_barrier();       // and V is read
+            if (has_next && ph == 0) dma_v(nxt.kvh, 0, 0, 0);
+        };
+        uint32_t st = 0;
+        bool odd = false;
+        while (st + 1 < ntiles) {
+            // (opaque: strength reduction of what st indexes took 30 vector registers and spilled)
+            asm volatile("" : "+s"(st));
+            step(0, st, Sa, Sb);
+            if (++st + 1 >= ntiles) {
+                odd = true;
+                break;
+            }
+            step(1, st, Sb, Sa);
+            ++st;
+        }
+        if (odd) last(1, st, Sb);
+        else last(0, st, Sa);
+
+        // Epilogue.  A lane holds four dimensions at a time of one query: stored (and the gate read) like that, an
+        // instruction would touch 32 rows.  V buffer 1 is free (the next item fills it in its first step), so
+        // each wave turns its 32 x 32 blocks of O over in 4 KB of it and then handles 8 rows of 32 dimensions per
+        // instruction.  The gate's loads go out first.
+        {
+            int le;  // the lane afresh, so that nothing of this is kept through the key loop
+            asm volatile("v_mov_b32 %0, %1" : "=v"(le) : "v"((int)threadIdx.x & 63));
+            const int er = le >> 3, ec = le & 7;  // row within a group of 8, four dimensions
+            const uint32_t col = hf * DH + 4 * ec;
+            const bool partial = SPLIT && a.n_split > 1;
+            const bool gated = a.gate && !partial;
+            // rows 8 u + er: the first element written (and of the gate), and whether the row exists
+            size_t at[4], gat[4];
+            bool valid[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const PRow rw = row_of<SPLIT>(a, cur, qw * 32 + 8 * u + er);
+                valid[u] = rw.valid;
+                at[u] = partial ? (((size_t)cur.split * a.n_heads + rw.h) * a.B + rw.b) * D + col
+                                : (size_t)rw.b * a.out_stride + (size_t)rw.h * D + col;
+                gat[u] = (size_t)rw.b * a.gate_stride + (size_t)rw.h * D + col;
+            }
+            f32x4 gt[2][4];
+            auto load_gate = [&](int b) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // gate rows are float-aligned
+                    gt[b & 1][u] = *reinterpret_cast<const f32x4u*>(a.gate + gat[u] + 32 * b);
+                }
+            };
+            if (gated) load_gate(0);
+            l += Ml[wave ^ 1][lane];
+            float inv = 1.0f / l;
+            if (partial) {  // (max, sum) and the unnormalised O of the row over this split's keys
+                inv = 1.0f;
+                const PRow rw = row_of<SPLIT>(a, cur, qw * 32 + (le & 31));
+                if (rw.valid && le < 32 && hf == 0) {
+                    typedef float f32x2 __attribute__((ext_vector_type(2)));
+                    *reinterpret_cast<f32x2*>(a.part_ml + 2 * (((size_t)cur.split * a.n_heads + rw.h) * a.B + rw.b)) =
+                        f32x2{m, l};
+                }
+            }
+            f32x4* area = reinterpret_cast<f32x4*>(&Vl1[0]) + wave * 256;  // [32 rows][8 chunks], swizzled
+#pragma unroll
+            for (int b = 0; b < NDB; ++b) {
+                if (gated && b + 1 < NDB) load_gate(b + 1);
+#pragma unroll
+                for (int i4 = 0; i4 < 4; ++i4) {
+                    f32x4 v;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[e] = o[b][4 * i4 + e] * inv;
+                    area[(le & 31) * 8 + ((2 * i4 + (le >> 5)) ^ (le & 7))] = v;
+                }
+                __builtin_amdgcn_wave_barrier();  // one wave's LDS operations stay in order
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    f32x4 v = area[(8 * u + er) * 8 + (ec ^ er)];
+                    if (gated) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            v[e] *= __builtin_amdgcn_rcpf(1.0f + fast_exp2(gt[b & 1][u][e] * -1.4426950408889634f));
+                    }
+                    if (!valid[u]) continue;
+                    if (partial) *reinterpret_cast<f32x4*>(a.part_o + at[u] + 32 * b) = v;
+                    else store_out4(a.out, at[u] + 32 * b, a.out_dtype, v);
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+        }
+        if (!has_next) break;
+        cur = nxt;
+    }
+}
+
 // One thread per (row, 4 output dimensions) of the split mode: the splits'
 // (max, sum, O) partials of query b of head h are combined in the log2
 // domain, then normalised, gated and stored.  Rows are b * n_heads + h, so a
@@ -1005,19 +1422,24 @@ namespace {
 // threads of a prefill workgroup: 4 waves per key group, 8 in pair mode
 constexpr int prefill_threads(int D, int NG) { return 256 * NG * (D > 128 ? 2 : 1); }
 
-template <int D, int NG, bool QS>
-hipError_t launch_prefill_d(PrefillArgs a, hipStream_t st)
+// the XCD mapping needs whole kv groups per XCD group and an equal share
+// per XCD (measured 470 -> 478 TFLOP/s at 2048 tokens x 28 heads)
+uint32_t xcd_mapped(const PrefillArgs& a)
 {
-    // the XCD mapping needs whole kv groups per XCD group and an equal share
-    // per XCD (measured 470 -> 478 TFLOP/s at 2048 tokens x 28 heads)
     static const int env = [] {
         const char* e = getenv("YHIP_PREFILL_XCD");
         return e ? atoi(e) : 1;
     }();
-    const uint32_t nqb0 = (a.B + BM - 1) / BM;
-    a.xcd_map = env != 0 && a.n_kv <= 8 && 8 % a.n_kv == 0 && a.n_heads % a.n_kv == 0 &&
-                ((uint64_t)nqb0 * (a.n_heads / a.n_kv)) % (8 / a.n_kv) == 0;
-    const uint32_t items = nqb0 * a.n_heads;
+    const uint32_t nqb = (a.B + BM - 1) / BM;
+    return env != 0 && a.n_kv <= 8 && 8 % a.n_kv == 0 && a.n_heads % a.n_kv == 0 &&
+           ((uint64_t)nqb * (a.n_heads / a.n_kv)) % (8 / a.n_kv) == 0;
+}
+
+template <int D, int NG, bool QS>
+hipError_t launch_prefill_d(PrefillArgs a, hipStream_t st)
+{
+    a.xcd_map = xcd_mapped(a);
+    const uint32_t items = (a.B + BM - 1) / BM * a.n_heads;
     // resident workgroups: one round of the grid fills every slot once
     static const int per_cu = [] {
         int n = 0;
@@ -1048,13 +1470,41 @@ hipError_t launch_prefill_d(PrefillArgs a, hipStream_t st)
     return hipGetLastError();
 }
 
+// The split mode at head_dim 256 with 16-bit queries: walks of up to four
+// 32-key tiles stay with prefill_kernel, whose first scores need half the
+// bytes and MFMAs (16 / 2 heads, us with it / with prefill_halves_kernel: 64
+// tokens at 0 12.0 / 14.2, 33 at 100 15.6 / 18.5, four tiles each at 1984 23.0 /
+// 23.2); longer ones are shorter in the other (64 tokens at 16000 54 / 45, 1000
+// at 4000 215 / 98).
+bool split_halves(uint32_t D, uint32_t q_dtype, uint32_t split_tiles)
+{
+    return D > 128 && q_dtype != kF32 && split_tiles > 4;
+}
+
+// one workgroup per CU walking the items in snake order
+hipError_t launch_prefill_halves(PrefillArgs a, hipStream_t st)
+{
+    a.xcd_map = xcd_mapped(a);
+    const uint32_t items = (a.B + BM - 1) / BM * a.n_heads;
+    uint32_t grid = items < (uint32_t)n_cus() ? items : (uint32_t)n_cus();
+    if (a.xcd_map && grid >= 8u) grid = grid / 8u * 8u;  // whole XCD groups (items are a multiple of 8)
+    hipLaunchKernelGGL((prefill_halves_kernel<256, false>), dim3(grid), dim3(512), 0, st, a);
+    return hipGetLastError();
+}
+
 template <int D, bool QS>
 hipError_t launch_prefill_split_d(const PrefillArgs& a, hipStream_t st)
 {
     const uint32_t ipg = a.n_rb * (a.pack ? 1u : a.gmax);
     const uint32_t groups = a.n_kv * a.n_split;
-    const uint32_t grid = (groups + 7u) / 8u * 8u * ipg;
-    hipLaunchKernelGGL((prefill_kernel<D, 1, true, QS>), dim3(grid), dim3(prefill_threads(D, 1)), 0, st, a);
+    const uint32_t grid = (groups * ipg + 7u) / 8u * 8u;  // split_item's order over 8 XCDs
+    bool halves = false;
+    if constexpr (D > 128 && !QS) {
+        halves = split_halves(a.D, a.q_dtype, a.split_tiles);
+        if (halves) hipLaunchKernelGGL((prefill_halves_kernel<D, true>), dim3(grid), dim3(512), 0, st, a);
+    }
+    if (!halves)
+        hipLaunchKernelGGL((prefill_kernel<D, 1, true, QS>), dim3(grid), dim3(prefill_threads(D, 1)), 0, st, a);
     if (a.n_split > 1) {
         const uint64_t threads = (uint64_t)a.B * a.n_heads * (D / 4);
         hipLaunchKernelGGL(prefill_merge_kernel<D>, dim3((uint32_t)((threads + 255) / 256)), dim3(256), 0, st, a);
@@ -1146,12 +1596,38 @@ size_t prefill_plan(PrefillArgs& a)
     split_shape(a.B, a.n_heads, a.n_kv, a.D, a.pack, a.n_rb, a.gmax, base, target);
     a.split_mode = 1;
     const uint32_t ntiles = (a.pos_start + a.B - 1) / bn_of((int)a.D) + 1;
-    uint64_t S = target / base;
-    if (S > t.max_split) S = t.max_split;
+    uint64_t most = target / base;
+    if (most > t.max_split) most = t.max_split;
     const uint32_t by_tiles = (ntiles + t.min_tiles - 1) / t.min_tiles;
-    if (S > by_tiles) S = by_tiles;
-    if (S < 1) S = 1;
+    if (most > by_tiles) most = by_tiles;
+    // Of up to `most` splits, the number with the least cost: the walk of the
+    // longest split (us per 64 keys, half again as long with two workgroups on
+    // a CU) and, from two on, the merge launch and the partials written and
+    // read (1.4 us, 5 TB/s; 28 / 4 heads of 128, f16: 1000 tokens 25.6 us
+    // unsplit, 34.4 in two; f32 38 and 55; 64 tokens at 1984 16 us in eight;
+    // 2 tokens at 300 11.8 unsplit, 9.7 in two).
+    const float per64 = (0.35f + (float)a.D / 160.0f) * (a.q_dtype == kF32 ? 1.6f : 1.0f);
+    const float rows_us = (float)a.n_heads * a.B * a.D * 8.0f / 5.0e6f;
+    uint64_t S = 1;
+    float best = 0.0f;
+    for (uint64_t n = 1; n <= most; ++n) {
+        const float walk = (float)((ntiles + n - 1) / n * bn_of((int)a.D)) / 64.0f * per64;
+        const float cost = walk * (base * n > (uint64_t)n_cus() ? 1.5f : 1.0f) + (n > 1 ? 1.4f + rows_us * n : 0.0f);
+        if (n == 1 || cost < best) {
+            best = cost;
+            S = n;
+        }
+    }
+    // An unsplit launch of whole query blocks over 512 keys or more runs the
+    // plain mode (two key groups for 16-bit queries up to d 128): 1000 tokens
+    // 24.9 against 25.6 us, 14 / 2 heads of 64 16.6 against 17.4.
+    if (S == 1 && !a.pack && ntiles * bn_of((int)a.D) >= 512) {
+        a.split_mode = 0;
+        return 0;
+    }
     a.split_tiles = (ntiles + (uint32_t)S - 1) / (uint32_t)S;
+    // prefill_halves_kernel walks pairs of 32-key tiles
+    if (split_halves(a.D, a.q_dtype, a.split_tiles)) a.split_tiles += a.split_tiles & 1u;
     a.n_split = (ntiles + a.split_tiles - 1) / a.split_tiles;
     return split_bytes(a.n_split, a.B, a.n_heads, a.D);
 }
@@ -1207,7 +1683,7 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t st)
     case 128:
         return qs ? launch_prefill_d<128, 1, true>(a, st)
                   : ng == 2 ? launch_prefill_d<128, 2, false>(a, st) : launch_prefill_d<128, 1, false>(a, st);
-    case 256: return qs ? launch_prefill_d<256, 1, true>(a, st) : launch_prefill_d<256, 1, false>(a, st);
+    case 256: return qs ? launch_prefill_d<256, 1, true>(a, st) : launch_prefill_halves(a, st);
     default: return hipErrorInvalidValue;
     }
 }
