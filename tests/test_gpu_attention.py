@@ -669,6 +669,13 @@ def _prefill_f64(q, cache, start, nh, gate=None):
     (14, 2, 64, 1500, 0, "f16", "f32", False),
     (14, 2, 64, 700, 3000, "f32", "f32", False),
     (28, 4, 128, 700, 0, "f32", "f32", False),
+    # fp32 queries on two key groups: lo parts in LDS, several items per workgroup, a group without tiles, split walks
+    (32, 8, 128, 1100, 0, "f32", "f32", False),
+    (40, 5, 128, 1000, 30, "f32", "f16", True),
+    (56, 4, 64, 640, 3, "f32", "f32", True),
+    (14, 2, 64, 2500, 0, "f32", "bf16", False),
+    (28, 4, 128, 64, 3000, "f32", "f32", True),
+    (14, 2, 64, 40, 5000, "f32", "f32", False),
     (15, 3, 128, 140, 900, "bf16", "f32", False),
     (5, 5, 64, 70, 800, "f16", "f32", True),
 ])

@@ -60,35 +60,22 @@ __device__ inline int lds_row_of_key(int r)
 // key (within a 32-key half) of accumulator element i for lane half hh
 __device__ inline int key_of_acc(int i, int hh) { return i < 8 ? 8 * hh + i : 16 + 8 * hh + (i - 8); }
 
-__device__ inline void load_q8(f16x8& dst, const void* q, size_t off, uint32_t dt)
+// 8 bf16 queries, as loaded, to f16
+__device__ inline void bf16_to_f16(f16x8& q)
 {
-    if (dt == kF32) {
-        const f32x4 a = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(q) + off);
-        const f32x4 b = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(q) + off + 4);
+    const u32x4 w = __builtin_bit_cast(u32x4, q);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            dst[j] = (_Float16)a[j];
-            dst[j + 4] = (_Float16)b[j];
-        }
-    } else if (dt == kF16) {
-        dst = *reinterpret_cast<const f16x8*>(reinterpret_cast<const uint16_t*>(q) + off);
-    } else {
-        const u32x4 w = *reinterpret_cast<const u32x4*>(reinterpret_cast<const uint16_t*>(q) + off);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            dst[2 * j] = (_Float16)__builtin_bit_cast(float, w[j] << 16);
-            dst[2 * j + 1] = (_Float16)__builtin_bit_cast(float, w[j] & 0xffff0000u);
-        }
+    for (int j = 0; j < 4; ++j) {
+        q[2 * j] = (_Float16)__builtin_bit_cast(float, w[j] << 16);
+        q[2 * j + 1] = (_Float16)__builtin_bit_cast(float, w[j] & 0xffff0000u);
     }
 }
 
-// fp32 query elements off..off+7 as f16 hi + lo parts: hi = f16(x), lo =
-// f16(x - hi), so hi + lo carries ~22 bits of x and K.hi + K.lo (two MFMAs
-// into one fp32 accumulator) keeps the score at fp32-level error
-__device__ inline void load_q8_split(f16x8& hi, f16x8& lo, const float* q, size_t off)
+// 8 fp32 query elements as f16 hi + lo parts: hi = f16(x), lo = f16(x - hi),
+// so hi + lo carries ~22 bits of x and K.hi + K.lo (two MFMAs into one fp32
+// accumulator) keeps the score at fp32-level error
+__device__ inline void split_q8(f16x8& hi, f16x8& lo, const f32x4& a, const f32x4& b)
 {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(q + off);
-    const f32x4 b = *reinterpret_cast<const f32x4*>(q + off + 4);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         hi[j] = (_Float16)a[j];
@@ -335,16 +322,18 @@ __device__ inline bool split_item(const PrefillArgs& a, PItem& I)
 
 // SPLIT: the split mode (one item per workgroup, packed rows, a key range
 // per split); a separate instantiation keeps the plain mode's registers.
-// QS: fp32 queries as f16 hi + lo parts, two score MFMAs per k-chunk (32 more
-// registers per lane at d = 128: one workgroup of 4 waves per CU, one key
-// group).
+// QS: fp32 queries as f16 hi + lo parts, two score MFMAs per k-chunk.  With
+// two key groups the lo parts live in LDS (both groups read the same ones; the
+// 160 KB are full at d = 128) instead of 32 registers, so that two waves share
+// a SIMD.
 template <int D, int NG, bool SPLIT, bool QS = false>
 __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 && !QS) ? 2 : 1) void prefill_kernel(
     PrefillArgs a)
 {
     static_assert(NG == 1 || NG == 2, "one or two key groups");
-    static_assert(!SPLIT || NG == 1, "the split mode runs one key group");
-    static_assert(!QS || NG == 1, "split queries run one key group");
+    static_assert(!SPLIT || NG == 1 || QS, "the split mode of 16-bit queries runs one key group");
+    // QL: the queries' lo parts in LDS (fragment order) instead of 32 registers
+    constexpr bool QL = QS && NG == 2;
     // Pair mode (head_dim 256): a wave's 32 queries with all 256 dimensions
     // need 64 registers of Q and 128 of O, which leaves one wave per SIMD.
     // Instead two waves share 32 queries and each owns half the dimensions
@@ -396,8 +385,10 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
     // [parity][wave][float4 j][lane] (consecutive lanes, consecutive 16
     // bytes).  Two key groups: (max, sum) of group 1's queries for the merge.
     // (One array: pair mode fills the 160 KB of LDS exactly.)
-    __shared__ f32x4 Xl[PAIR ? 2 * 8 * 4 * NS * 64 : NG > 1 ? 128 : 1];
-    float* const s_ml = reinterpret_cast<float*>(&Xl[0]);
+    __shared__ f32x4 Xl[PAIR ? 2 * 8 * 4 * NS * 64 : NG > 1 && !QL ? 128 : 1];
+    // [query wave][k-chunk][lane]; between items it holds (max, sum) for the merge
+    __shared__ f16x8 Qlo[QL ? 4 : 1][QL ? NKK : 1][QL ? 64 : 1];
+    float* const s_ml = QL ? reinterpret_cast<float*>(&Qlo[0][0][0]) : reinterpret_cast<float*>(&Xl[0]);
 
     // Items (query block, head) in heaviest-first order are dealt to the
     // resident workgroups in snake order (item slot it*W + j on even rounds,
@@ -492,7 +483,7 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
             else __builtin_amdgcn_s_waitcnt(0x0f70);
         };
         f16x8 qf[NKK];
-        f16x8 ql[QS ? NKK : 1];  // QS: the lo parts
+        f16x8 ql[QS && !QL ? NKK : 1];  // QS: the lo parts
         // the first loads of an item, see above: the K tiles, the first V
         // tile and the queries
         auto item_steps = [&](const PItem& I, uint32_t& t0) {
@@ -508,7 +499,7 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
             if (igsteps > 1) dma_k_of(rk, 1, t0 + grp + NG);
         };
         auto issue_item_q = [&](const PItem& I) {
-            if (a.q_dtype == kF16) {
+            if constexpr (!QS) {  // bf16 as it is, converted when the item starts
                 const PRow rw = row_of<SPLIT>(a, I, qw * 32 + r32);
                 const uint16_t* qp = reinterpret_cast<const uint16_t*>(a.q) + (size_t)rw.b * a.q_stride +
                                      (size_t)rw.h * D + hf * DQ + hh * 8;
@@ -625,16 +616,23 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
 #pragma unroll
             for (int i = 0; i < 16; ++i) o[b][i] = 0.0f;
 
+        auto read_lo = [&](int kk) {
+            if constexpr (QL) return Qlo[qw][kk][lane];
+            else return ql[QS ? kk : 0];
+        };
         // scores of the tile in K buffer P into S (its 32-key halves)
         auto qk = [&](f32x16 (&S)[NS], int par) {
 #pragma unroll
-            for (int kk = 0; kk < NKK; ++kk)
+            for (int kk = 0; kk < NKK; ++kk) {
+                f16x8 lf;
+                if constexpr (QS) lf = read_lo(kk);
 #pragma unroll
                 for (int j = 0; j < NS; ++j) {
                     const f16x8 kf = read_k(par, j, kk);
                     S[j] = kk == 0 ? mfma32(kf, qf[0], f32x16{}) : mfma32(kf, qf[kk], S[j]);
-                    if constexpr (QS) S[j] = mfma32(kf, ql[kk], S[j]);
+                    if constexpr (QS) S[j] = mfma32(kf, lf, S[j]);
                 }
+            }
         };
         // running max update of the lane's query from tile scores S (raw, masked)
         auto update_max = [&](const f32x16 (&S)[NS]) {
@@ -687,9 +685,11 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
             constexpr FusedSchedule<NQ, NPV, NDB, NKC> sch{};
             constexpr int MAXP = 8;
             const float nm = -m;
-            f16x8 pf[NKC], kf[3], vf[3];
+            constexpr int KR = QL ? 2 : 3;  // K ring: read two MFMAs ahead (a score slot of split queries has two)
+            f16x8 pf[NKC], kf[KR], vf[3], lf[2];
             kf[0] = read_k(kpar, 0, 0);
-            kf[1] = read_k(kpar, 1 % NS, 1 / NS);
+            if constexpr (!QL) kf[1] = read_k(kpar, 1 % NS, 1 / NS);
+            if constexpr (QL) lf[0] = read_lo(0);
             vf[0] = read_v(vpar, 0, 0);
             vf[1] = read_v(vpar, 1 % NDB, 1 / NDB);
 #pragma unroll
@@ -699,10 +699,13 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
                     if (n + 2 < NPV) vf[(n + 2) % 3] = read_v(vpar, (n + 2) % NDB, (n + 2) / NDB);
                     o[n % NDB] = mfma32(vf[n % 3], pf[n / NDB], o[n % NDB]);
                 } else {
-                    if (n + 2 < NQ) kf[(n + 2) % 3] = read_k(kpar, (n + 2) % NS, (n + 2) / NS);
-                    Snext[n % NS] = n < NS ? mfma32(kf[n % 3], qf[0], f32x16{})
-                                           : mfma32(kf[n % 3], qf[n / NS], Snext[n % NS]);
-                    if constexpr (QS) Snext[n % NS] = mfma32(kf[n % 3], ql[n / NS], Snext[n % NS]);
+                    if (n + KR - 1 < NQ) kf[(n + KR - 1) % KR] = read_k(kpar, (n + KR - 1) % NS, (n + KR - 1) / NS);
+                    if constexpr (QL)
+                        if (n % NS == 0 && n / NS + 1 < NKK) lf[(n / NS + 1) & 1] = read_lo(n / NS + 1);
+                    Snext[n % NS] = n < NS ? mfma32(kf[n % KR], qf[0], f32x16{})
+                                           : mfma32(kf[n % KR], qf[n / NS], Snext[n % NS]);
+                    if constexpr (QL) Snext[n % NS] = mfma32(kf[n % KR], lf[(n / NS) & 1], Snext[n % NS]);
+                    else if constexpr (QS) Snext[n % NS] = mfma32(kf[n % KR], ql[n / NS], Snext[n % NS]);
                 }
 #pragma unroll
                 for (int u = 0; u < MAXP; ++u) {
@@ -729,19 +732,27 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
         };
 
         // prologue: this item's first loads are in flight (issued above or at the
-        // end of the previous item); f32 and bf16 queries are loaded and
-        // converted here.  All loads are complete before the key loop, whose
+        // end of the previous item); bf16 queries are converted here, f32 ones loaded
+        // and split (prefetched like the others they spilled: 2048 tokens 63 -> 79 us).  All loads are complete before the key loop, whose
         // waits then count only tile loads (in pair mode K(2) and V(1) may
         // still be in flight; the first step waits for them).
         dma_wait_but(deep_loads);
-        if (a.q_dtype != kF16) {
-            const size_t qbase = (size_t)myrow.b * a.q_stride + (size_t)myrow.h * D + hf * DQ + hh * 8;
+        if (QL && it > 0) lds_barrier();  // the merge has read (max, sum)
+        if constexpr (QS) {
+            const float* qp = reinterpret_cast<const float*>(a.q) + (size_t)myrow.b * a.q_stride + (size_t)myrow.h * D +
+                              hf * DQ + hh * 8;
 #pragma unroll
             for (int kk = 0; kk < NKK; ++kk) {
-                if constexpr (QS) load_q8_split(qf[kk], ql[kk], reinterpret_cast<const float*>(a.q), qbase + kk * 16);
-                else load_q8(qf[kk], a.q, qbase + kk * 16, a.q_dtype);
+                f16x8 lo;
+                split_q8(qf[kk], lo, *reinterpret_cast<const f32x4*>(qp + kk * 16),
+                         *reinterpret_cast<const f32x4*>(qp + kk * 16 + 4));
+                if constexpr (!QL) ql[kk] = lo;
+                else if (grp == 0) Qlo[qw][kk][lane] = lo;  // both groups hold the same queries
             }
             if (NB == 2) dma_done();
+        } else if (a.q_dtype == kBF16) {
+#pragma unroll
+            for (int kk = 0; kk < NKK; ++kk) bf16_to_f16(qf[kk]);
         }
         if constexpr (NB > 2) lds_barrier();
         else __syncthreads();
@@ -1155,14 +1166,7 @@ __global__ __launch_bounds__(512) void prefill_halves_kernel(PrefillArgs a)
         dma_done();
         if (a.q_dtype == kBF16) {
 #pragma unroll
-            for (int kk = 0; kk < NKK; ++kk) {
-                const u32x4 w = __builtin_bit_cast(u32x4, qf[kk]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    qf[kk][2 * j] = (_Float16)__builtin_bit_cast(float, w[j] << 16);
-                    qf[kk][2 * j + 1] = (_Float16)__builtin_bit_cast(float, w[j] & 0xffff0000u);
-                }
-            }
+            for (int kk = 0; kk < NKK; ++kk) bf16_to_f16(qf[kk]);
         }
         lds_barrier();
         f32x16 Sa, Sb;
@@ -1503,7 +1507,15 @@ hipError_t launch_prefill_split_d(const PrefillArgs& a, hipStream_t st)
         halves = split_halves(a.D, a.q_dtype, a.split_tiles);
         if (halves) hipLaunchKernelGGL((prefill_halves_kernel<D, true>), dim3(grid), dim3(512), 0, st, a);
     }
-    if (!halves)
+    bool two = false;
+    if constexpr (D <= 128 && QS) {
+        // fp32 queries: two key groups from four tiles per split on (28 / 4 heads of 128, us with one / two: 64
+        // tokens at 0 10.2 / 12.0, at 1000 20.3 / 19.6, at 16000 47 / 40, 400 at 2000 57 / 49); at d 64, where a CU
+        // holds two workgroups of one group, only while the grid leaves it at one (400 at 2000 22.4 / 26.7)
+        two = a.split_tiles >= 4 && (D == 128 || grid <= (uint32_t)n_cus());
+        if (two) hipLaunchKernelGGL((prefill_kernel<D, 2, true, QS>), dim3(grid), dim3(prefill_threads(D, 2)), 0, st, a);
+    }
+    if (!halves && !two)
         hipLaunchKernelGGL((prefill_kernel<D, 1, true, QS>), dim3(grid), dim3(prefill_threads(D, 1)), 0, st, a);
     if (a.n_split > 1) {
         const uint64_t threads = (uint64_t)a.B * a.n_heads * (D / 4);
@@ -1529,6 +1541,11 @@ int prefill_groups(const PrefillArgs& a)
     if (a.D > 128) return 1;
     if (env == 1 || env == 2) return env;
     const uint64_t wgs = (uint64_t)((a.B + BM - 1) / BM) * a.n_heads;
+    // fp32 queries: at d 128 always two (one group alone, 352 registers, is one
+    // wave per SIMD: 28 / 4 heads, 2048 tokens 80 -> 68 us, 6000 478 -> 410); at
+    // d 64 one workgroup per CU or less gains nothing from it (14 / 2 heads, 1500
+    // tokens 29.7 / 30.3, 3000 59 -> 44, 6000 130 either way)
+    if (a.q_dtype == kF32) return a.D == 128 || (wgs > (uint64_t)n_cu && wgs <= 2 * (uint64_t)n_cu) ? 2 : 1;
     return wgs <= 2 * (uint64_t)n_cu ? 2 : 1;
 }
 
@@ -1665,7 +1682,7 @@ void prefill_bind_workspace(PrefillArgs& a, void* workspace)
 
 hipError_t launch_prefill(const PrefillArgs& a, hipStream_t st)
 {
-    // fp32 queries keep fp32-level scores (hi + lo parts, one key group)
+    // fp32 queries keep fp32-level scores (hi + lo parts)
     const bool qs = a.q_dtype == kF32;
     if (a.split_mode) {
         switch (a.D) {
@@ -1678,10 +1695,10 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t st)
     const int ng = prefill_groups(a);
     switch (a.D) {
     case 64:
-        return qs ? launch_prefill_d<64, 1, true>(a, st)
+        return qs ? (ng == 2 ? launch_prefill_d<64, 2, true>(a, st) : launch_prefill_d<64, 1, true>(a, st))
                   : ng == 2 ? launch_prefill_d<64, 2, false>(a, st) : launch_prefill_d<64, 1, false>(a, st);
     case 128:
-        return qs ? launch_prefill_d<128, 1, true>(a, st)
+        return qs ? launch_prefill_d<128, 2, true>(a, st)
                   : ng == 2 ? launch_prefill_d<128, 2, false>(a, st) : launch_prefill_d<128, 1, false>(a, st);
     case 256: return qs ? launch_prefill_d<256, 1, true>(a, st) : launch_prefill_halves(a, st);
     default: return hipErrorInvalidValue;
