@@ -87,6 +87,7 @@ def test_o_proj_f16_attention_output(cuda, oracle, B):
 
 @pytest.mark.parametrize("att16", [False, True], ids=["f32att", "f16att"])
 @pytest.mark.parametrize("B,hidden,qdim", [
+    (3, 40, 72), (5, 1000, 904), (8, 56, 4200),  # rows kernel, f32 products up to 8 f32 tokens
     (16, 896, 896), (17, 40, 264), (33, 1000, 4104), (63, 48, 4200),  # rows kernel: 16-token blocks, ragged K, two rounds
     (65, 300, 72), (250, 1100, 40),       # 64 x 64 tiles, fewer K steps than LDS stages
     (520, 1540, 360),                     # 64 x 128 tiles (f16 too), partial in both directions
@@ -114,6 +115,21 @@ def test_o_proj_tile_edges(cuda, B, hidden, qdim, att16):
         + 2.0 ** -23 * want.abs() + 2.0 ** -23 * x0[:, :hidden].double().abs()
     assert ((x[:, :hidden].double() - want).abs() <= bound).all()
     assert torch.equal(x[:, hidden:], x0[:, hidden:])
+
+
+@pytest.mark.parametrize("att16", [False, True], ids=["f32att", "f16att"])
+def test_o_proj_few_large_tokens(cuda, att16):
+    """Up to 8 f32 tokens keep f32 products: values past f16's range stay finite."""
+    from yllm_amd.attention import o_proj
+
+    g = torch.Generator(device="cuda").manual_seed(6)
+    att = torch.randn(8, 128, generator=g, device=cuda) * (1000.0 if att16 else 1e6)
+    att = att.half() if att16 else att
+    w = torch.randn(80, 128, generator=g, device=cuda).half()
+    x = torch.zeros(8, 80, device=cuda)
+    want = att.double() @ w.double().t()
+    o_proj(x, att, w)
+    assert float((x.double() - want).norm() / want.norm()) <= 1e-6
 
 
 @pytest.mark.parametrize("att16", [False, True], ids=["f32att", "f16att"])

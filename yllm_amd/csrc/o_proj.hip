@@ -4,14 +4,15 @@
 //
 // W_o is [hidden][qdim] (f16 or f32), att [B][qdim] f32 (or f16 when the
 // attention kernel wrote f16; f16 att takes f16 weights), x [B][hidden] f32.
-//  * Few tokens (decode, B <= kGemvRows): oproj_gemv_kernel reads W_o once
-//    from HBM and applies it to all B rows; activations stay f32 and every
+//  * Few tokens (decode, B <= kGemvRows; with f16 weights up to 2 f16 or 4 f32
+//    tokens): oproj_gemv_kernel reads W_o once from HBM and applies it to all
+//    B rows; activations stay f32 and every
 //    product and sum is f32 (the reference's arithmetic, summed in another
 //    order).  A wave owns kRows output rows; its lanes take 8 consecutive
 //    inputs each (16-byte weight loads at f16), eight iterations of loads in
 //    flight (all of a 4096-wide row), then a shuffle reduction and the
 //    residual add.
-//  * 9 to kRowsMax tokens with f16 weights (the engine's 64-token prefill calls):
+//  * Then up to kRowsMax tokens with f16 weights (the engine's 64-token prefill calls):
 //    oproj_rows_kernel streams W_o through MFMA, a workgroup per 16 output
 //    rows and its waves splitting the contraction.
 //  * More tokens: oproj_gemm_kernel, an f16 MFMA GEMM with f32 accumulation
@@ -212,9 +213,14 @@ __device__ inline void split_raw(const Raw<F32>& raw, f16x8& hi, f16x8& lo)
 // wave order, so the result does not depend on timing.  3584 x 3584, us for 64
 // / 32 / 16 f32 tokens: 18.7 / 14.4 / 12.0; the 64 x 64 GEMM tiles before it
 // (56 workgroups, 224 steps each, and a launch to split att) took 79.
-template <int NT, bool AF32>
+//
+// X32 (f32 tokens, up to kGemvRows of them): the products stay f32, on the
+// f32 MFMA (k-slot g of MFMA e is k 8 g + e), with the one-pass kernel's range
+// and error; 8 x 16 cycles more per step than the f16 parts, under the loads.
+template <int NT, bool AF32, bool X32 = false>
 __global__ __launch_bounds__(512, 1) void oproj_rows_kernel(OProjArgs a)
 {
+    static_assert(!X32 || (AF32 && NT == 1), "a few f32 tokens");
     constexpr int EB = AF32 ? 4 : 2, CPR = kBK * EB / 16;  // bytes per element, chunks per row of 32 k
     constexpr int SB = NT * 16 * kBK * EB;                 // bytes of a stage: 16 NT rows
     constexpr int NLD = SB / 1024;                         // loads per lane and step
@@ -255,6 +261,11 @@ __global__ __launch_bounds__(512, 1) void oproj_rows_kernel(OProjArgs a)
     f32x4 acc[NT];
 #pragma unroll
     for (int b = 0; b < NT; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // 16 tokens and fewer: more accumulators, for shorter sums (the one-pass kernel's error, and no longer chain)
+    constexpr int NX = X32 ? 8 : NT == 1 ? 2 : 1;
+    f32x4 accx[NX];
+#pragma unroll
+    for (int e = 0; e < NX; ++e) accx[e] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     for (uint32_t r0 = 0; r0 < n; r0 += RW) {
         // step i of the round covers k0 .. k0 + 31; past this wave's steps and past K every load reads zeros
@@ -308,16 +319,25 @@ __global__ __launch_bounds__(512, 1) void oproj_rows_kernel(OProjArgs a)
                 asm volatile("" ::: "memory");
                 issue(i + kDep);
             }
+            if constexpr (X32) {
 #pragma unroll
-            for (int b = 0; b < NT; ++b) {
-                f16x8 hi, lo;
-                split_raw<AF32>(raw[b], hi, lo);
-                acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, w[i], acc[b], 0, 0, 0);
-                if (AF32) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, w[i], acc[b], 0, 0, 0);
+                for (int e = 0; e < 8; ++e)
+                    accx[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(raw[0].v[e / 4][e % 4], (float)w[i][e], accx[e], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int b = 0; b < NT; ++b) {
+                    f16x8 hi, lo;
+                    split_raw<AF32>(raw[b], hi, lo);
+                    f32x4& c = NT == 1 ? accx[i & 1] : acc[b];
+                    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, w[i], c, 0, 0, 0);
+                    if (AF32) c = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, w[i], c, 0, 0, 0);
+                }
             }
         }
         wait_vm<0>();  // nothing in flight into the ring before it is used again
     }
+    if constexpr (X32) acc[0] = ((accx[0] + accx[1]) + (accx[2] + accx[3])) + ((accx[4] + accx[5]) + (accx[6] + accx[7]));
+    else if constexpr (NT == 1) acc[0] = accx[0] + accx[1];
     __syncthreads();
     f32x4* red = reinterpret_cast<f32x4*>(&ring[0][0][0]);  // [wave][block][lane]
 #pragma unroll
@@ -637,8 +657,21 @@ size_t oproj_workspace(uint32_t B, uint32_t qdim, uint32_t w_f16, uint32_t att_f
 
 const char* launch_oproj(const OProjArgs& a, void* ws, size_t ws_bytes, hipStream_t st)
 {
+    // the MFMA kernels address a tile's rows with 32-bit byte offsets
+    const bool near = 256ull * 4 * (a.att_stride > a.qdim ? a.att_stride : a.qdim) < 0xf0000000ull;
     if (a.B <= kGemvRows) {
         hipError_t e;
+        // f16 weights, from 3 f16 or 5 f32 tokens on: the rows kernel reads each token row once per 16 output rows, the
+        // one-pass kernel once per two (4096 x 4096, us one-pass / rows: f16 2 tokens 11.8 / 10.2, 3 13.6 / 10.2, 8 22.4 /
+        // 10.9; f32 4 14.4 / 13.8, 5 15.8 / 13.9, 8 19.6 / 14.2; 896 x 896 f16 2 4.0 / 4.5, 3 4.8 / 4.6, f32 4 5.1 / 5.4,
+        // 5 6.0 / 5.4)
+        if (a.w_f16 && a.B >= (a.att_f16 ? 3u : 5u) && near) {
+            const dim3 grid((a.hidden + 15) / 16);
+            if (a.att_f16) hipLaunchKernelGGL((oproj_rows_kernel<1, false>), grid, dim3(512), 0, st, a);
+            else hipLaunchKernelGGL((oproj_rows_kernel<1, true, true>), grid, dim3(512), 0, st, a);
+            e = hipGetLastError();
+            return e == hipSuccess ? nullptr : hipGetErrorString(e);
+        }
         if (a.w_f16)
             e = a.att_f16 ? launch_gemv<1, 1>(a, st) : launch_gemv<1, 0>(a, st);
         else
@@ -647,10 +680,8 @@ const char* launch_oproj(const OProjArgs& a, void* ws, size_t ws_bytes, hipStrea
     }
     (void)ws;
     (void)ws_bytes;
-    // the MFMA kernels address a tile's rows with 32-bit byte offsets; rows too
-    // long for that go through the one-pass kernel, eight tokens at a time
-    const uint64_t row = 4ull * (a.att_stride > a.qdim ? a.att_stride : a.qdim);
-    if (256u * row >= 0xf0000000ull) {
+    // rows too long for the MFMA kernels go through the one-pass kernel, eight tokens at a time
+    if (!near) {
         for (uint32_t b0 = 0; b0 < a.B; b0 += kGemvRows) {
             OProjArgs p = a;
             p.B = a.B - b0 < kGemvRows ? a.B - b0 : kGemvRows;
