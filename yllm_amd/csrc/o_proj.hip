@@ -378,9 +378,9 @@ __global__ __launch_bounds__(512, 1) void oproj_rows_kernel(OProjArgs a)
 // half's MFMAs issue while the next step's first fragments are read and the
 // loads four steps ahead go into the stage just read.  The four stages are
 // separate variables and the loop is unrolled by four, so the compiler sees
-// that loads in flight never alias the reads.  The residual is added with one
-// float atomic add per element at L2 (one add per element, so the result is
-// the load, add and store's), which keeps x's read off the kernel's tail.
+// loads in flight never alias the reads.  f16 8192 x 4096 x 4096 350 -> 265 us
+// (1040 TFLOP/s; 1250 in the loop alone), f32 att 2048 x 3584 x 3584 193 + 15 for
+// the split pass -> 100.
 struct GemmArgs {
     const char* t;  // token rows
     const char* w;  // W_o rows, ld K
@@ -528,6 +528,23 @@ __global__ __launch_bounds__(256, WPC) void oproj_gemm_kernel(GemmArgs a)
     constexpr int NMF = TM * TN * (1 + AF32 + WF32);              // MFMAs per half step
     constexpr int NRD = TM * (AF32 ? 2 : 1) + TN * (WF32 ? 2 : 1);  // fragment reads per half step
 
+    // the residual of a whole tile: accumulator (m, n, i) is token 32 m + 8 (i /
+    // 4) + i % 4 + 4 hh of the wave's, output 32 n + r32: a scalar row and a lane
+    // offset
+    const bool whole = nt == (uint32_t)BT && no == (uint32_t)BO;  // workgroup-uniform
+    float* const xw = a.x + (size_t)(t0 + wt * TM * 32) * a.x_stride + o0 + wo * TN * 32;
+    const uint32_t xlane = 4u * hh * a.x_stride + r32;
+    auto x_row = [&](int m, int i) { return xw + (size_t)(32 * m + 8 * (i / 4) + i % 4) * a.x_stride; };
+    float xv[2][16][TN];
+    auto load_x = [&](int m) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+#pragma unroll
+            for (int n = 0; n < TN; ++n) xv[m & 1][i][n] = x_row(m, i)[xlane + 32 * n];
+    };
+    constexpr bool kEarlyX = TM < 4;  // (256 x 256 tiles have no registers left for it and spilled: 271 -> 362 us)
+    if (kEarlyX && whole) load_x(0);
+
     Frags f0, f1;
 #pragma unroll
     for (int s = 0; s < kStages; ++s) {
@@ -558,20 +575,33 @@ __global__ __launch_bounds__(256, WPC) void oproj_gemm_kernel(GemmArgs a)
     }
     wait_vm<0>();  // the loads past the end land before the workgroup ends
 
-    // x[t][o] += acc with float atomics at L2 (each element receives one
-    // add: the result equals a load, add and store), no load of x on the way
-    float* xp = a.x + (size_t)t0 * a.x_stride + o0;
-    const uint32_t tb = wt * TM * 32 + 4 * hh, ob = wo * TN * 32 + r32;
-    const bool whole = nt == (uint32_t)BT && no == (uint32_t)BO;  // workgroup-uniform
+    // x[t][o] += acc.  Whole tiles: the loads of one row of blocks ahead of
+    // the adds and stores of the one before, the first row's from before the K
+    // loop where they fit (as float atomics the epilogue took three times as
+    // long: 8192 x 4096 x 4096, f16, 312 -> 265 us).  Partial tiles, where each access has its own
+    // bounds test: float atomics, which nothing waits for (one add per element,
+    // so the result is the load, add and store's).
+    if (whole) {
+        if (!kEarlyX) load_x(0);
+#pragma unroll
+        for (int m = 0; m < TM; ++m) {
+            if (m + 1 < TM) load_x(m + 1);
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+#pragma unroll
+                for (int n = 0; n < TN; ++n) x_row(m, i)[xlane + 32 * n] = xv[m & 1][i][n] + acc[m][n][i];
+        }
+        return;
+    }
 #pragma unroll
     for (int m = 0; m < TM; ++m)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            const uint32_t t = tb + 32 * m + 8 * (i / 4) + i % 4;
-            float* row = xp + (size_t)t * a.x_stride + ob;
+            const uint32_t t = wt * TM * 32 + 4 * hh + 32 * m + 8 * (i / 4) + i % 4, o = wo * TN * 32 + r32;
+            float* row = a.x + (size_t)(t0 + t) * a.x_stride + o0;
 #pragma unroll
             for (int n = 0; n < TN; ++n)
-                if (whole || (t < nt && ob + 32u * n < no)) unsafeAtomicAdd(row + 32 * n, acc[m][n][i]);
+                if (t < nt && o + 32u * n < no) unsafeAtomicAdd(row + o + 32 * n, acc[m][n][i]);
         }
 }
 
@@ -588,11 +618,12 @@ hipError_t launch_gemm_tiles(const GemmArgs& a, hipStream_t st)
 // Tile choice: the largest tile of which there are enough for three quarters
 // of the CUs.  A larger tile moves fewer LDS and L2 bytes per MFMA, but one
 // workgroup per CU cannot fill a chip of which it leaves a quarter idle.
-// f16 att, 4096 x 4096, us with 256 x 256 / 128 x 256 / 128 x 128 / 64 x 128 /
-// 64 x 64 tiles: 8192 tokens 320 / 359 / 372, 2048 tokens 108 / 96 / 104, 1024
-// 96 / 72 / 55 / 73 / 85, 512 - / 66 / 47 / 43 / 47, 256 - / - / 44 / 39 / 29.
-// f32 att, 3584 x 3584, 128 x 256 / 64 x 128 / 64 x 64: 2048 tokens 118 / 147,
-// 1024 90 / 76 / 99, 512 85 / 45 / 55, 256 (4096 x 4096) - / 44 / 39.
+// (With the residual still added by atomics) f16 att, 4096 x 4096, us with 256 x
+// 256 / 128 x 256 / 128 x 128 / 64 x 128 / 64 x 64 tiles: 8192 tokens 320 / 359 /
+// 372, 2048 tokens 108 / 96 / 104, 1024 96 / 72 / 55 / 73 / 85, 512 - / 66 / 47 /
+// 43 / 47, 256 - / - / 44 / 39 / 29.  f32 att, 3584 x 3584, 128 x 256 / 64 x 128 /
+// 64 x 64: 2048 tokens 118 / 147, 1024 90 / 76 / 99, 512 85 / 45 / 55, 256 (4096 x
+// 4096) - / 44 / 39.
 hipError_t launch_gemm(const GemmArgs& a, bool af32, bool wf32, hipStream_t st)
 {
     const uint64_t enough = (uint64_t)n_cus() * 3 / 4;
