@@ -634,12 +634,12 @@ __global__ __launch_bounds__(256, 2) void gdn_prep_kernel(GdnArgs a)
 // operands 52 KB, the Q~ and P rows 48 KB); with two parts a CU loads 76 KB.
 // Both forms give the same bits.
 template <int D, int PARTS>
-__global__ __launch_bounds__(256, 1) void gdn_chain_kernel(GdnArgs a)
+__global__ __launch_bounds__(512) void gdn_chain_kernel(GdnArgs a)
 {
     constexpr int J = 16;          // state rows (d_v indices) per workgroup
     constexpr int NSA = D / 32;    // phase A k-steps (d_k, 8 per lane group each)
-    constexpr int NBW = D / 64;    // phase B: 16-wide d_k blocks per wave
-    constexpr int NQ = NSA / PARTS, NP = 2 / PARTS;  // Q~ and P k-steps per wave
+    constexpr int NBW = D / 64;    // phase B: 16-wide d_k blocks per recurrence wave
+    constexpr int NQ = NSA / PARTS, NP = 2 / PARTS;  // Q~ and P k-steps per output wave
     static_assert(kC == 64 && D % 64 == 0, "four token tiles and four waves of d_k blocks");
     static_assert(PARTS == 1 || PARTS == 2, "one or two workgroups per slice");
     constexpr int MP = D + 8, DP = kC + 8;  // bf16 row strides (16-byte rows, staggered banks)
@@ -647,215 +647,262 @@ __global__ __launch_bounds__(256, 1) void gdn_chain_kernel(GdnArgs a)
     __shared__ __attribute__((aligned(16))) __bf16 Dh[J][DP], Dlo[J][DP];   // Delta^T of the chunk, rows j
     __shared__ f32x4 Ox[PARTS == 2 ? 4 : 1][64];                            // output halves (PARTS = 2)
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 15, g = lane >> 4;
+    const int tid = threadIdx.x, lane = tid & 63, wave8 = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, g = lane >> 4, wave = wave8 & 3;
     // workgroup b = (part * D/16 + slice) * n_v + h: consecutive workgroups
     // go to different XCDs, so the slices of one head (b mod 8 fixed when n_v
     // is a multiple of 8) share an L2 and read the head's chunk data once
     const uint32_t h = blockIdx.x % a.n_v, sl = blockIdx.x / a.n_v, jt = sl % (D / 16), j0 = jt * J;
     const int part = (int)(sl / (D / 16));
-    const int ot = PARTS == 1 ? wave : 2 * part + (wave & 1);  // the wave's output token tile
-    const int oh = PARTS == 1 ? 0 : wave >> 1;                 // and half (PARTS = 2)
-    const float* S = a.S + ((size_t)h * D + j0) * D;
-    float* So = a.S_out + ((size_t)h * D + j0) * D;
     const uint32_t nlast = a.n_chunks - 1;
-    const float scale = 1.0f / sqrtf((float)D);
 
-    // one chunk's register operands of this wave
-    struct Ops {
-        bf16x8 w[NSA];        // -W[16 wave + r][g D/4 + 8s .. +7] (bf16)
-        f32x4 u;              // U^T[j0 + r][16 wave + 4g .. +3]
-        bf16x8 q[NQ][2];      // Q~[16 ot + r][g D/4 + 8s .. +7] of its k-steps, hi and lo
-        bf16x8 k[NBW][2][2];  // K~[16g + 8s .. +7][16 (NBW wave + bb) + r], hi and lo
-        bf16x8 p[NP][2];      // P[16 ot + r][16g + 8s .. +7] of its k-steps, hi and lo
-        float gl;
-    };
-    // the loads of one register set in two halves (-W, U and Q~; K~, P and
-    // gamma_last)
-    auto load_a = [&](Ops& o, uint32_t c) {
-        ChunkWs<D> w(a.ws, h, c, a.n_chunks);
-        const bf16x8* wb = reinterpret_cast<const bf16x8*>(w.Wb);
-#pragma unroll
-        for (int sk = 0; sk < NSA; ++sk) o.w[sk] = wb[(size_t)(wave * NSA + sk) * 64 + lane];
-        o.u = *reinterpret_cast<const f32x4*>(w.U + (size_t)(j0 + r) * kC + 16 * wave + 4 * g);
-        const bf16x8* qb = reinterpret_cast<const bf16x8*>(w.Q);
-#pragma unroll
-        for (int i = 0; i < NQ; ++i)
-#pragma unroll
-            for (int hl = 0; hl < 2; ++hl) o.q[i][hl] = qb[((size_t)(ot * NSA + oh * NQ + i) * 2 + hl) * 64 + lane];
-    };
-    auto load_b = [&](Ops& o, uint32_t c) {
-        ChunkWs<D> w(a.ws, h, c, a.n_chunks);
-        const bf16x8* kb = reinterpret_cast<const bf16x8*>(w.Kb);
-#pragma unroll
-        for (int bb = 0; bb < NBW; ++bb)
-#pragma unroll
-            for (int sk = 0; sk < 2; ++sk)
-#pragma unroll
-                for (int hl = 0; hl < 2; ++hl)
-                    o.k[bb][sk][hl] = kb[((size_t)((NBW * wave + bb) * 2 + sk) * 2 + hl) * 64 + lane];
-        const bf16x8* pb = reinterpret_cast<const bf16x8*>(w.P);
-#pragma unroll
-        for (int i = 0; i < NP; ++i)
-#pragma unroll
-            for (int hl = 0; hl < 2; ++hl) o.p[i][hl] = pb[((size_t)(ot * 2 + oh * NP + i) * 2 + hl) * 64 + lane];
-        o.gl = w.gl[0];
-    };
-    auto load = [&](Ops& o, uint32_t c) {
-        load_a(o, c);
-        load_b(o, c);
-    };
-    // the state tiles of this wave in fp32: mt[bb][e] = M[j0 + 4g + e][16 (NBW wave + bb) + r]
-    f32x4 mt[NBW];
-    auto put_state = [&] {
-#pragma unroll
-        for (int bb = 0; bb < NBW; ++bb)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int i = 16 * (NBW * wave + bb) + r;
-                const __bf16 hi = (__bf16)mt[bb][e];
-                Mh[4 * g + e][i] = hi;
-                Mlo[4 * g + e][i] = (__bf16)(mt[bb][e] - (float)hi);
-            }
-    };
-    // output rows 16 ot + 4g + i of chunk c, column j0 + r, for i in [i0, i0
-    // + n); with PARTS = 2 the half of a previous chunk in LDS is added first
-    // (its partner wave stored it before the last barrier).  Lanes with
-    // nothing to write (chunk c < 0, or a token past the last) store to the
-    // chunk's padding word, so every chunk runs the same memory instructions.
-    auto put_out = [&](int64_t c, f32x4 o) {
-        if (PARTS == 2) o = o + Ox[(wave & 1) * 2 + (oh ^ 1)][lane];
-        const uint32_t cc = c < 0 ? 0u : (uint32_t)c;
-        float* pad = ChunkWs<D>(a.ws, h, cc, a.n_chunks).gl + 1;
-#pragma unroll
-        for (int i = 0; i < 4 / PARTS; ++i) {
-            const int ii = PARTS == 1 ? i : 2 * oh + i;
-            const uint32_t t = cc * kC + 16 * ot + 4 * g + ii;
-            float* dst = c >= 0 && t < a.T ? a.out + (size_t)t * a.out_stride + (size_t)h * D + j0 + r : pad;
-            *dst = o[ii] * scale;
+    // Every chunk is two phases, each ended by a barrier of all eight waves; `walk` runs a role's two phases for
+    // every chunk with the operand sets rotating: chunk c's were loaded two chunks before.  Whole rounds of three
+    // chunks in a loop without exits in between, the rest after it: with an exit test after every chunk the
+    // compiler's waits for the register sets at the loop head covered every load in flight (vmcnt(1)), once per
+    // round.
+    auto walk = [&](auto& chunk, auto& oa, auto& ob, auto& oc) {
+        const uint32_t rounds = a.n_chunks / 3;
+        uint32_t c = 0;
+        for (uint32_t rd = 0; rd < rounds; ++rd, c += 3) {
+            chunk(c, oa, oc, min(c + 2, nlast));
+            chunk(c + 1, ob, oa, min(c + 3, nlast));
+            chunk(c + 2, oc, ob, min(c + 4, nlast));
+        }
+        if (c <= nlast) {
+            chunk(c, oa, oc, min(c + 2, nlast));
+            if (c + 1 <= nlast) chunk(c + 1, ob, oa, min(c + 3, nlast));
         }
     };
-#pragma unroll
-    for (int bb = 0; bb < NBW; ++bb)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) mt[bb][e] = S[(size_t)(4 * g + e) * D + 16 * (NBW * wave + bb) + r];
-    put_state();
-    Ops oa, ob, oc;  // chunks c, c+1, c+2 of a round of three
-    load(oa, 0);
-    load(ob, min(1u, nlast));
-    __syncthreads();
-    f32x4 oprev = f32x4{0.f, 0.f, 0.f, 0.f};  // PARTS = 2: this wave's half of the previous chunk
 
-    // One chunk with operand set o; the loads of the set for chunk cf go out
-    // in between the MFMAs (the -W / Q~ half in phase A, the K~ / P half in
-    // phase B): a wave that issued its loads in one burst waited for the
-    // CU's memory pipeline instead of issuing MFMAs.
-    auto chunk = [&](uint32_t c, const Ops& o, Ops& of, uint32_t cf) {
-        // phase A: Delta rows 16 wave + 4g + e, column j0 + r = U - W M^T;
-        // then the Q~ M^T part of the output halves
-        f32x4 o0 = f32x4{0.f, 0.f, 0.f, 0.f}, o1 = o0;
-        {
-            f32x4 acc = o.u;
-            bf16x8 bh[NSA], bl[NSA];
+    if (wave8 < 4) {
+        // ---- the recurrence ----
+        typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+        const float* S = a.S + ((size_t)h * D + j0) * D;
+        float* So = a.S_out + ((size_t)h * D + j0) * D;
+        // one chunk's register operands of this wave
+        struct Ops {
+            bf16x8 w[NSA];        // -W[16 wave + r][g D/4 + 8s .. +7] (bf16)
+            f32x4 u;              // U^T[j0 + r][16 wave + 4g .. +3]
+            bf16x8 k[NBW][2][2];  // K~[16g + 8s .. +7][16 (NBW wave + bb) + r], hi and lo
+            float gl;
+        };
+        // the loads of one register set in two halves (-W and U; K~ and gamma_last)
+        auto load_a = [&](Ops& o, uint32_t c) {
+            ChunkWs<D> w(a.ws, h, c, a.n_chunks);
+            const bf16x8* wb = reinterpret_cast<const bf16x8*>(w.Wb);
 #pragma unroll
-            for (int sk = 0; sk < NSA; ++sk) {
-                bh[sk] = *reinterpret_cast<const bf16x8*>(&Mh[r][g * (D / 4) + 8 * sk]);
-                bl[sk] = *reinterpret_cast<const bf16x8*>(&Mlo[r][g * (D / 4) + 8 * sk]);
+            for (int sk = 0; sk < NSA; ++sk) o.w[sk] = wb[(size_t)(wave * NSA + sk) * 64 + lane];
+            o.u = *reinterpret_cast<const f32x4*>(w.U + (size_t)(j0 + r) * kC + 16 * wave + 4 * g);
+        };
+        auto load_b = [&](Ops& o, uint32_t c) {
+            ChunkWs<D> w(a.ws, h, c, a.n_chunks);
+            const bf16x8* kb = reinterpret_cast<const bf16x8*>(w.Kb);
+#pragma unroll
+            for (int bb = 0; bb < NBW; ++bb)
+#pragma unroll
+                for (int sk = 0; sk < 2; ++sk)
+#pragma unroll
+                    for (int hl = 0; hl < 2; ++hl)
+                        o.k[bb][sk][hl] = kb[((size_t)((NBW * wave + bb) * 2 + sk) * 2 + hl) * 64 + lane];
+            o.gl = w.gl[0];
+        };
+        // the state tiles of this wave in fp32: mt[bb][e] = M[j0 + r][16 (NBW wave + bb) + 4g + e].  The products of
+        // phase B are taken transposed (K~^T Delta) for it: the four d_k a lane holds are one 8-byte store of a row
+        // of Mh and Mlo, where rows along e were four 2-byte stores each.
+        f32x4 mt[NBW];
+        auto put_state = [&] {
+#pragma unroll
+            for (int bb = 0; bb < NBW; ++bb) {
+                bf16x4 mh, ml;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    mh[e] = (__bf16)mt[bb][e];
+                    ml[e] = (__bf16)(mt[bb][e] - (float)mh[e]);
+                }
+                *reinterpret_cast<bf16x4*>(&Mh[r][16 * (NBW * wave + bb) + 4 * g]) = mh;
+                *reinterpret_cast<bf16x4*>(&Mlo[r][16 * (NBW * wave + bb) + 4 * g]) = ml;
             }
-            if (PARTS == 2) put_out((int64_t)c - 1, oprev);
-            load_a(of, cf);
+        };
 #pragma unroll
-            for (int sk = 0; sk < NSA; ++sk) {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.w[sk], bl[sk], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.w[sk], bh[sk], acc, 0, 0, 0);
+        for (int bb = 0; bb < NBW; ++bb)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mt[bb][e] = S[(size_t)r * D + 16 * (NBW * wave + bb) + 4 * g + e];
+        put_state();
+        Ops oa, ob, oc;  // chunks c, c+1, c+2 of a round of three
+        load_a(oa, 0);
+        load_b(oa, 0);
+        load_a(ob, min(1u, nlast));
+        load_b(ob, min(1u, nlast));
+        __syncthreads();
+
+        // One chunk with operand set o; the loads of the set for chunk cf go out
+        // in between the MFMAs (-W and U in phase A, K~ in phase B): a wave that
+        // issued its loads in one burst waited for the CU's memory pipeline
+        // instead of issuing MFMAs.
+        auto chunk = [&](uint32_t, const Ops& o, Ops& of, uint32_t cf) {
+            // phase A: Delta rows 16 wave + 4g + e, column j0 + r = U - W M^T
+            {
+                f32x4 acc = o.u;
+                bf16x8 bh[NSA], bl[NSA];
+#pragma unroll
+                for (int sk = 0; sk < NSA; ++sk) {
+                    bh[sk] = *reinterpret_cast<const bf16x8*>(&Mh[r][g * (D / 4) + 8 * sk]);
+                    bl[sk] = *reinterpret_cast<const bf16x8*>(&Mlo[r][g * (D / 4) + 8 * sk]);
+                }
+                load_a(of, cf);
+#pragma unroll
+                for (int sk = 0; sk < NSA; ++sk) {
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.w[sk], bl[sk], acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.w[sk], bh[sk], acc, 0, 0, 0);
+                }
+                // all reads of LDS first: one read in front of each MFMA put its latency on the chain 2 NSA times
+                __builtin_amdgcn_sched_group_barrier(0x100, 2 * NSA, 0);
+#pragma unroll
+                for (int k = 0; k < 2 * NSA; ++k) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
+                    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // one global load
+                }
+                bf16x4 dh, dl;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    dh[e] = (__bf16)acc[e];
+                    dl[e] = (__bf16)(acc[e] - (float)dh[e]);
+                }
+                *reinterpret_cast<bf16x4*>(&Dh[r][16 * wave + 4 * g]) = dh;
+                *reinterpret_cast<bf16x4*>(&Dlo[r][16 * wave + 4 * g]) = dl;
             }
+            lds_barrier();
+            // phase B: M <- gamma_last M + Delta^T K~ on this wave's d_k blocks
+            bf16x8 ah[2], al[2];
 #pragma unroll
-            for (int k = 0; k < 2 * NSA; ++k) {
+            for (int sk = 0; sk < 2; ++sk) {
+                ah[sk] = *reinterpret_cast<const bf16x8*>(&Dh[r][16 * g + 8 * sk]);
+                al[sk] = *reinterpret_cast<const bf16x8*>(&Dlo[r][16 * g + 8 * sk]);
+            }
+            load_b(of, cf);
+#pragma unroll
+            for (int bb = 0; bb < NBW; ++bb) mt[bb] *= o.gl;
+#pragma unroll
+            for (int sk = 0; sk < 2; ++sk) {  // hi lo', lo hi', hi hi' as in mfma_x3, the blocks' chains side by side
+#pragma unroll
+                for (int bb = 0; bb < NBW; ++bb)
+                    mt[bb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.k[bb][sk][0], al[sk], mt[bb], 0, 0, 0);
+#pragma unroll
+                for (int bb = 0; bb < NBW; ++bb)
+                    mt[bb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.k[bb][sk][1], ah[sk], mt[bb], 0, 0, 0);
+#pragma unroll
+                for (int bb = 0; bb < NBW; ++bb)
+                    mt[bb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.k[bb][sk][0], ah[sk], mt[bb], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+            for (int k = 0; k < 6 * NBW; ++k) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
                 __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // one global load
             }
-            typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-            bf16x4 dh, dl;
+            put_state();
+            lds_barrier();
+        };
+        walk(chunk, oa, ob, oc);
+        if (part == 0) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                dh[e] = (__bf16)acc[e];
-                dl[e] = (__bf16)(acc[e] - (float)dh[e]);
+            for (int bb = 0; bb < NBW; ++bb)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) So[(size_t)r * D + 16 * (NBW * wave + bb) + 4 * g + e] = mt[bb][e];
+        }
+    } else {
+        // ---- the outputs ----
+        const int ot = PARTS == 1 ? wave : 2 * part + (wave & 1);  // the wave's token tile
+        const int oh = PARTS == 1 ? 0 : wave >> 1;                 // and half (PARTS = 2)
+        const float scale = 1.0f / sqrtf((float)D);
+        struct Ops {
+            bf16x8 q[NQ][2];  // Q~[16 ot + r][g D/4 + 8s .. +7] of its k-steps, hi and lo
+            bf16x8 p[NP][2];  // P[16 ot + r][16g + 8s .. +7] of its k-steps, hi and lo
+        };
+        auto load_q = [&](Ops& o, uint32_t c) {
+            const bf16x8* qb = reinterpret_cast<const bf16x8*>(ChunkWs<D>(a.ws, h, c, a.n_chunks).Q);
+#pragma unroll
+            for (int i = 0; i < NQ; ++i)
+#pragma unroll
+                for (int hl = 0; hl < 2; ++hl) o.q[i][hl] = qb[((size_t)(ot * NSA + oh * NQ + i) * 2 + hl) * 64 + lane];
+        };
+        auto load_p = [&](Ops& o, uint32_t c) {
+            const bf16x8* pb = reinterpret_cast<const bf16x8*>(ChunkWs<D>(a.ws, h, c, a.n_chunks).P);
+#pragma unroll
+            for (int i = 0; i < NP; ++i)
+#pragma unroll
+                for (int hl = 0; hl < 2; ++hl) o.p[i][hl] = pb[((size_t)(ot * 2 + oh * NP + i) * 2 + hl) * 64 + lane];
+        };
+        // output rows 16 ot + 4g + i of chunk c, column j0 + r; with PARTS = 2 the half of a previous chunk in LDS is
+        // added first (its partner wave stored it before the last barrier) and this wave writes half of the rows.
+        // Lanes with nothing to write (chunk c < 0, or a token past the last) store to the chunk's padding word, so
+        // every chunk runs the same memory instructions.
+        auto put_out = [&](int64_t c, f32x4 o) {
+            if (PARTS == 2) o = o + Ox[(wave & 1) * 2 + (oh ^ 1)][lane];
+            const uint32_t cc = c < 0 ? 0u : (uint32_t)c;
+            float* pad = ChunkWs<D>(a.ws, h, cc, a.n_chunks).gl + 1;
+#pragma unroll
+            for (int i = 0; i < 4 / PARTS; ++i) {
+                const int ii = PARTS == 1 ? i : 2 * oh + i;
+                const uint32_t t = cc * kC + 16 * ot + 4 * g + ii;
+                float* dst = c >= 0 && t < a.T ? a.out + (size_t)t * a.out_stride + (size_t)h * D + j0 + r : pad;
+                *dst = o[ii] * scale;
             }
-            *reinterpret_cast<bf16x4*>(&Dh[r][16 * wave + 4 * g]) = dh;
-            *reinterpret_cast<bf16x4*>(&Dlo[r][16 * wave + 4 * g]) = dl;
-            if (PARTS == 1) {
-#pragma unroll
-                for (int i = 0; i < NSA / 2; ++i) o0 = mfma_x3(o.q[i][0], o.q[i][1], bh[i], bl[i], o0);
-#pragma unroll
-                for (int i = NSA / 2; i < NSA; ++i) o1 = mfma_x3(o.q[i][0], o.q[i][1], bh[i], bl[i], o1);
-            } else if (oh == 0) {  // uniform over the wave; the B operands are k-steps oh NQ ..
-#pragma unroll
-                for (int i = 0; i < NQ; ++i) o0 = mfma_x3(o.q[i][0], o.q[i][1], bh[i], bl[i], o0);
-            } else {
-#pragma unroll
-                for (int i = 0; i < NQ; ++i) o0 = mfma_x3(o.q[i][0], o.q[i][1], bh[NQ + i], bl[NQ + i], o0);
-            }
-        }
-        lds_barrier();
-        // phase B: M <- gamma_last M + Delta^T K~ on this wave's d_k blocks;
-        // then the P Delta part of the output halves
-        bf16x8 ah[2], al[2];
-#pragma unroll
-        for (int sk = 0; sk < 2; ++sk) {
-            ah[sk] = *reinterpret_cast<const bf16x8*>(&Dh[r][16 * g + 8 * sk]);
-            al[sk] = *reinterpret_cast<const bf16x8*>(&Dlo[r][16 * g + 8 * sk]);
-        }
-        load_b(of, cf);
-#pragma unroll
-        for (int bb = 0; bb < NBW; ++bb) {
-            f32x4 acc = mt[bb] * o.gl;
-#pragma unroll
-            for (int sk = 0; sk < 2; ++sk) acc = mfma_x3(ah[sk], al[sk], o.k[bb][sk][0], o.k[bb][sk][1], acc);
-            mt[bb] = acc;
-        }
-#pragma unroll
-        for (int k = 0; k < 6 * NBW; ++k) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-            __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);  // one global load
-        }
-        put_state();
-        if (PARTS == 1) {
-            o0 = mfma_x3(o.p[0][0], o.p[0][1], ah[0], al[0], o0);
-            o1 = mfma_x3(o.p[1][0], o.p[1][1], ah[1], al[1], o1);
-            put_out(c, o0 + o1);
-        } else {
-            if (oh == 0)
-                o0 = mfma_x3(o.p[0][0], o.p[0][1], ah[0], al[0], o0);
-            else
-                o0 = mfma_x3(o.p[0][0], o.p[0][1], ah[1], al[1], o0);
-            Ox[(wave & 1) * 2 + oh][lane] = o0;  // the partner adds it after the barrier
-            oprev = o0;
-        }
-        lds_barrier();
-    };
-    // chunk c's operands are in a register set loaded two chunks before.
-    // Whole rounds of three chunks in a loop without exits in between, the
-    // rest after it: with an exit test after every chunk the compiler's
-    // waits for the register sets at the loop head covered every load in
-    // flight (vmcnt(1)), once per round.
-    const uint32_t rounds = a.n_chunks / 3;
-    uint32_t c = 0;
-    for (uint32_t rd = 0; rd < rounds; ++rd, c += 3) {
-        chunk(c, oa, oc, min(c + 2, nlast));
-        chunk(c + 1, ob, oa, min(c + 3, nlast));
-        chunk(c + 2, oc, ob, min(c + 4, nlast));
-    }
-    if (c <= nlast) {
-        chunk(c, oa, oc, min(c + 2, nlast));
-        if (c + 1 <= nlast) chunk(c + 1, ob, oa, min(c + 3, nlast));
-    }
-    if (PARTS == 2) put_out(nlast, oprev);
+        };
+        Ops oa, ob, oc;
+        load_q(oa, 0);
+        load_p(oa, 0);
+        load_q(ob, min(1u, nlast));
+        load_p(ob, min(1u, nlast));
+        __syncthreads();
+        f32x4 oprev = f32x4{0.f, 0.f, 0.f, 0.f};  // PARTS = 2: this wave's half of the previous chunk
 
-    if (part == 0) {
+        auto chunk = [&](uint32_t c, const Ops& o, Ops& of, uint32_t cf) {
+            // phase A: the Q~ M^T part of the output halves
+            f32x4 o0 = f32x4{0.f, 0.f, 0.f, 0.f}, o1 = o0;
+            {
+                bf16x8 bh[NQ], bl[NQ];
+                const int s0 = PARTS == 1 ? 0 : oh * NQ;
 #pragma unroll
-        for (int bb = 0; bb < NBW; ++bb)
+                for (int i = 0; i < NQ; ++i) {
+                    bh[i] = *reinterpret_cast<const bf16x8*>(&Mh[r][g * (D / 4) + 8 * (s0 + i)]);
+                    bl[i] = *reinterpret_cast<const bf16x8*>(&Mlo[r][g * (D / 4) + 8 * (s0 + i)]);
+                }
+                if (PARTS == 2) put_out((int64_t)c - 1, oprev);
+                load_q(of, cf);
+                if (PARTS == 1) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) So[(size_t)(4 * g + e) * D + 16 * (NBW * wave + bb) + r] = mt[bb][e];
+                    for (int i = 0; i < NSA / 2; ++i) o0 = mfma_x3(o.q[i][0], o.q[i][1], bh[i], bl[i], o0);
+#pragma unroll
+                    for (int i = NSA / 2; i < NQ; ++i) o1 = mfma_x3(o.q[i][0], o.q[i][1], bh[i], bl[i], o1);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < NQ; ++i) o0 = mfma_x3(o.q[i][0], o.q[i][1], bh[i], bl[i], o0);
+                }
+            }
+            lds_barrier();
+            // phase B: the P Delta part
+            bf16x8 ah[NP], al[NP];
+            const int s0 = PARTS == 1 ? 0 : oh;
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+                ah[i] = *reinterpret_cast<const bf16x8*>(&Dh[r][16 * g + 8 * (s0 + i)]);
+                al[i] = *reinterpret_cast<const bf16x8*>(&Dlo[r][16 * g + 8 * (s0 + i)]);
+            }
+            load_p(of, cf);
+            o0 = mfma_x3(o.p[0][0], o.p[0][1], ah[0], al[0], o0);
+            if (PARTS == 1) {
+                o1 = mfma_x3(o.p[NP - 1][0], o.p[NP - 1][1], ah[NP - 1], al[NP - 1], o1);
+                put_out(c, o0 + o1);
+            } else {
+                Ox[(wave & 1) * 2 + oh][lane] = o0;  // the partner adds it after the barrier
+                oprev = o0;
+            }
+            lds_barrier();
+        };
+        walk(chunk, oa, ob, oc);
+        if (PARTS == 2) put_out(nlast, oprev);
     }
 }
 
@@ -955,9 +1002,9 @@ hipError_t launch_gdn_d(const GdnArgs& a, hipStream_t st)
         // before the other part has read it)
         const uint32_t slices = a.n_v * (D / 16);
         if (a.S_out != a.S && 2 * slices <= (uint32_t)n_cus())
-            hipLaunchKernelGGL((gdn_chain_kernel<D, 2>), dim3(2 * slices), dim3(256), 0, st, a);
+            hipLaunchKernelGGL((gdn_chain_kernel<D, 2>), dim3(2 * slices), dim3(512), 0, st, a);
         else
-            hipLaunchKernelGGL((gdn_chain_kernel<D, 1>), dim3(slices), dim3(256), 0, st, a);
+            hipLaunchKernelGGL((gdn_chain_kernel<D, 1>), dim3(slices), dim3(512), 0, st, a);
     } else {
         hipLaunchKernelGGL(gdn_kernel<D>, dim3(a.n_v * (D / kCols)), dim3(256), 0, st, a);
     }
