@@ -287,11 +287,17 @@ struct ChunkWs {
     }
 };
 
+// Eight waves, two workgroups per CU.  What bounds a chunk is the fp32 MFMA: 20 Gram tile products and the
+// substitution's 16 column tiles are 10240 cycles of each SIMD, 4.3 us; at 4096 tokens the 230 MB read and
+// written are the other half.  So waves 0-3 take the Gram products, five each, while waves 4-7 convert and write
+// Q~ and K~, and v is loaded with q and k for the substitution far below.  The barriers wait for LDS alone:
+// nothing written to memory is read here, and __syncthreads() waited for those writes and for v.
 template <int D>
-__global__ __launch_bounds__(256, 2) void gdn_prep_kernel(GdnArgs a)
+__global__ __launch_bounds__(512, 4) void gdn_prep_kernel(GdnArgs a)
 {
     constexpr int KP = D + 4;  // LDS row stride of the q / k rows (16-byte rows, staggered banks)
     constexpr int AP = kC + 4;
+    constexpr int NTH = 512;
     constexpr int KQ = D / 4;  // contraction indices per lane group in the Gram MFMAs
     // A and P share their LDS with the q rows: once Q~ is written out and
     // each wave holds its Gram rows of Q in registers, Qn is dead.  84 -> 68
@@ -304,7 +310,7 @@ __global__ __launch_bounds__(256, 2) void gdn_prep_kernel(GdnArgs a)
     float(*Am)[AP] = reinterpret_cast<float(*)[AP]>(QA);
     float(*Pm)[kC] = reinterpret_cast<float(*)[kC]>(QA + kC * AP);
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
     const uint32_t c = blockIdx.x, h = blockIdx.y, kh = h % a.n_k;
     const uint32_t t0 = c * kC;
@@ -318,19 +324,35 @@ __global__ __launch_bounds__(256, 2) void gdn_prep_kernel(GdnArgs a)
     const size_t gi = (size_t)(t0 + min(lane, nt - 1)) * a.n_v + h;
     const float g_raw = a.gate[gi], b_raw = a.beta[gi];
 
+    // Wave w owns the 16-column tiles w and, at D = 128, w + 8 of the substitution's right-hand sides: tiles
+    // below D / 16 are columns of V, the rest of K.
+    constexpr int CTW = 2 * D / 16 / 8;
+    static_assert(CTW == 1 || CTW == 2, "head_dim 64 or 128");
+    const bool v_wave = CTW == 2 || wave < 4;  // the wave's first tile is one of V
+
     // q and k rows of the chunk (zero past the last token): all loads issued
     // before any LDS store; the l2 norms are taken in registers (a row's D/4
     // float4s sit in D/4 consecutive lanes)
+    f32x4 X[CTW][4];
     {
-        constexpr int NE = kC * D / 4 / 256;
+        constexpr int NE = kC * D / 4 / NTH;
         constexpr int RL = D / 4;
         f32x4 kv[NE], qv[NE];
 #pragma unroll
         for (int u = 0; u < NE; ++u) {
-            const int e = tid + 256 * u, t = e / (D / 4), i = (e % (D / 4)) * 4;
+            const int e = tid + NTH * u, t = e / (D / 4), i = (e % (D / 4)) * 4;
             const size_t off = (size_t)(t0 + min(t, nt - 1)) * a.qk_stride + (size_t)kh * D + i;
             kv[u] = *reinterpret_cast<const f32x4*>(a.k + off);
             qv[u] = *reinterpret_cast<const f32x4*>(a.q + off);
+        }
+        // the V columns (rows past the last token are clamped: their beta is 0)
+        if (v_wave) {
+            const float* vp = a.v + (size_t)h * D + 16 * wave + r;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    X[0][i][e] = vp[(size_t)(t0 + min(16 * i + 4 * g + e, nt - 1)) * a.v_stride];
         }
         if (a.eps > 0.0f) {
 #pragma unroll
@@ -349,7 +371,7 @@ __global__ __launch_bounds__(256, 2) void gdn_prep_kernel(GdnArgs a)
         }
 #pragma unroll
         for (int u = 0; u < NE; ++u) {
-            const int e = tid + 256 * u, t = e / (D / 4), i = (e % (D / 4)) * 4;
+            const int e = tid + NTH * u, t = e / (D / 4), i = (e % (D / 4)) * 4;
             const float keep = t < nt ? 1.0f : 0.0f;
             *reinterpret_cast<f32x4*>(&Kn[t][i]) = kv[u] * keep;
             *reinterpret_cast<f32x4*>(&Qn[t][i]) = qv[u] * keep;
@@ -371,113 +393,131 @@ __global__ __launch_bounds__(256, 2) void gdn_prep_kernel(GdnArgs a)
         see[lane] = expf(glast - gv);
         if (lane == 0) w.gl[0] = expf(glast);
     }
-    __syncthreads();
-
-    // Q~ = diag(gamma) Q and K~ = diag(e) K as bf16 hi / lo in the chain
-    // kernel's register order (ChunkWs)
-    for (int e = tid; e < 4 * (D / 32) * 64; e += 256) {
-        const int l = e % 64, ws_ = e / 64, sk = ws_ % (D / 32), wt = ws_ / (D / 32);
-        const int t = 16 * wt + (l & 15), i = (l >> 4) * (D / 4) + 8 * sk;
-        const f32x4 x0 = *reinterpret_cast<const f32x4*>(&Qn[t][i]);
-        const f32x4 x1 = *reinterpret_cast<const f32x4*>(&Qn[t][i + 4]);
-        float x[8];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {  // rounded products (not contracted into the split)
-            x[u] = __fmul_rn(x0[u], sgam[t]);
-            x[u + 4] = __fmul_rn(x1[u], sgam[t]);
-        }
-        bf16x8 hi, lo;
-        split_bf16(x, hi, lo);
-        bf16x8* dst = reinterpret_cast<bf16x8*>(w.Q) + (size_t)ws_ * 128 + l;
-        dst[0] = hi;
-        dst[64] = lo;
-    }
-    for (int e = tid; e < (D / 16) * 2 * 64; e += 256) {
-        const int l = e % 64, bs = e / 64, sk = bs % 2, b = bs / 2;
-        const int tk = 16 * (l >> 4) + 8 * sk, ik = 16 * b + (l & 15);
-        float x[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = Kn[tk + u][ik] * see[tk + u];
-        bf16x8 hi, lo;
-        split_bf16(x, hi, lo);
-        bf16x8* dst = reinterpret_cast<bf16x8*>(w.Kb) + (size_t)bs * 128 + l;
-        dst[0] = hi;
-        dst[64] = lo;
-    }
+    lds_barrier();
 
     // Gram matrices K K^T and Q K^T over the ten 16x16 tiles (tb, sb) with
-    // sb <= tb (A needs s < t, P needs s <= t; P is zero above); wave w takes
-    // tiles w, w+4, w+8.  Lane group g contracts over d_k indices g*KQ ..
-    // g*KQ+KQ-1.  The sums stay in registers until every read of Qn is done,
-    // then A overwrites Qn.
-    {
-        static_assert(kC == 64, "four 16-token blocks per chunk");
-        constexpr int NTL = 10, TPW = 3;
-        f32x4 gkk[TPW], gqk[TPW];
+    // sb <= tb (A needs s < t, P needs s <= t; P is zero above): wave w < 4
+    // takes both products of tiles w and w + 4, and one of the last two
+    // tiles'.  Lane group g contracts over d_k indices g*KQ .. g*KQ+KQ-1.  The
+    // results stay in registers until every read of Qn is done, then A and P
+    // overwrite it.
+    static_assert(kC == 64, "four 16-token blocks per chunk");
+    f32x4 av[3], pv[3];
+    const int t8 = 8 + (wave >> 1 & 1);  // the third tile (3, 2) or (3, 3): K K^T of an even wave, Q K^T of an odd one
+    auto tile_of = [&](int j, int& tb, int& sbk) {
+        const int ti = j < 2 ? (wave & 3) + 4 * j : t8;
+        tb = ti >= 6 ? 3 : ti >= 3 ? 2 : ti >= 1 ? 1 : 0;
+        sbk = ti - tb * (tb + 1) / 2;
+    };
+    if (wave < 4) {
+        auto row = [&](const float (*m)[KP], int b, int kb) {
+            return *reinterpret_cast<const f32x4*>(&m[16 * b + r][g * KQ + kb]);
+        };
 #pragma unroll
-        for (int j = 0; j < TPW; ++j) {
-            const int ti = wave + 4 * j;
-            gkk[j] = gqk[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            if (ti < NTL) {  // uniform over the wave
-                const int tb = ti >= 6 ? 3 : ti >= 3 ? 2 : ti >= 1 ? 1 : 0, sbk = ti - tb * (tb + 1) / 2;
-                f32x4 skk[2], sqk[2];
-#pragma unroll
-                for (int e = 0; e < 2; ++e) skk[e] = sqk[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < 3; ++j) {
+            int tb, sbk;
+            tile_of(j, tb, sbk);
+            f32x4 skk[2] = {}, sqk[2] = {};
+            if (j < 2) {
 #pragma unroll
                 for (int kb = 0; kb < KQ; kb += 4) {
-                    const f32x4 x = *reinterpret_cast<const f32x4*>(&Kn[16 * tb + r][g * KQ + kb]);
-                    const f32x4 y = *reinterpret_cast<const f32x4*>(&Qn[16 * tb + r][g * KQ + kb]);
-                    const f32x4 b = *reinterpret_cast<const f32x4*>(&Kn[16 * sbk + r][g * KQ + kb]);
+                    const f32x4 x = row(Kn, tb, kb), y = row(Qn, tb, kb), b = row(Kn, sbk, kb);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         skk[e & 1] = mfma_f32(x[e], b[e], skk[e & 1]);
                         sqk[e & 1] = mfma_f32(y[e], b[e], sqk[e & 1]);
                     }
                 }
-                gkk[j] = skk[0] + skk[1];
-                gqk[j] = sqk[0] + sqk[1];
-            }
-        }
-        __syncthreads();  // every read of Qn is done: A may overwrite it
+            } else {
+                const float(*m)[KP] = wave & 1 ? Qn : Kn;
 #pragma unroll
-        for (int j = 0; j < TPW; ++j) {
-            const int ti = wave + 4 * j;
-            if (ti < NTL) {
-                const int tb = ti >= 6 ? 3 : ti >= 3 ? 2 : ti >= 1 ? 1 : 0, sbk = ti - tb * (tb + 1) / 2;
-                const int s = 16 * sbk + r;
+                for (int kb = 0; kb < KQ; kb += 4) {
+                    const f32x4 x = row(m, tb, kb), b = row(Kn, sbk, kb);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int t = 16 * tb + 4 * g + i;
-                    const float dec = s <= t ? expf(sg[t] - sg[s]) : 0.0f;
-                    Am[t][s] = s < t ? sb[t] * dec * gkk[j][i] : 0.0f;
-                    Pm[t][s] = dec * gqk[j][i];
+                    for (int e = 0; e < 4; ++e) skk[e & 1] = mfma_f32(x[e], b[e], skk[e & 1]);
                 }
+                sqk[0] = skk[0];
+                sqk[1] = skk[1];
+            }
+            const f32x4 gkk = skk[0] + skk[1], gqk = sqk[0] + sqk[1];
+            const int s = 16 * sbk + r;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int t = 16 * tb + 4 * g + i;
+                const float dec = s <= t ? expf(sg[t] - sg[s]) : 0.0f;
+                av[j][i] = s < t ? sb[t] * dec * gkk[i] : 0.0f;
+                pv[j][i] = dec * gqk[i];
             }
         }
-        // P above the diagonal blocks: row block `wave`, column blocks wave+1 ..
-        for (int cb = wave + 1; cb < kC / 16; ++cb)
+    } else {
+        // Q~ = diag(gamma) Q and K~ = diag(e) K as bf16 hi / lo in the chain kernel's register order (ChunkWs)
+        for (int e = tid - 256; e < 4 * (D / 32) * 64; e += 256) {
+            const int l = e % 64, ws_ = e / 64, sk = ws_ % (D / 32), wt = ws_ / (D / 32);
+            const int t = 16 * wt + (l & 15), i = (l >> 4) * (D / 4) + 8 * sk;
+            const f32x4 x0 = *reinterpret_cast<const f32x4*>(&Qn[t][i]);
+            const f32x4 x1 = *reinterpret_cast<const f32x4*>(&Qn[t][i + 4]);
+            float x[8];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) Pm[16 * wave + 4 * g + i][16 * cb + r] = 0.0f;
+            for (int u = 0; u < 4; ++u) {  // rounded products (not contracted into the split)
+                x[u] = __fmul_rn(x0[u], sgam[t]);
+                x[u + 4] = __fmul_rn(x1[u], sgam[t]);
+            }
+            bf16x8 hi, lo;
+            split_bf16(x, hi, lo);
+            bf16x8* dst = reinterpret_cast<bf16x8*>(w.Q) + (size_t)ws_ * 128 + l;
+            dst[0] = hi;
+            dst[64] = lo;
+        }
+        for (int e = tid - 256; e < (D / 16) * 2 * 64; e += 256) {
+            const int l = e % 64, bs = e / 64, sk = bs % 2, b = bs / 2;
+            const int tk = 16 * (l >> 4) + 8 * sk, ik = 16 * b + (l & 15);
+            float x[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) x[u] = Kn[tk + u][ik] * see[tk + u];
+            bf16x8 hi, lo;
+            split_bf16(x, hi, lo);
+            bf16x8* dst = reinterpret_cast<bf16x8*>(w.Kb) + (size_t)bs * 128 + l;
+            dst[0] = hi;
+            dst[64] = lo;
+        }
     }
-    __syncthreads();
+    lds_barrier();  // every read of Qn is done: A and P may overwrite it
+    if (wave < 4) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            int tb, sbk;
+            tile_of(j, tb, sbk);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int t = 16 * tb + 4 * g + i, s = 16 * sbk + r;
+                if (j < 2 || !(wave & 1)) Am[t][s] = av[j][i];
+                if (j < 2 || wave & 1) Pm[t][s] = pv[j][i];
+            }
+        }
+    } else {
+        // P above the diagonal blocks: row block wave - 4, column blocks from wave - 3 on
+        for (int cb = wave - 3; cb < kC / 16; ++cb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) Pm[16 * (wave - 4) + 4 * g + i][16 * cb + r] = 0.0f;
+    }
+    lds_barrier();
 
     // Forward substitution (I + A) X = [diag(beta) V | diag(beta*gamma) K]
     // in 16-row blocks on fp32 MFMA: X_i = T_ii (B_i - sum_{j<i} A_ij X_j),
     // T_ii = (I + A_ii)^-1.  The four T_ii come first, by substitution
     // (threads 0..63: column tid % 16 of block tid / 16), and replace the
-    // diagonal blocks of A.  Wave w then owns the 16-column tiles w, w + 4,
-    // ... of X as MFMA accumulators (lane (g, r): rows 4g .. 4g+3 of each
+    // diagonal blocks of A.  Each wave then holds its 16-column tiles of X
+    // as MFMA accumulators (lane (g, r): rows 4g .. 4g+3 of each
     // block, column r); in the products the contraction over the 16 rows of
     // X_j runs in the order the accumulators hold them (step e takes row
     // 4g + e from lane group g, against A_ij[m][4g + e]), so X stays in
     // registers.  The column-per-thread substitution this replaces read
     // every A row through LDS in every thread (11.5 us of a ~32 us
     // workgroup).
-    constexpr int CTW = 2 * D / 64;  // 16-column tiles per wave
     {
         const int bi = tid >> 4, cc = tid & 15;
-        float tc[16];
-        if (tid < 64) {
+        if (wave == 0) {
+            float tc[16];
 #pragma unroll
             for (int m = 0; m < 16; ++m) {
                 float acc = m == cc ? 1.0f : 0.0f;
@@ -485,10 +525,14 @@ __global__ __launch_bounds__(256, 2) void gdn_prep_kernel(GdnArgs a)
                 for (int k = 0; k < m; ++k) acc = fmaf(-Am[16 * bi + m][16 * bi + k], tc[k], acc);
                 tc[m] = acc;
             }
-        } else {
-            // meanwhile the other three waves write P as bf16 hi / lo in the
-            // chain kernel's register order (ChunkWs)
-            for (int e = tid - 64; e < 4 * 2 * 64; e += 192) {
+            // only this wave reads the diagonal blocks of A, and its reads are ahead of these stores
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int m = 0; m < 16; ++m) Am[16 * bi + m][16 * bi + cc] = tc[m];
+        } else if (wave >= 4) {
+            // meanwhile waves 4-7 write P as bf16 hi / lo in the chain kernel's
+            // register order (ChunkWs)
+            for (int e = tid - 256; e < 4 * 2 * 64; e += 256) {
                 const int l = e % 64, ws_ = e / 64, sk = ws_ % 2, wt = ws_ / 2;
                 const int t = 16 * wt + (l & 15), s = 16 * (l >> 4) + 8 * sk;
                 const f32x4 x0 = *reinterpret_cast<const f32x4*>(&Pm[t][s]);
@@ -506,36 +550,19 @@ __global__ __launch_bounds__(256, 2) void gdn_prep_kernel(GdnArgs a)
                 dst[64] = lo;
             }
         }
-        __syncthreads();
-        if (tid < 64) {
-#pragma unroll
-            for (int m = 0; m < 16; ++m) Am[16 * bi + m][16 * bi + cc] = tc[m];
-        }
     }
-    // right-hand sides: tiles ct < CTW / 2 are V columns (tile w + 4 ct < D / 16
-    // for every wave), the rest K columns; rows past the last token have
-    // beta = 0, so their (clamped, valid) V rows contribute nothing
-    f32x4 X[CTW][4];
+    // right-hand sides; rows past the last token have beta = 0
     {
-        const float* vp = a.v + (size_t)h * D;
-#pragma unroll
-        for (int ct = 0; ct < CTW / 2; ++ct)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int t = 16 * i + 4 * g + e;
-                    X[ct][i][e] = vp[(size_t)(t0 + min(t, nt - 1)) * a.v_stride + 16 * (wave + 4 * ct) + r];
-                }
-#pragma unroll
-        for (int ct = CTW / 2; ct < CTW; ++ct)
+        constexpr int KT = CTW - 1;  // the wave's tile of K columns, if it has one
+        if (CTW == 2 || !v_wave) {
 #pragma unroll
             for (int i = 0; i < 4; ++i)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const int t = 16 * i + 4 * g + e;
-                    X[ct][i][e] = sgam[t] * Kn[t][16 * (wave + 4 * ct) + r - D];
+                    X[KT][i][e] = sgam[t] * Kn[t][16 * (wave + 8 * KT) + r - D];
                 }
+        }
 #pragma unroll
         for (int ct = 0; ct < CTW; ++ct)
 #pragma unroll
@@ -543,7 +570,7 @@ __global__ __launch_bounds__(256, 2) void gdn_prep_kernel(GdnArgs a)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) X[ct][i][e] *= sb[16 * i + 4 * g + e];
     }
-    __syncthreads();  // T_ii in place
+    lds_barrier();  // T_ii in place
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
@@ -564,22 +591,23 @@ __global__ __launch_bounds__(256, 2) void gdn_prep_kernel(GdnArgs a)
         }
     }
     // U^T rows (the V columns): four consecutive tokens per lane
-#pragma unroll
-    for (int ct = 0; ct < CTW / 2; ++ct)
+    if (v_wave) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-            *reinterpret_cast<f32x4*>(w.U + (size_t)(16 * (wave + 4 * ct) + r) * kC + 16 * i + 4 * g) = X[ct][i];
+            *reinterpret_cast<f32x4*>(w.U + (size_t)(16 * wave + r) * kC + 16 * i + 4 * g) = X[0][i];
+    }
     // -W through LDS (A is dead once every wave has read it)
-    __syncthreads();
-#pragma unroll
-    for (int ct = CTW / 2; ct < CTW; ++ct)
+    lds_barrier();
+    if (CTW == 2 || !v_wave) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) QA[(16 * i + 4 * g + e) * KP + 16 * (wave + 4 * ct) + r - D] = -X[ct][i][e];
-    __syncthreads();
+            for (int e = 0; e < 4; ++e)
+                QA[(16 * i + 4 * g + e) * KP + 16 * (wave + 8 * (CTW - 1)) + r - D] = -X[CTW - 1][i][e];
+    }
+    lds_barrier();
     // -W as bf16 in the chain kernel's register order (ChunkWs)
-    for (int e = tid; e < 4 * (D / 32) * 64; e += 256) {
+    for (int e = tid; e < 4 * (D / 32) * 64; e += NTH) {
         const int l = e % 64, ws_ = e / 64, sk = ws_ % (D / 32), wt = ws_ / (D / 32);
         const float* src = QA + (16 * wt + (l & 15)) * KP + (l >> 4) * (D / 4) + 8 * sk;
         float x[8];
@@ -996,7 +1024,7 @@ hipError_t launch_gdn_d(const GdnArgs& a, hipStream_t st)
     if (a.T == 1) {
         hipLaunchKernelGGL(gdn_step_kernel<D>, dim3(a.n_v * (D / 16)), dim3(256), 0, st, a);
     } else if (a.ws) {
-        hipLaunchKernelGGL(gdn_prep_kernel<D>, dim3(a.n_chunks, a.n_v), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(gdn_prep_kernel<D>, dim3(a.n_chunks, a.n_v), dim3(512), 0, st, a);
         // two workgroups per state slice when they fit the GPU and the state
         // goes out of place (in place, one part's final state could reach S
         // before the other part has read it)
