@@ -669,6 +669,12 @@ def _prefill_f64(q, cache, start, nh, gate=None):
     (14, 2, 64, 1500, 0, "f16", "f32", False),
     (14, 2, 64, 700, 3000, "f32", "f32", False),
     (28, 4, 128, 700, 0, "f32", "f32", False),
+    # whole groups to the XCDs with a remainder (3, 7 splits of 4 kv heads), split items dealt evenly (3 and 4 splits)
+    (28, 4, 128, 64, 512, "f16", "f32", False),
+    (28, 4, 128, 128, 1536, "bf16", "f32", False),
+    (28, 4, 128, 600, 1000, "f16", "f32", False),
+    (14, 2, 64, 600, 1000, "f16", "f32", True),
+    (16, 2, 256, 400, 1500, "bf16", "f32", True),
     # fp32 queries on two key groups: lo parts in LDS, several items per workgroup, a group without tiles, split walks
     (32, 8, 128, 1100, 0, "f32", "f32", False),
     (40, 5, 128, 1000, 30, "f32", "f16", True),

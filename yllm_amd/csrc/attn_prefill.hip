@@ -278,37 +278,37 @@ __device__ inline bool plain_item(const PrefillArgs& a, uint32_t nqb, uint32_t i
 
 // The split mode's item of this workgroup; false where the grid has none.  The
 // items of a (kv head, split) tile group read the same K/V tiles, so they should
-// share an XCD's L2 (consecutive workgroups go to the 8 XCDs in turn).  With a
-// multiple of 8 groups XCD x serves groups x, x+8, ...  Otherwise whole groups
-// would leave XCDs idle (2 kv heads without a split: six of eight; 1800 tokens
-// of 16 / 2 heads of 256 took 195 us), so each XCD takes an eighth of the items
-// in group order; within a group the order deals the row blocks out evenly, so
-// that every run of it holds heavy and light ones.
+// share an XCD's L2 (consecutive workgroups go to the 8 XCDs in turn): XCD x
+// serves groups x, x+8, ... where no XCD gets more of them than it has CUs for
+// (split_grid; 64 tokens at 512 in three splits, 28 / 4 heads of 128: 12.6 us,
+// dealt evenly 13.2; 128 tokens at 1536 in seven: 16.7 and 17.4).  Otherwise
+// whole groups leave XCDs idle while others queue (2 kv heads without a split:
+// six of eight; 1800 tokens of 16 / 2 heads of 256 took 195 us), so each XCD
+// takes an eighth of the items in group order; within a group the order deals
+// the row blocks out evenly, so that every run of it holds heavy and light ones.
 __device__ inline bool split_item(const PrefillArgs& a, PItem& I)
 {
     const uint32_t x = blockIdx.x % 8u, j = blockIdx.x / 8u;
     const uint32_t ipg = a.n_rb * (a.pack ? 1u : a.gmax), groups = a.n_kv * a.n_split;
-    uint32_t tg, w;
-    if (groups % 8u == 0) {
-        tg = (j / ipg) * 8u + x;
-        w = j % ipg;
-    } else {
-        const uint32_t per = gridDim.x / 8u, i = x * per + j;
-        if (i >= groups * ipg) return false;
-        tg = i / ipg;
-        w = i - tg * ipg;
-        if (!a.pack) {
-            // position w of the group's order: the items 0 mod 8 first, then 1 mod 8, ... (packed rows walk the
-            // same keys)
-            const uint32_t len = ipg / 8u, rem = ipg % 8u;
-            const bool lead = w < rem * (len + 1u);  // the first `rem` residues have one item more
-            const uint32_t r1 = lead ? w : w - rem * (len + 1u), l1 = lead ? len + 1u : len, q = r1 / l1;
-            w = (lead ? 0u : rem) + q + 8u * (r1 - q * l1);
-        }
-    }
+    // both orders share their divisions: a second set cost 0.1 us of a 15 us launch
+    const bool whole = a.xcd_map;
+    const uint32_t i = whole ? j : x * ((groups * ipg + 7u) / 8u) + j, gi = i / ipg;
+    const uint32_t tg = whole ? gi * 8u + x : gi;
     if (tg >= groups) return false;
-    I.kvh = tg % a.n_kv;
-    I.split = tg / a.n_kv;
+    uint32_t w = i - gi * ipg;
+    const uint32_t den = whole ? a.n_kv : a.n_split, hi = tg / den, lo = tg - hi * den;
+    I.kvh = whole ? lo : hi;
+    // dealt items: a kv head's splits follow each other, first, last, second, last but one: the later ones are cut
+    // by the causal edge (600 tokens at 1000 in three, 14 / 2 heads of 64: 17.5 us, 18.3 in split order)
+    I.split = whole ? hi : lo % 2u ? a.n_split - 1u - lo / 2u : lo / 2u;
+    if (!whole && !a.pack) {
+        // position w of the group's order: the items 0 mod 8 first, then 1 mod 8, ... (packed rows walk the
+        // same keys)
+        const uint32_t len = ipg / 8u, rem = ipg % 8u;
+        const bool lead = w < rem * (len + 1u);  // the first `rem` residues have one item more
+        const uint32_t r1 = lead ? w : w - rem * (len + 1u), l1 = lead ? len + 1u : len, q = r1 / l1;
+        w = (lead ? 0u : rem) + q + 8u * (r1 - q * l1);
+    }
     const uint32_t h0 = head0(a, I.kvh), h1 = head0(a, I.kvh + 1);
     if (a.pack) {
         I.qb = w;
@@ -1496,12 +1496,20 @@ hipError_t launch_prefill_halves(PrefillArgs a, hipStream_t st)
     return hipGetLastError();
 }
 
-template <int D, bool QS>
-hipError_t launch_prefill_split_d(const PrefillArgs& a, hipStream_t st)
+// The split mode's order (split_item) and grid: whole tile groups to XCDs
+// where the fullest XCD still has a CU for each of its items.
+uint32_t split_grid(PrefillArgs& a)
 {
-    const uint32_t ipg = a.n_rb * (a.pack ? 1u : a.gmax);
-    const uint32_t groups = a.n_kv * a.n_split;
-    const uint32_t grid = (groups * ipg + 7u) / 8u * 8u;  // split_item's order over 8 XCDs
+    const uint32_t ipg = a.n_rb * (a.pack ? 1u : a.gmax), groups = a.n_kv * a.n_split;
+    const uint32_t most = (groups + 7u) / 8u * ipg;
+    a.xcd_map = groups % 8u == 0 || most <= (uint32_t)n_cus() / 8u;
+    return a.xcd_map ? most * 8u : (groups * ipg + 7u) / 8u * 8u;
+}
+
+template <int D, bool QS>
+hipError_t launch_prefill_split_d(PrefillArgs a, hipStream_t st)
+{
+    const uint32_t grid = split_grid(a);
     bool halves = false;
     if constexpr (D > 128 && !QS) {
         halves = split_halves(a.D, a.q_dtype, a.split_tiles);
