@@ -608,7 +608,7 @@ def run_gated_prefill(L: int, nh: int, nkv: int, hd: int, steps: int, warmup: in
                                f"epilogue, bf16 out; N(0,1)*0.5 seed {hex(seed)}; {n_sets} rotating input sets "
                                f"(> 256 MB MALL)",
                    "tokens": L, "n_heads": nh, "n_kv_heads": nkv, "head_dim": hd},
-        "roofline": {"bound": "mfma", "kernel": "prefill_kernel<%d>" % hd, "achieved": achieved / 1e12,
+        "roofline": {"bound": "mfma", "kernel": "prefill_halves_kernel<%d>" % hd, "achieved": achieved / 1e12,
                      "peak": MFMA_F16_PEAK / 1e12, "unit": "TFLOP/s", "frac": achieved / MFMA_F16_PEAK,
                      "flops_per_launch": flops, "launch_ms": kern_ms, "traffic": traffic_of(f"gated{L}")},
     }
@@ -659,8 +659,7 @@ def run_oproj(B: int, hidden: int, qdim: int, steps: int, warmup: int, cpu: bool
                 "traffic": traffic_of(f"oproj{B}")}
         value, unit = nbytes / (ms * 1e-3) / 1e9, "GB/s"
     else:
-        roof = {"bound": "mfma", "kernel": ("oproj_gemm_kernel<%d,%d>" % ((2, 4) if B > 128 else (1, 1))) +
-                ("" if att_dt == torch.float16 else " (+ oproj_split_kernel)"),
+        roof = {"bound": "mfma", "kernel": "oproj_gemm_kernel<4,4>" if B > 64 else "oproj_rows_kernel<4>",
                 "achieved": flops / (kern_ms * 1e-3) / 1e12, "peak": MFMA_F16_PEAK / 1e12, "unit": "TFLOP/s",
                 "frac": flops / (kern_ms * 1e-3) / MFMA_F16_PEAK, "flops_per_launch": flops, "launch_ms": kern_ms,
                 "traffic": traffic_of(f"oproj{B}")}

@@ -626,22 +626,24 @@ __global__ __launch_bounds__(512, 4) void gdn_prep_kernel(GdnArgs a)
 
 // The recurrence across chunks with each chunk's output: per chunk,
 // Delta = U - W M^T, O = (Q~ M^T + P Delta) / sqrt(d) and then
-// M <- gamma_last M + Delta^T K~.  A workgroup of four waves owns J = 16
+// M <- gamma_last M + Delta^T K~.  A workgroup of eight waves owns J = 16
 // state rows (d_v indices j0..j0+15) of one head, walks the chunks in order
-// and writes the output columns j0..j0+15.  Both output products reuse
-// operands the recurrence already holds: Q~ M^T has phase A's state
-// operands (B) and P Delta has phase B's Delta^T operands; only Q~ and P
-// rows are extra loads.  (A separate output pass over all chunks needed the
+// and writes the output columns j0..j0+15.  Waves 0-3 run the recurrence and
+// waves 4-7 the outputs, whose products take the state and Delta the
+// recurrence leaves in LDS: Q~ M^T beside phase A, P Delta beside phase B.
+// With both on the same four waves the output products and half of the loads
+// stood in the chunk's serial path (4096 tokens, 16 heads: chain 86 us, 70
+// on eight waves).  (A separate output pass over all chunks needed the
 // chunk's starting state and Delta recorded in the workspace: 96 KB written
 // and read again per chunk and head, and a third launch.)
 //
 // Every operand element of a chunk is read by exactly one wave, so each wave
 // loads its own straight into registers, two chunks ahead (three register
-// sets): phase A, wave w forms the Delta tile of tokens 16w..16w+15 from -W
+// sets): phase A, recurrence wave w forms the Delta tile of tokens 16w..16w+15 from -W
 // rows (its A operand), the U^T slice (the accumulator's start) and the state
 // rows in LDS (B); phase B, wave w updates the state tiles of d_k blocks
-// w D/64 .. (kept in its registers in fp32) from Delta^T in LDS (A) and K~
-// (B).  Only the state slice and the Delta tile pass through LDS, as bf16
+// w D/64 .. (kept in its registers in fp32, transposed) from K~ (A) and
+// Delta^T in LDS (B).  Only the state slice and the Delta tile pass through LDS, as bf16
 // hi / lo pairs; two barriers per chunk.  The products are split-bf16
 // (mfma_x3: three bf16 MFMAs per product, fp32 accumulation; the state,
 // Delta and the outputs themselves stay fp32), except that -W enters rounded
@@ -654,12 +656,15 @@ __global__ __launch_bounds__(512, 4) void gdn_prep_kernel(GdnArgs a)
 //
 // An output tile (16 tokens x the 16 columns) is two halves summed in fp32:
 // half 0 is Q~ M^T over the first D/2 of d_k plus P Delta over the first
-// k-step of the chunk's tokens, half 1 the rest.  PARTS = 1: wave w forms
-// both halves of token tile w.  PARTS = 2 (two workgroups per slice, both
+// k-step of the chunk's tokens, half 1 the rest.  PARTS = 1: output wave w
+// forms both halves of token tile w.  PARTS = 2 (two workgroups per slice, both
 // running the recurrence): part p writes token tiles 2p and 2p + 1, wave w
-// forms half w / 2 of tile 2p + w % 2, and the two halves meet in LDS.  The
-// chain is bound by the bytes each CU loads per chunk (the -W, K~ and U^T
-// operands 52 KB, the Q~ and P rows 48 KB); with two parts a CU loads 76 KB.
+// forms half w / 2 of tile 2p + w % 2, and the two halves meet in LDS.  A
+// CU loads 100 KB per chunk (the -W, K~ and U^T operands 52 KB, the Q~ and P
+// rows 48 KB), 76 KB with two parts.  What bounds the chain is the serial path
+// of a chunk, 1.1 us: the LDS reads of the state and Delta by eight waves
+// (~580 cycles), 14 dependent MFMAs, two barriers; with every load left out
+// 49 of the 70 us stay.
 // Both forms give the same bits.
 template <int D, int PARTS>
 __global__ __launch_bounds__(512) void gdn_chain_kernel(GdnArgs a)
