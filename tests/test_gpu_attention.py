@@ -708,3 +708,27 @@ def test_prefill_plan_and_halves_edges(cuda, nh, nkv, d, T, start, qdt, odt, gat
     rows = float(((got - want).norm(dim=1) / want.norm(dim=1)).max())
     print(f"prefill {nh}/{nkv} d={d} {T}@{start} {qdt}->{odt}: rel_l2 {err:.2e}, worst row {rows:.2e}")
     assert err <= 1e-3 + add and rows <= 3e-3 + add
+
+
+@pytest.mark.parametrize("nh,nkv,d,T,start,gated", [
+    (28, 4, 128, 64, 1984, False),   # the engine's call on a prefix: packed rows
+    (28, 4, 128, 400, 2000, True),   # query blocks
+    (14, 2, 64, 40, 5000, False),
+])
+def test_prefill_f32_split_repeats_exactly(cuda, nh, nkv, d, T, start, gated):
+    """fp32 queries, keys split over two key groups and several ranges: each
+    row's (max, sum) of a range is stored once, so calls repeat bit for bit."""
+    from yllm_amd.attention import LayerKV, attn_prefill, kv_store, prefill_workspace_bytes
+
+    g = torch.Generator(device="cuda").manual_seed(T + start)
+    n = start + T
+    cache = LayerKV.empty(nkv, d, n, device=cuda)
+    kv_store(cache, torch.randn(n, nkv * d, generator=g, device=cuda).half(),
+             torch.randn(n, nkv * d, generator=g, device=cuda).half(), 0)
+    q = torch.randn(T, nh * d, generator=g, device=cuda) * 1.5
+    gate = torch.randn(T, nh * d, generator=g, device=cuda) if gated else None
+    ws = torch.empty(prefill_workspace_bytes(T, n, nh, nkv, d), dtype=torch.uint8, device=cuda)
+    assert ws.numel() > 0
+    first = attn_prefill(q, cache, start, nh, gate=gate, workspace=ws)
+    for _ in range(30):
+        assert torch.equal(attn_prefill(q, cache, start, nh, gate=gate, workspace=ws), first)

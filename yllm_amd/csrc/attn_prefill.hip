@@ -920,7 +920,9 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
                 // split partials: (max, sum) and the unnormalised O of this
                 // row over this split's keys
                 const size_t pr = ((size_t)cur.split * a.n_heads + rw.h) * a.B + rw.b;
-                if ((lane_e >> 5) == 0 && hf_e == 0) {
+                // (one key group's sum: the groups round l differently, and two
+                // stores to one slot in no order would leave either)
+                if ((lane_e >> 5) == 0 && hf_e == 0 && grp == 0) {
                     typedef float f32x2 __attribute__((ext_vector_type(2)));
                     *reinterpret_cast<f32x2*>(a.part_ml + 2 * pr) = f32x2{m, l};
                 }
