@@ -732,3 +732,30 @@ def test_prefill_f32_split_repeats_exactly(cuda, nh, nkv, d, T, start, gated):
     first = attn_prefill(q, cache, start, nh, gate=gate, workspace=ws)
     for _ in range(30):
         assert torch.equal(attn_prefill(q, cache, start, nh, gate=gate, workspace=ws), first)
+
+
+@pytest.mark.parametrize("T,start", [(4096, 0), (300, 1500), (1000, 0), (64, 0)])
+def test_prefill_d256_gate_precision(cuda, T, start):
+    """The gate of every d 256 kernel of 16-bit queries (query blocks, merge,
+    unsplit, pair mode) is an fp32 sigmoid.  With q = 0 and V = 1 the attention
+    output is 1 up to two roundings (every probability and their sums are
+    exact: n < 2^24), so the result shows the gate's own error: expf within
+    2 ulp, the sum, the divide and the product, 2^-24 each and doubled where
+    the next binade starts: under 8 x 2^-24 relative."""
+    from yllm_amd.attention import LayerKV, attn_prefill, kv_store
+
+    nh, nkv, d, n = 16, 2, 256, start + T
+    g = torch.Generator(device="cuda").manual_seed(T)
+    cache = LayerKV.empty(nkv, d, n, device=cuda)
+    kv_store(cache, torch.randn(n, nkv * d, generator=g, device=cuda).half(),
+             torch.ones(n, nkv * d, device=cuda).half(), 0)
+    q = torch.zeros(T, nh * d, dtype=torch.bfloat16, device=cuda)
+    gate = torch.empty(T, nh * d, device=cuda).uniform_(-60.0, 60.0, generator=g)
+    gate[:, ::7] = torch.randn(T, (nh * d + 6) // 7, generator=g, device=cuda)
+    for i, x in enumerate((float("inf"), -float("inf"), 0.0, 40.0, -40.0, 87.0, -87.0, 200.0, -200.0)):
+        gate[:, 16 * i + 5] = x
+    got = attn_prefill(q, cache, start, nh, gate=gate).double()
+    want = gate.double().sigmoid()
+    rel = ((got - want).abs() / want.clamp_min(2.0 ** -126)).max()
+    print(f"gate {T}@{start}: {float(rel):.2e}")
+    assert float(rel) <= 8 * 2.0 ** -24

@@ -975,8 +975,10 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
 // half of the dimensions of O over all 64 keys.  Split by dimensions on both
 // sides (prefill_kernel's pair mode, which keeps f32 queries), the waves exchange fp32 partial scores and both form every
 // probability: 1.75 KB of LDS traffic per MFMA against 1.38, and twice the exp2.
-// 4096 tokens, 16 / 2 heads, bf16, gated: 215 -> 166 us (825 TFLOP/s), ungated
-// 188 -> 153.
+// 4096 tokens, 16 / 2 heads, bf16, gated: 215 -> 170 us (808 TFLOP/s), ungated
+// 188 -> 153.  (The gate is the fp32 sigmoid of the other kernels; by the
+// approximate reciprocal of 1 + exp2 it took 6 us less and was up to 3.5e-6
+// off at gates of -60, 2.3e-7 now.)
 //
 // Step t starts with the raw scores of tile t in registers and their maxima
 // in LDS.  The next tile's score MFMAs begin; the pair's common maximum is
@@ -1330,8 +1332,7 @@ __global__ __launch_bounds__(512) void prefill_halves_kernel(PrefillArgs a)
                     f32x4 v = area[(8 * u + er) * 8 + (ec ^ er)];
                     if (gated) {
 #pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            v[e] *= __builtin_amdgcn_rcpf(1.0f + fast_exp2(gt[b & 1][u][e] * -1.4426950408889634f));
+                        for (int e = 0; e < 4; ++e) v[e] *= sigmoid_ref(gt[b & 1][u][e]);
                     }
                     if (!valid[u]) continue;
                     if (partial) *reinterpret_cast<f32x4*>(a.part_o + at[u] + 32 * b) = v;
