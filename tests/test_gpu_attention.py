@@ -759,3 +759,34 @@ def test_prefill_d256_gate_precision(cuda, T, start):
     rel = ((got - want).abs() / want.clamp_min(2.0 ** -126)).max()
     print(f"gate {T}@{start}: {float(rel):.2e}")
     assert float(rel) <= 8 * 2.0 ** -24
+
+
+@pytest.mark.parametrize("qdt", ["bf16", "f32"])
+@pytest.mark.parametrize("T,start,keys", [
+    (4096, 0, (40, 2040, 4090)),      # query blocks
+    (300, 1504, (1515, 1570, 1790)),  # split ranges, unpacked rows
+    (64, 16000, (16040,)),            # packed rows
+])
+def test_prefill_d256_later_value_stays_out(cuda, qdt, T, start, keys):
+    """A value row that is not finite (an fp32 value past f16's range is stored
+    as inf) reaches no query of the 32-row blocks before its own 32 keys: a
+    masked key's probability is 0, but 0 x inf in the output product is not."""
+    from yllm_amd.attention import LayerKV, attn_prefill, kv_store
+
+    nh, nkv, d, n = 16, 2, 256, start + T
+    g = torch.Generator(device="cuda").manual_seed(T)
+    cache = LayerKV.empty(nkv, d, n, device=cuda)
+    k = torch.randn(n, nkv * d, generator=g, device=cuda).half()
+    v = torch.randn(n, nkv * d, generator=g, device=cuda)
+    q = torch.randn(T, nh * d, generator=g, device=cuda)
+    q = q if qdt == "f32" else q.bfloat16()
+    kv_store(cache, k.float(), v, 0)
+    clean = attn_prefill(q, cache, start, nh)
+    for key in keys:
+        bad = v.clone()
+        bad[key] = 1e6
+        kv_store(cache, k.float(), bad, 0)
+        got = attn_prefill(q, cache, start, nh)
+        rows = max(0, key // 32 * 32 - start)
+        assert torch.equal(got[:rows], clean[:rows]), (key, int((got[:rows] != clean[:rows]).any(1).nonzero()[0, 0]))
+        assert not got[key - start:].isfinite().any()

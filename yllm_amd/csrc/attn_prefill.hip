@@ -1122,6 +1122,14 @@ __global__ __launch_bounds__(512) void prefill_halves_kernel(PrefillArgs a)
 #pragma unroll
             for (int i = 0; i < 16; ++i) o[b][i] = 0.0f;
 
+        // In a pair's last tile the upper 32 keys can lie past all its queries: their P is 0 but their V need not be
+        // finite (an inf of a later key would reach these rows as NaN), so their products read the lower keys' V.
+        // Leaves vo like that: nothing follows that tile.
+        auto upper_v = [&](uint32_t st) {
+            if ((int)(st * BN) + 32 <= wpos_last) return;  // uniform over the wave
+#pragma unroll
+            for (int s = 0; s < 2; ++s) vo[0][s] = vo[1][s] = hf ? vo[1][s] : vo[0][s];
+        };
         // mask the wave's keys of tile st past the lanes' positions, form their maximum and publish it
         auto tile_max = [&](f32x16& S, uint32_t st) {
             const int k0 = (int)st * BN + 32 * hf;
@@ -1191,6 +1199,7 @@ __global__ __launch_bounds__(512) void prefill_halves_kernel(PrefillArgs a)
             for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(ko[j]));
 #pragma unroll
             for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(vo[j >> 1][j & 1]));
+            upper_v(st);
             f16x8 pf[2];
             if (st < wsteps) {
                 const float other = Ml[wave ^ 1][lane];
@@ -1232,6 +1241,7 @@ __global__ __launch_bounds__(512) void prefill_halves_kernel(PrefillArgs a)
                 issue_k(nxt);
                 if (ph == 1) dma_v(nxt.kvh, 0, 0, 0);
             }
+            upper_v(st);
             if (p0 / BN + ntiles == kmax / BN + 1 && (kmax + 1) % BN != 0) {  // uniform
                 zero_v_tail(ph);
                 lds_barrier();
