@@ -307,3 +307,14 @@ def test_prefill_plan_fits_its_workspace(hiplib):
                         assert rc == -5, (nh, nkv, d, B, end, start, dt, rc, hiplib.yhip_last_error())
                         n += 1
     assert n > 1000
+
+
+def test_building_and_binding_need_no_torch(hiplib):
+    """The C library builds and binds where torch is not installed."""
+    import subprocess
+    import sys
+
+    code = ("import sys; sys.modules['torch'] = None; import yllm_amd, yllm_amd.build; "
+            "assert yllm_amd.build.sources(); print(yllm_amd.lib().yhip_version().decode())")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert r.returncode == 0 and "gfx950" in r.stdout, r.stderr

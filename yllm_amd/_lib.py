@@ -9,8 +9,6 @@ import ctypes
 from ctypes import POINTER, c_char_p, c_float, c_int, c_size_t, c_uint16, c_uint32, c_uint64, c_void_p
 from pathlib import Path
 
-import torch
-
 LIB_PATH = Path(__file__).resolve().parent / "libyllm_hip.so"
 
 F16, F32, BF16 = 0, 1, 2
@@ -71,6 +69,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_C = None  # torch._C
 
 
 class YhipError(RuntimeError):
@@ -100,8 +99,13 @@ def current_stream() -> int:
     """The raw handle of torch's current stream on the current device: what
     torch.cuda.current_stream().cuda_stream gives, without the Stream object
     (2.7 us of a small operator's ~9 us call; 0.15 us this way).  For callers
-    that hold GPU tensors: torch has set up its GPU state then."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    that hold GPU tensors: torch has set up its GPU state then, and this module
+    does without torch until the first call, for those who only build or bind
+    the library."""
+    global _C
+    if _C is None:
+        from torch import _C
+    return _C._cuda_getCurrentRawStream(_C._cuda_getDevice())
 
 
 def check(rc: int) -> None:
