@@ -790,3 +790,39 @@ def test_prefill_d256_later_value_stays_out(cuda, qdt, T, start, keys):
         rows = max(0, key // 32 * 32 - start)
         assert torch.equal(got[:rows], clean[:rows]), (key, int((got[:rows] != clean[:rows]).any(1).nonzero()[0, 0]))
         assert not got[key - start:].isfinite().any()
+
+
+def test_prefill_forced_key_groups_reach_f32_queries(cuda):
+    """YHIP_PREFILL_NG, read once per process, selects the key groups of fp32
+    queries too, in both modes: one and two groups sum in different orders, so
+    their outputs differ in some bits and both stay at the usual bound."""
+    import os
+    import subprocess
+    import sys
+    from pathlib import Path
+
+    code = """
+import hashlib, sys, torch
+sys.path.insert(0, "tests")
+from test_gpu_attention import _prefill_f64
+from yllm_amd.attention import LayerKV, attn_prefill, kv_store
+for nh, nkv, d, T, start in ((32, 8, 128, 1100, 0), (28, 4, 128, 64, 1984), (14, 2, 64, 40, 5000)):
+    g = torch.Generator(device="cuda").manual_seed(T)
+    n = start + T
+    cache = LayerKV.empty(nkv, d, n)
+    kv_store(cache, torch.randn(n, nkv * d, generator=g, device="cuda").half(),
+             torch.randn(n, nkv * d, generator=g, device="cuda").half(), 0)
+    q = torch.randn(T, nh * d, generator=g, device="cuda")
+    got = attn_prefill(q, cache, start, nh)
+    want = _prefill_f64(q, cache, start, nh)
+    assert float((got.double() - want).norm() / want.norm()) <= 1e-3
+    print(hashlib.sha256(got.cpu().numpy().tobytes()).hexdigest())
+"""
+    root = Path(__file__).resolve().parent.parent
+    out = {}
+    for ng in ("1", "2"):
+        env = dict(os.environ, YHIP_PREFILL_NG=ng, PYTHONPATH=f"{root}:{root / 'oracle'}")
+        r = subprocess.run([sys.executable, "-c", code], cwd=root, env=env, capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0, r.stderr
+        out[ng] = r.stdout.split()
+    assert len(out["1"]) == 3 and all(a != b for a, b in zip(out["1"], out["2"]))

@@ -1452,6 +1452,26 @@ uint32_t xcd_mapped(const PrefillArgs& a)
            ((uint64_t)nqb * (a.n_heads / a.n_kv)) % (8 / a.n_kv) == 0;
 }
 
+// YHIP_PREFILL_PERSIST=0/1 forces resident workgroups off / on, YHIP_PREFILL_NG
+// =1/2 the key groups of head_dim 64 and 128, for comparisons (-1, 0: unset).
+int forced_persist()
+{
+    static const int env = [] {
+        const char* e = getenv("YHIP_PREFILL_PERSIST");
+        return e ? atoi(e) : -1;
+    }();
+    return env;
+}
+int forced_groups()
+{
+    static const int env = [] {
+        const char* e = getenv("YHIP_PREFILL_NG");
+        const int n = e ? atoi(e) : 0;
+        return n == 1 || n == 2 ? n : 0;
+    }();
+    return env;
+}
+
 template <int D, int NG, bool QS>
 hipError_t launch_prefill_d(PrefillArgs a, hipStream_t st)
 {
@@ -1471,11 +1491,8 @@ hipError_t launch_prefill_d(PrefillArgs a, hipStream_t st)
     // a workgroup's start and end (2048 tokens x 28 heads: 57.1 -> 55.7 us);
     // with two 4-wave workgroups per CU the hardware's own dispatch of the
     // next workgroup already overlaps them and is about 1 % faster (8192
-    // tokens).  YHIP_PREFILL_PERSIST=0/1 forces the choice for comparisons.
-    static const int persist = [] {
-        const char* e = getenv("YHIP_PREFILL_PERSIST");
-        return e ? atoi(e) : -1;
-    }();
+    // tokens).
+    const int persist = forced_persist();
     uint32_t grid = items;
     if (persist > 0 || (persist < 0 && prefill_threads(D, NG) > 256)) {
         const uint64_t slots = (uint64_t)per_cu * (uint64_t)n_cus();
@@ -1503,7 +1520,7 @@ hipError_t launch_prefill_halves(PrefillArgs a, hipStream_t st)
 {
     a.xcd_map = xcd_mapped(a);
     const uint32_t items = (a.B + BM - 1) / BM * a.n_heads;
-    uint32_t grid = items < (uint32_t)n_cus() ? items : (uint32_t)n_cus();
+    uint32_t grid = items < (uint32_t)n_cus() || forced_persist() == 0 ? items : (uint32_t)n_cus();
     if (a.xcd_map && grid >= 8u) grid = grid / 8u * 8u;  // whole XCD groups (items are a multiple of 8)
     hipLaunchKernelGGL((prefill_halves_kernel<256, false>), dim3(grid), dim3(512), 0, st, a);
     return hipGetLastError();
@@ -1533,7 +1550,8 @@ hipError_t launch_prefill_split_d(PrefillArgs a, hipStream_t st)
         // fp32 queries: two key groups from four tiles per split on (28 / 4 heads of 128, us with one / two: 64
         // tokens at 0 10.2 / 12.0, at 1000 20.3 / 19.6, at 16000 47 / 40, 400 at 2000 57 / 49); at d 64, where a CU
         // holds two workgroups of one group, only while the grid leaves it at one (400 at 2000 22.4 / 26.7)
-        two = a.split_tiles >= 4 && (D == 128 || grid <= (uint32_t)n_cus());
+        two = forced_groups() ? forced_groups() == 2
+                              : a.split_tiles >= 4 && (D == 128 || grid <= (uint32_t)n_cus());
         if (two) hipLaunchKernelGGL((prefill_kernel<D, 2, true, QS>), dim3(grid), dim3(prefill_threads(D, 2)), 0, st, a);
     }
     if (!halves && !two)
@@ -1551,16 +1569,12 @@ hipError_t launch_prefill_split_d(PrefillArgs a, hipStream_t st)
 // with many workgroups per CU two independent 4-wave workgroups hide latency
 // better than one 8-wave workgroup under one barrier (8192 tokens: 888 vs
 // 790 TFLOP/s).  Two groups need the LDS of two groups' tiles (head_dim <=
-// 128).  YHIP_PREFILL_NG=1/2 forces the choice for comparisons.
+// 128).
 int prefill_groups(const PrefillArgs& a)
 {
-    static const int env = [] {
-        const char* e = getenv("YHIP_PREFILL_NG");
-        return e ? atoi(e) : 0;
-    }();
     const int n_cu = n_cus();
     if (a.D > 128) return 1;
-    if (env == 1 || env == 2) return env;
+    if (forced_groups()) return forced_groups();
     const uint64_t wgs = (uint64_t)((a.B + BM - 1) / BM) * a.n_heads;
     // fp32 queries: at d 128 always two (one group alone, 352 registers, is one
     // wave per SIMD: 28 / 4 heads, 2048 tokens 80 -> 68 us, 6000 478 -> 410); at
@@ -1719,7 +1733,7 @@ hipError_t launch_prefill(const PrefillArgs& a, hipStream_t st)
         return qs ? (ng == 2 ? launch_prefill_d<64, 2, true>(a, st) : launch_prefill_d<64, 1, true>(a, st))
                   : ng == 2 ? launch_prefill_d<64, 2, false>(a, st) : launch_prefill_d<64, 1, false>(a, st);
     case 128:
-        return qs ? launch_prefill_d<128, 2, true>(a, st)
+        return qs ? (ng == 2 ? launch_prefill_d<128, 2, true>(a, st) : launch_prefill_d<128, 1, true>(a, st))
                   : ng == 2 ? launch_prefill_d<128, 2, false>(a, st) : launch_prefill_d<128, 1, false>(a, st);
     case 256: return qs ? launch_prefill_d<256, 1, true>(a, st) : launch_prefill_halves(a, st);
     default: return hipErrorInvalidValue;
