@@ -88,6 +88,7 @@ def test_o_proj_f16_attention_output(cuda, oracle, B):
 @pytest.mark.parametrize("att16", [False, True], ids=["f32att", "f16att"])
 @pytest.mark.parametrize("B,hidden,qdim", [
     (3, 40, 72), (5, 1000, 904), (8, 56, 4200),  # rows kernel, f32 products up to 8 f32 tokens
+    (3, 300, 3072), (4, 300, 904), (5, 4096, 72), (6, 333, 72), (7, 5000, 136),  # where it starts, by size and dtype
     (16, 896, 896), (17, 40, 264), (33, 1000, 4104), (63, 48, 4200),  # rows kernel: 16-token blocks, ragged K, two rounds
     (65, 300, 72), (250, 1100, 40),       # 64 x 64 tiles, fewer K steps than LDS stages
     (520, 1540, 360),                     # 64 x 128 tiles (f16 too), partial in both directions

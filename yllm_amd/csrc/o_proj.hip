@@ -4,8 +4,8 @@
 //
 // W_o is [hidden][qdim] (f16 or f32), att [B][qdim] f32 (or f16 when the
 // attention kernel wrote f16; f16 att takes f16 weights), x [B][hidden] f32.
-//  * Few tokens (decode, B <= kGemvRows; with f16 weights up to 2 f16 or 4 f32
-//    tokens): oproj_gemv_kernel reads W_o once from HBM and applies it to all
+//  * Few tokens (decode, B <= kGemvRows; with f16 weights fewer than rows_from):
+//    oproj_gemv_kernel reads W_o once from HBM and applies it to all
 //    B rows; activations stay f32 and every
 //    product and sum is f32 (the reference's arithmetic, summed in another
 //    order).  A wave owns kRows output rows; its lanes take 8 consecutive
@@ -675,6 +675,26 @@ hipError_t launch_rows(const OProjArgs& a, hipStream_t st)
     return hipGetLastError();
 }
 
+// The fewest tokens that take the rows kernel instead of the one-pass kernel
+// (f16 weights; kGemvRows at most).  It reads each token row once per 16 output
+// rows, the other once per two, but starts slower (a ring and a reduction in
+// LDS), and as one workgroup per CU, so that a part-filled last round costs a
+// whole one.  us one-pass / rows, weights from HBM (in the caches the one-pass
+// kernel is up to 10 % better at these edges): f16 3 tokens 4096 x 4096 13.7 /
+// 9.6, 2048 x 4096 10.4 / 8.7, 1024 x 2048 6.5 / 6.2 (in the caches 5.4 / 6.3),
+// 896 x 896 4.8 / 4.8 (4.4 / 5.0), 8192 x 8192 29.7 / 30.9; 4 tokens 896 x 896
+// 5.5 / 5.0, 8192 x 8192 36.0 / 31.3; 320 or 384 workgroups: 5120 x 5120 4
+// tokens 22.7 / 23.2, 6 26.1 / 23.1.  f32 5 tokens 4096 x 4096 16.1 / 13.2,
+// 11008 x 4096 36.2 / 28.8, 1536 x 1536 7.1 / 7.7, 5120 x 5120 21.1 / 28.0; 6
+// tokens 896 x 896 6.6 / 5.8, 5120 x 5120 24.3 / 28.4, 7 29.0 / 28.7.
+uint32_t rows_from(uint32_t hidden, uint32_t qdim, bool att_f16)
+{
+    const uint32_t wgs = (hidden + 15) / 16, cus = (uint32_t)n_cus(), rounds = (wgs + cus - 1) / cus;
+    const bool one = rounds == 1, full = (uint64_t)wgs * 20 >= (uint64_t)rounds * cus * 17;
+    if (att_f16) return one && qdim >= 3072 ? 3u : one || full ? 4u : 6u;
+    return full ? 5u : one ? 6u : 7u;
+}
+
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
 }  // namespace
@@ -692,11 +712,7 @@ const char* launch_oproj(const OProjArgs& a, void* ws, size_t ws_bytes, hipStrea
     const bool near = 256ull * 4 * (a.att_stride > a.qdim ? a.att_stride : a.qdim) < 0xf0000000ull;
     if (a.B <= kGemvRows) {
         hipError_t e;
-        // f16 weights, from 3 f16 or 5 f32 tokens on: the rows kernel reads each token row once per 16 output rows, the
-        // one-pass kernel once per two (4096 x 4096, us one-pass / rows: f16 2 tokens 11.8 / 10.2, 3 13.6 / 10.2, 8 22.4 /
-        // 10.9; f32 4 14.4 / 13.8, 5 15.8 / 13.9, 8 19.6 / 14.2; 896 x 896 f16 2 4.0 / 4.5, 3 4.8 / 4.6, f32 4 5.1 / 5.4,
-        // 5 6.0 / 5.4)
-        if (a.w_f16 && a.B >= (a.att_f16 ? 3u : 5u) && near) {
+        if (a.w_f16 && a.B >= rows_from(a.hidden, a.qdim, a.att_f16) && near) {
             const dim3 grid((a.hidden + 15) / 16);
             if (a.att_f16) hipLaunchKernelGGL((oproj_rows_kernel<1, false>), grid, dim3(512), 0, st, a);
             else hipLaunchKernelGGL((oproj_rows_kernel<1, true, true>), grid, dim3(512), 0, st, a);
