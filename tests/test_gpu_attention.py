@@ -682,6 +682,13 @@ def _prefill_f64(q, cache, start, nh, gate=None):
     (14, 2, 64, 2500, 0, "f32", "bf16", False),
     (28, 4, 128, 64, 3000, "f32", "f32", True),
     (14, 2, 64, 40, 5000, "f32", "f32", False),
+    # short ranges over two rounds of workgroups (one group), two ranges of one round, few and many query blocks at d 64
+    (32, 32, 128, 64, 4000, "f32", "f32", False),
+    (28, 4, 128, 400, 2000, "f32", "f32", True),
+    (40, 5, 64, 1000, 3, "f32", "f32", False),
+    (40, 5, 64, 1100, 3, "f32", "f32", True),
+    # 16-bit d 256: packed rows that do not fill a workgroup, in ranges of eight tiles
+    (8, 8, 256, 33, 4000, "bf16", "f32", True),
     (15, 3, 128, 140, 900, "bf16", "f32", False),
     (5, 5, 64, 70, 800, "f16", "f32", True),
 ])

@@ -1505,14 +1505,18 @@ hipError_t launch_prefill_d(PrefillArgs a, hipStream_t st)
 }
 
 // The split mode at head_dim 256 with 16-bit queries: walks of up to four
-// 32-key tiles stay with prefill_kernel, whose first scores need half the
-// bytes and MFMAs (16 / 2 heads, us with it / with prefill_halves_kernel: 64
-// tokens at 0 12.0 / 14.2, 33 at 100 15.6 / 18.5, four tiles each at 1984 23.0 /
-// 23.2); longer ones are shorter in the other (64 tokens at 16000 54 / 45, 1000
-// at 4000 215 / 98).
-bool split_halves(uint32_t D, uint32_t q_dtype, uint32_t split_tiles)
+// 32-key tiles (eight where packed rows do not fill a workgroup, so that idle
+// waves leave the other kernel's shorter steps uncovered) stay with
+// prefill_kernel, whose first scores need half the bytes and MFMAs (16 / 2
+// heads, us with it / with prefill_halves_kernel: 64 tokens at 0 12.0 / 14.2,
+// 33 at 100 15.6 / 18.5, four tiles each at 1984 23.0 / 23.2; 8 / 8 heads, 33
+// tokens at 4000 in eight 18.4 / 19.8); longer ones are shorter in the other
+// (64 tokens at 4000 in eight 27.6 / 26.1, at 16000 54 / 45, 1000 at 4000 215 /
+// 98).
+bool split_halves(const PrefillArgs& a)
 {
-    return D > 128 && q_dtype != kF32 && split_tiles > 4;
+    const uint32_t most = a.pack && a.gmax * a.B < (uint32_t)BM ? 8u : 4u;
+    return a.D > 128 && a.q_dtype != kF32 && a.split_tiles > most;
 }
 
 // one workgroup per CU walking the items in snake order
@@ -1542,16 +1546,17 @@ hipError_t launch_prefill_split_d(PrefillArgs a, hipStream_t st)
     const uint32_t grid = split_grid(a);
     bool halves = false;
     if constexpr (D > 128 && !QS) {
-        halves = split_halves(a.D, a.q_dtype, a.split_tiles);
+        halves = split_halves(a);
         if (halves) hipLaunchKernelGGL((prefill_halves_kernel<D, true>), dim3(grid), dim3(512), 0, st, a);
     }
     bool two = false;
     if constexpr (D <= 128 && QS) {
         // fp32 queries: two key groups from four tiles per split on (28 / 4 heads of 128, us with one / two: 64
-        // tokens at 0 10.2 / 12.0, at 1000 20.3 / 19.6, at 16000 47 / 40, 400 at 2000 57 / 49); at d 64, where a CU
-        // holds two workgroups of one group, only while the grid leaves it at one (400 at 2000 22.4 / 26.7)
+        // tokens at 0 10.2 / 12.0, at 1000 20.3 / 19.6, at 16000 47 / 40), six where the workgroups go round twice
+        // (32 / 32 heads, 64 tokens at 4000 in four 36.1 / 38.3); at d 64, where a CU holds two workgroups of one
+        // group, only while the grid leaves it at one (400 at 2000 22.4 / 26.7)
         two = forced_groups() ? forced_groups() == 2
-                              : a.split_tiles >= 4 && (D == 128 || grid <= (uint32_t)n_cus());
+                              : grid <= (uint32_t)n_cus() ? a.split_tiles >= 4 : D == 128 && a.split_tiles >= 6;
         if (two) hipLaunchKernelGGL((prefill_kernel<D, 2, true, QS>), dim3(grid), dim3(prefill_threads(D, 2)), 0, st, a);
     }
     if (!halves && !two)
@@ -1579,8 +1584,13 @@ int prefill_groups(const PrefillArgs& a)
     // fp32 queries: at d 128 always two (one group alone, 352 registers, is one
     // wave per SIMD: 28 / 4 heads, 2048 tokens 80 -> 68 us, 6000 478 -> 410); at
     // d 64 one workgroup per CU or less gains nothing from it (14 / 2 heads, 1500
-    // tokens 29.7 / 30.3, 3000 59 -> 44, 6000 130 either way)
-    if (a.q_dtype == kF32) return a.D == 128 || (wgs > (uint64_t)n_cu && wgs <= 2 * (uint64_t)n_cu) ? 2 : 1;
+    // tokens 29.7 / 30.3, 3000 59 -> 44, 6000 130 either way), nor do heads of
+    // few query blocks, which two workgroups per CU balance better (64 / 8 heads,
+    // 635 tokens at 500 27.9 -> 30.6, 800 19.8 -> 22.5; 32 / 8, 1147 25.3 -> 21.3)
+    if (a.q_dtype == kF32) {
+        const bool pays = wgs > (uint64_t)n_cu && wgs <= 2 * (uint64_t)n_cu && a.B > 8u * (uint32_t)BM;
+        return a.D == 128 || pays ? 2 : 1;
+    }
     return wgs <= 2 * (uint64_t)n_cu ? 2 : 1;
 }
 
@@ -1653,18 +1663,22 @@ size_t prefill_plan(PrefillArgs& a)
     const uint32_t by_tiles = (ntiles + t.min_tiles - 1) / t.min_tiles;
     if (most > by_tiles) most = by_tiles;
     // Of up to `most` splits, the number with the least cost: the walk of the
-    // longest split (us per 64 keys, half again as long with two workgroups on
-    // a CU) and, from two on, the merge launch and the partials written and
-    // read (1.4 us, 5 TB/s; 28 / 4 heads of 128, f16: 1000 tokens 25.6 us
-    // unsplit, 34.4 in two; f32 38 and 55; 64 tokens at 1984 16 us in eight;
-    // 2 tokens at 300 11.8 unsplit, 9.7 in two).
-    const float per64 = (0.35f + (float)a.D / 160.0f) * (a.q_dtype == kF32 ? 1.6f : 1.0f);
+    // longest split (us per 64 keys; past one workgroup per CU half again as
+    // long where a CU holds two, twice where it holds one: fp32 queries at
+    // head_dim 128) and, from two on, the merge launch and the partials written
+    // and read (1.4 us, 5 TB/s; 28 / 4 heads of 128, f16: 1000 tokens 25.6 us
+    // unsplit, 34.4 in two; f32 38 and 55, 400 tokens at 2000 49 in four, 42 in
+    // two; 64 tokens at 1984 16 us in eight; 2 tokens at 300 11.8 unsplit, 9.7
+    // in two; 16 / 2 heads of 256, f32: 256 tokens at 512 30.1 in four, 28.0 in six).
+    const bool f32q = a.q_dtype == kF32;
+    const float per64 = !f32q ? 0.35f + (float)a.D / 160.0f : a.D > 128 ? 3.5f : 1.6f * (0.35f + (float)a.D / 160.0f);
+    const float round2 = f32q && a.D == 128 ? 2.0f : 1.5f;
     const float rows_us = (float)a.n_heads * a.B * a.D * 8.0f / 5.0e6f;
     uint64_t S = 1;
     float best = 0.0f;
     for (uint64_t n = 1; n <= most; ++n) {
         const float walk = (float)((ntiles + n - 1) / n * bn_of((int)a.D)) / 64.0f * per64;
-        const float cost = walk * (base * n > (uint64_t)n_cus() ? 1.5f : 1.0f) + (n > 1 ? 1.4f + rows_us * n : 0.0f);
+        const float cost = walk * (base * n > (uint64_t)n_cus() ? round2 : 1.0f) + (n > 1 ? 1.4f + rows_us * n : 0.0f);
         if (n == 1 || cost < best) {
             best = cost;
             S = n;
@@ -1679,7 +1693,7 @@ size_t prefill_plan(PrefillArgs& a)
     }
     a.split_tiles = (ntiles + (uint32_t)S - 1) / (uint32_t)S;
     // prefill_halves_kernel walks pairs of 32-key tiles
-    if (split_halves(a.D, a.q_dtype, a.split_tiles)) a.split_tiles += a.split_tiles & 1u;
+    if (split_halves(a)) a.split_tiles += a.split_tiles & 1u;
     a.n_split = (ntiles + a.split_tiles - 1) / a.split_tiles;
     return split_bytes(a.n_split, a.B, a.n_heads, a.D);
 }
