@@ -85,25 +85,47 @@ def test_o_proj_f16_attention_output(cuda, oracle, B):
     assert err <= TOL
 
 
-@pytest.mark.parametrize("att16", [False, True], ids=["f32att", "f16att"])
-@pytest.mark.parametrize("B,hidden,qdim", [
-    (3, 40, 72), (5, 1000, 904), (8, 56, 4200),  # rows kernel, f32 products up to 8 f32 tokens
-    (3, 300, 3072), (4, 300, 904), (5, 4096, 72), (6, 333, 72), (7, 5000, 136),  # where it starts, by size and dtype
+def gemm_tile(B, hidden, kind):
+    """The tile launch_gemm takes for B tokens: the largest of its list of which
+    there are three quarters of the CUs, else the last."""
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    tiles = {"f16": [(256, 256), (128, 256), (128, 128), (64, 128), (64, 64)],
+             "f32": [(128, 256), (64, 128), (64, 64)],
+             "w32": [(128, 128), (64, 64)]}[kind]
+    for bt, bo in tiles[:-1]:
+        if -(-B // bt) * -(-hidden // bo) >= cus * 3 // 4:
+            return bt, bo
+    return tiles[-1]
+
+
+# B, hidden, qdim and, past the rows kernel, the tile of f32 / f16 att (f16 weights)
+EDGES = [
+    (3, 40, 72), (5, 1000, 904), (8, 56, 4200),  # one-pass or rows kernel, f32 products up to 8 f32 tokens
+    (3, 300, 3072), (4, 300, 904), (5, 4096, 72), (6, 333, 72), (7, 5000, 136),  # where the rows kernel starts
     (16, 896, 896), (17, 40, 264), (33, 1000, 4104), (63, 48, 4200),  # rows kernel: 16-token blocks, ragged K, two rounds
-    (65, 300, 72), (250, 1100, 40),       # 64 x 64 tiles, fewer K steps than LDS stages
-    (520, 1540, 360),                     # 64 x 128 tiles (f16 too), partial in both directions
-    (1030, 3100, 136),                    # 128 x 128 (f16) / 64 x 128 (f32) tiles
-    (2050, 3330, 200),                    # 128 x 256 tiles
-    (3600, 4000, 104),                    # 256 x 256 tiles (f16)
-])
-def test_o_proj_tile_edges(cuda, B, hidden, qdim, att16):
-    """Every kernel and tile of the dispatch at sizes that leave partial tiles,
-    partial K steps and a K shorter than the pipeline, against float64.  Bound:
+    (65, 300, 72, (64, 64), (64, 64)), (250, 1100, 40, (64, 64), (64, 64)),  # fewer K steps than LDS stages
+    (520, 1540, 360, (64, 64), (64, 64)),      # partial in both directions, as all below
+    (520, 2900, 72, (64, 128), (64, 128)),
+    (1030, 3100, 136, (64, 128), (128, 128)),
+    (2050, 3330, 200, (128, 256), (128, 256)),
+    (3600, 4000, 104, (128, 256), (256, 256)),
+]
+
+
+@pytest.mark.parametrize("att16", [False, True], ids=["f32att", "f16att"])
+@pytest.mark.parametrize("B,hidden,qdim,tile", [(*e[:3], e[3:]) for e in EDGES],
+                         ids=["-".join(map(str, e[:3])) for e in EDGES])
+def test_o_proj_tile_edges(cuda, B, hidden, qdim, tile, att16):
+    """Every kernel and tile of the dispatch of f16 weights at sizes that leave
+    partial tiles, partial K steps and a K shorter than the pipeline, against
+    float64.  Bound:
     qdim products of |w att| accumulate in fp32 (each addition within 2^-24 of
     the running sum) and the split of f32 att leaves 2^-22 of each product, so
     the error stays under (qdim 2^-24 + 2^-22) sum |w att| + 2^-23 |x|."""
     from yllm_amd.attention import o_proj
 
+    if B > 64:
+        assert gemm_tile(B, hidden, "f16" if att16 else "f32") == tile[att16]
     g = torch.Generator(device="cuda").manual_seed(B)
     att = torch.randn(B, qdim, generator=g, device=cuda) * 0.5
     att = att.half() if att16 else att
@@ -113,6 +135,32 @@ def test_o_proj_tile_edges(cuda, B, hidden, qdim, att16):
     o_proj(x[:, :hidden], att, w)
     want = x0[:, :hidden].double() + att.double() @ w.double().t()
     bound = (qdim * 2.0 ** -24 + 2.0 ** -22) * (att.double().abs() @ w.double().abs().t()) \
+        + 2.0 ** -23 * want.abs() + 2.0 ** -23 * x0[:, :hidden].double().abs()
+    assert ((x[:, :hidden].double() - want).abs() <= bound).all()
+    assert torch.equal(x[:, hidden:], x0[:, hidden:])
+
+
+@pytest.mark.parametrize("B,hidden,qdim,tile", [
+    (9, 40, 72, (64, 64)), (64, 300, 1032, (64, 64)), (300, 1100, 40, (64, 64)),
+    (1800, 1700, 40, (128, 128)), (1800, 1700, 328, (128, 128)),  # fewer K steps than stages, a ragged last one
+    (2048, 2048, 256, (128, 128)),                                # whole tiles only
+])
+def test_o_proj_f32_weight_tiles(cuda, B, hidden, qdim, tile):
+    """Both tiles of f32 weights against float64.  Three products per pair (hi
+    hi, lo hi, hi lo), so 3 qdim additions in fp32, and 2^-22 each of att's
+    split, w's and the dropped lo lo: under (3 qdim 2^-24 + 3 2^-22) sum
+    |w att| + 2^-23 |x|."""
+    from yllm_amd.attention import o_proj
+
+    assert gemm_tile(B, hidden, "w32") == tile
+    g = torch.Generator(device="cuda").manual_seed(B + qdim)
+    att = torch.randn(B, qdim, generator=g, device=cuda) * 0.5
+    w = torch.randn(hidden, qdim, generator=g, device=cuda) * qdim ** -0.5
+    x0 = torch.randn(B, hidden + 8, generator=g, device=cuda)
+    x = x0.clone()
+    o_proj(x[:, :hidden], att, w)
+    want = x0[:, :hidden].double() + att.double() @ w.double().t()
+    bound = (3 * qdim * 2.0 ** -24 + 3 * 2.0 ** -22) * (att.double().abs() @ w.double().abs().t()) \
         + 2.0 ** -23 * want.abs() + 2.0 ** -23 * x0[:, :hidden].double().abs()
     assert ((x[:, :hidden].double() - want).abs() <= bound).all()
     assert torch.equal(x[:, hidden:], x0[:, hidden:])
