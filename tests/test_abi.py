@@ -318,3 +318,22 @@ def test_building_and_binding_need_no_torch(hiplib):
             "assert yllm_amd.build.sources(); print(yllm_amd.lib().yhip_version().decode())")
     r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
     assert r.returncode == 0 and "gfx950" in r.stdout, r.stderr
+
+
+def test_host_workspace_never_reaches_the_gpu(hiplib, monkeypatch):
+    """A workspace in host memory, too short for the sizes the call is planned
+    for but long enough for the call itself, is replaced like any short one."""
+    import torch
+
+    from yllm_amd import attention as A
+
+    host = torch.empty(4096, dtype=torch.uint8)
+    seen = []
+
+    def fn(ws, have, stream):
+        seen.append(ws)
+        return 0 if have >= 1024 else -28  # the call needs 1024 bytes, the bound is 8192
+
+    monkeypatch.setattr(A, "_stream", lambda: 0)
+    A._with_workspace(fn, (), host, lambda: 8192, torch.device("cpu"))
+    assert seen and host.data_ptr() not in seen
