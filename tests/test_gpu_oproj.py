@@ -1,12 +1,13 @@
 """o_proj on the GPU vs the oracle (engine.c:969-973, matvec.c:98-122).
 
-x[b] += W_o . att[b].  Up to 8 tokens the GEMV kernel keeps every product
-and sum in f32 (the reference's arithmetic in another order); more tokens go
-through the MFMA GEMM with f16 weights times the f16 hi + lo parts of f32 att
-(about 22 bits of each activation), f16 weights times f16 att (the attention
-kernel's f16 output) or, for f32 weights, the hi + lo parts of both.  Either way the
-result must be within relative L2 1e-5 of the f32 oracle (the stated bar is
-1e-3), on the updated x and on the product alone.
+x[b] += W_o . att[b].  Up to 8 tokens every product and sum is in f32 (the
+reference's arithmetic in another order), in the one-pass kernel or the rows
+kernel; more tokens go through the rows kernel or the MFMA GEMM with f16
+weights times the f16 hi + lo parts of f32 att (about 22 bits of each
+activation), f16 weights times f16 att (the attention kernel's f16 output) or,
+for f32 weights, the hi + lo parts of both.  Either way the result must be
+within relative L2 1e-5 of the f32 oracle (the stated bar is 1e-3), on the
+updated x and on the product alone.
 """
 from __future__ import annotations
 
@@ -39,15 +40,15 @@ def to_dev(cuda, w):
 @pytest.mark.parametrize("B,hidden,qdim,f16", [
     (1, 896, 896, True),      # decode, the 0.5B shape (14 heads x 64)
     (3, 4096, 4096, True),
-    (8, 2048, 4096, True),    # the largest GEMV batch
+    (8, 2048, 4096, True),    # the largest batch with f32 products
     (1, 1000, 512, False),    # f32 weights, a hidden size that is no multiple of the rows per wave
-    (9, 896, 896, True),      # the smallest GEMM batch
+    (9, 896, 896, True),      # the smallest batch with split products
     (64, 4096, 4096, True),
     (300, 2048, 4096, True),
     (77, 1024, 2048, False),  # f32 GEMM
-    (200, 4096, 4096, True),  # 256 x 256 tiles, a partial token tile
+    (200, 4096, 4096, True),  # 64 x 64 tiles, a partial token tile
     (200, 1000, 904, False),  # f32 weights; hidden and qdim no multiples of the tiles or of 64
-    (130, 520, 1032, True),   # the smallest 256-token tile config, ragged edges
+    (130, 520, 1032, True),   # ragged edges
     (64, 333, 904, True),     # the engine's 64-token chunk, ragged edges
 ])
 def test_o_proj_matches_oracle(cuda, oracle, B, hidden, qdim, f16):
@@ -69,8 +70,8 @@ def test_o_proj_matches_oracle(cuda, oracle, B, hidden, qdim, f16):
 
 @pytest.mark.parametrize("B", [1, 6, 200])
 def test_o_proj_f16_attention_output(cuda, oracle, B):
-    """att written as f16 by the attention kernel: the GEMV widens it, the
-    GEMM path runs one f16 GEMM; the oracle sees the same f16 values."""
+    """att written as f16 by the attention kernel: the one-pass kernel widens
+    it, the MFMA kernels take it as it is; the oracle sees the same f16 values."""
     from yllm_amd.attention import o_proj
 
     hidden, qdim = 2048, 4096

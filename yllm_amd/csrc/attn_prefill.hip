@@ -404,7 +404,7 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
     // An item's first loads are issued during the previous item: its
     // group's first K, V and second K tiles in the previous item's last key
     // step, into buffers that step no longer reads (the V tile only after
-    // the step when that step reads V buffer 0), and, for f16 queries, the
+    // the step when that step reads V buffer 0), and, for 16-bit queries, the
     // query fragments after the key loop (registers the key loop reads
     // cannot be loaded inside it without the compiler waiting for them
     // there).  Their latency hides under that step, the merge and the output
@@ -732,10 +732,11 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
         };
 
         // prologue: this item's first loads are in flight (issued above or at the
-        // end of the previous item); bf16 queries are converted here, f32 ones loaded
-        // and split (prefetched like the others they spilled: 2048 tokens 63 -> 79 us).  All loads are complete before the key loop, whose
-        // waits then count only tile loads (in pair mode K(2) and V(1) may
-        // still be in flight; the first step waits for them).
+        // end of the previous item); bf16 queries are converted here, f32 ones
+        // loaded and split (prefetched like the others they spilled: 2048 tokens 63
+        // -> 79 us).  All loads are complete before the key loop, whose waits then
+        // count only tile loads (in pair mode K(2) and V(1) may still be in
+        // flight; the first step waits for them).
         dma_wait_but(deep_loads);
         if (QL && it > 0) lds_barrier();  // the merge has read (max, sum)
         if constexpr (QS) {
@@ -973,8 +974,9 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
 // dimensions (Q in 64 registers), turns them into probabilities, hands the
 // 2 KB of f16 probabilities to its partner through LDS and accumulates its
 // half of the dimensions of O over all 64 keys.  Split by dimensions on both
-// sides (prefill_kernel's pair mode, which keeps f32 queries), the waves exchange fp32 partial scores and both form every
-// probability: 1.75 KB of LDS traffic per MFMA against 1.38, and twice the exp2.
+// sides (prefill_kernel's pair mode, which keeps f32 queries), the waves
+// exchange fp32 partial scores and both form every probability: 1.75 KB of LDS
+// traffic per MFMA against 1.38, and twice the exp2.
 // 4096 tokens, 16 / 2 heads, bf16, gated: 215 -> 170 us (808 TFLOP/s), ungated
 // 188 -> 153.  (The gate is the fp32 sigmoid of the other kernels; by the
 // approximate reciprocal of 1 + exp2 it took 6 us less and was up to 3.5e-6
@@ -986,8 +988,8 @@ __global__ __launch_bounds__(256 * NG * (D > 128 ? 2 : 1), (NG == 1 && D <= 128 
 // between the rest of the score MFMAs and then to LDS; the output MFMAs of the
 // wave's own 32 keys follow; a barrier; those of the partner's keys, under
 // which the next tile's maximum is formed; a barrier.  K is loaded two tiles
-// ahead, V one, straight into LDS, and an item's first tiles and queries during
-// the previous item's last step.
+// ahead, V one, straight into LDS, and an item's first K and V tiles during the
+// previous item's last step.
 template <int D, bool SPLIT>
 __global__ __launch_bounds__(512) void prefill_halves_kernel(PrefillArgs a)
 {
@@ -996,7 +998,7 @@ __global__ __launch_bounds__(512) void prefill_halves_kernel(PrefillArgs a)
     constexpr int NKK = D / 16, NDB = DH / 32;
     constexpr int KCH = D / 8, VCH = BN / 8;
     constexpr int CH = BN * D / (8 * 512);  // 16-byte chunks per thread per tile (K and V each)
-        constexpr float kSlack = 8.0f;
+    constexpr float kSlack = 8.0f;
     __shared__ __attribute__((aligned(16))) _Float16 Kl0[BN * D], Kl1[BN * D], Vl0[D * BN], Vl1[D * BN];
     __shared__ f16x8 Pl[8][2][64];  // each wave's probabilities: k-slot, lane
     __shared__ float Ml[8][64];     // each wave's tile maxima, then its row sums

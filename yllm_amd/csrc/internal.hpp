@@ -88,7 +88,7 @@ struct PrefillArgs {
     float c;
     // set by the launcher: the (query block, head) items are grouped by kv
     // head per XCD (xcd_map) and dealt to gridDim.x resident workgroups in
-    // snake order, heaviest first
+    // snake order, heaviest first; in split mode, whole tile groups go to XCDs
     uint32_t xcd_map;
     // Split mode (set by prefill_plan for launches with fewer work items
     // than CUs, e.g. the engine's 64-token chunks over a long prefix): an
@@ -139,9 +139,10 @@ struct OProjArgs {
     uint32_t x_stride, att_stride, B, hidden, qdim, w_f16, att_f16;
 };
 constexpr uint32_t kGemvRows = 8;  // up to this many tokens: f32 products, no workspace asked for
+// bytes yhip_o_proj asks its callers for; no kernel uses them
 size_t oproj_workspace(uint32_t B, uint32_t qdim, uint32_t w_f16, uint32_t att_f16, uint32_t hidden);
 // null on success, else a message
-const char* launch_oproj(const OProjArgs& a, void* ws, size_t ws_bytes, hipStream_t st);
+const char* launch_oproj(const OProjArgs& a, hipStream_t st);
 
 // ---- gdn_conv.hip ----
 struct GdnConvArgs {

@@ -4,14 +4,13 @@
 //
 // W_o is [hidden][qdim] (f16 or f32), att [B][qdim] f32 (or f16 when the
 // attention kernel wrote f16; f16 att takes f16 weights), x [B][hidden] f32.
-//  * Few tokens (decode, B <= kGemvRows; with f16 weights fewer than rows_from):
-//    oproj_gemv_kernel reads W_o once from HBM and applies it to all
-//    B rows; activations stay f32 and every
-//    product and sum is f32 (the reference's arithmetic, summed in another
-//    order).  A wave owns kRows output rows; its lanes take 8 consecutive
-//    inputs each (16-byte weight loads at f16), eight iterations of loads in
-//    flight (all of a 4096-wide row), then a shuffle reduction and the
-//    residual add.
+//  * Few tokens (decode, B <= kGemvRows; with f16 weights fewer than
+//    rows_from): oproj_gemv_kernel reads W_o once from HBM and applies it to
+//    all B rows; activations stay f32 and every product and sum is f32 (the
+//    reference's arithmetic, summed in another order).  A wave owns kRows
+//    output rows; its lanes take 8 consecutive inputs each (16-byte weight
+//    loads at f16), eight iterations of loads in flight (all of a 4096-wide
+//    row), then a shuffle reduction and the residual add.
 //  * Then up to kRowsMax tokens with f16 weights (the engine's 64-token prefill calls):
 //    oproj_rows_kernel streams W_o through MFMA, a workgroup per 16 output
 //    rows and its waves splitting the contraction.
@@ -25,7 +24,6 @@
 // are split the same way and hi.Whi + lo.Whi + hi.Wlo accumulate.
 #include "common.hpp"
 #include "internal.hpp"
-
 
 namespace yhip {
 namespace {
@@ -378,9 +376,10 @@ __global__ __launch_bounds__(512, 1) void oproj_rows_kernel(OProjArgs a)
 // half's MFMAs issue while the next step's first fragments are read and the
 // loads four steps ahead go into the stage just read.  The four stages are
 // separate variables and the loop is unrolled by four, so the compiler sees
-// loads in flight never alias the reads.  f16 8192 x 4096 x 4096 350 -> 265 us
-// (1040 TFLOP/s; 1250 in the loop alone), f32 att 2048 x 3584 x 3584 193 + 15 for
-// the split pass -> 100.
+// loads in flight never alias the reads.  f16 8192 x 4096 x 4096, operands from
+// HBM, 350 -> 291 us (945 TFLOP/s; 1250 in the loop alone; repeated on one set of
+// operands, whose 235 MB the last-level cache holds, 328 -> 265); f32 att 2048 x
+// 3584 x 3584, repeated, 186 with its split pass -> 103.
 struct GemmArgs {
     const char* t;  // token rows
     const char* w;  // W_o rows, ld K
@@ -578,9 +577,9 @@ __global__ __launch_bounds__(256, WPC) void oproj_gemm_kernel(GemmArgs a)
     // x[t][o] += acc.  Whole tiles: the loads of one row of blocks ahead of
     // the adds and stores of the one before, the first row's from before the K
     // loop where they fit (as float atomics the epilogue took three times as
-    // long: 8192 x 4096 x 4096, f16, 312 -> 265 us).  Partial tiles, where each access has its own
-    // bounds test: float atomics, which nothing waits for (one add per element,
-    // so the result is the load, add and store's).
+    // long: 8192 x 4096 x 4096, f16, repeated, 312 -> 265 us).  Partial tiles, where
+    // each access has its own bounds test: float atomics, which nothing waits for
+    // (one add per element, so the result is the load, add and store's).
     if (whole) {
         if (!kEarlyX) load_x(0);
 #pragma unroll
@@ -618,12 +617,15 @@ hipError_t launch_gemm_tiles(const GemmArgs& a, hipStream_t st)
 // Tile choice: the largest tile of which there are enough for three quarters
 // of the CUs.  A larger tile moves fewer LDS and L2 bytes per MFMA, but one
 // workgroup per CU cannot fill a chip of which it leaves a quarter idle.
-// (With the residual still added by atomics) f16 att, 4096 x 4096, us with 256 x
-// 256 / 128 x 256 / 128 x 128 / 64 x 128 / 64 x 64 tiles: 8192 tokens 320 / 359 /
-// 372, 2048 tokens 108 / 96 / 104, 1024 96 / 72 / 55 / 73 / 85, 512 - / 66 / 47 /
-// 43 / 47, 256 - / - / 44 / 39 / 29.  f32 att, 3584 x 3584, 128 x 256 / 64 x 128 /
-// 64 x 64: 2048 tokens 118 / 147, 1024 90 / 76 / 99, 512 85 / 45 / 55, 256 (4096 x
-// 4096) - / 44 / 39.
+// us with each tile, largest first, operands from HBM.  f16 att, 4096 x 4096,
+// 256 x 256 / 128 x 256 / 128 x 128 / 64 x 128 / 64 x 64: 8192 tokens 294 / 341 /
+// 375 / 492 / 608, 2048 122 / 95 / 98 / 139 / 175, 1024 117 / 81 / 57 / 75 / 92, 512
+// 111 / 76 / 50 / 43 / 50, 256 101 / 69 / 48 / 43 / 31.  f32 att, 3584 x 3584, 128 x
+// 256 / 64 x 128 / 64 x 64: 2048 111 / 143 / 171, 1024 89 / 71 / 94, 512 81 / 44 /
+// 53, 256 74 / 38 / 30.  f32 weights, 3584 x 3584, 128 x 128 / 64 x 64: 2048 181 /
+// 233, 1024 93 / 128, 512 78 / 67, 256 73 / 41.  It does not see a part-filled last
+// round: 640 tokens 4096 x 4096 f16 run 60 us as 320 tiles of 64 x 128, 52 as 160 of
+// 128 x 128.
 hipError_t launch_gemm(const GemmArgs& a, bool af32, bool wf32, hipStream_t st)
 {
     const uint64_t enough = (uint64_t)n_cus() * 3 / 4;
@@ -706,7 +708,7 @@ size_t oproj_workspace(uint32_t B, uint32_t qdim, uint32_t w_f16, uint32_t att_f
     return 2 * align256((size_t)B * qdim * 2) + (w_f16 ? 0 : 2 * align256((size_t)hidden * qdim * 2));
 }
 
-const char* launch_oproj(const OProjArgs& a, void* ws, size_t ws_bytes, hipStream_t st)
+const char* launch_oproj(const OProjArgs& a, hipStream_t st)
 {
     // the MFMA kernels address a tile's rows with 32-bit byte offsets
     const bool near = 256ull * 4 * (a.att_stride > a.qdim ? a.att_stride : a.qdim) < 0xf0000000ull;
@@ -725,8 +727,6 @@ const char* launch_oproj(const OProjArgs& a, void* ws, size_t ws_bytes, hipStrea
             e = a.att_f16 ? launch_gemv<0, 1>(a, st) : launch_gemv<0, 0>(a, st);
         return e == hipSuccess ? nullptr : hipGetErrorString(e);
     }
-    (void)ws;
-    (void)ws_bytes;
     // rows too long for the MFMA kernels go through the one-pass kernel, eight tokens at a time
     if (!near) {
         for (uint32_t b0 = 0; b0 < a.B; b0 += kGemvRows) {
@@ -734,7 +734,7 @@ const char* launch_oproj(const OProjArgs& a, void* ws, size_t ws_bytes, hipStrea
             p.B = a.B - b0 < kGemvRows ? a.B - b0 : kGemvRows;
             p.x = a.x + (size_t)b0 * a.x_stride;
             p.att = reinterpret_cast<const char*>(a.att) + (size_t)b0 * a.att_stride * (a.att_f16 ? 2 : 4);
-            if (const char* msg = launch_oproj(p, nullptr, 0, st)) return msg;
+            if (const char* msg = launch_oproj(p, st)) return msg;
         }
         return nullptr;
     }

@@ -84,8 +84,9 @@ __device__ inline void store_q_pair(void* out, size_t o, uint32_t e0, uint32_t e
 // 64).  Each thread's eight 8-byte loads go out together, from clamped, valid
 // rows: one row per trip of a loop with the load under its bounds test was a
 // memory round trip per trip, which launches of up to 700 tokens waited for
-// (28 / 4 heads of 128, 300 tokens: 9.4 us, now 5.8).  The tile is stored transposed in LDS; 8 positions of one channel leave as one
-// 16-byte store where all of them are stored rows and the cache allows it.
+// (28 / 4 heads of 128, 300 tokens: 9.4 us, now 5.8).  The tile is stored
+// transposed in LDS; 8 positions of one channel leave as one 16-byte store
+// where all of them are stored rows and the cache allows it.
 template <int D>
 __device__ void v_tile_block(const RopeArgs& a, uint32_t vb)
 {
