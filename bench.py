@@ -653,13 +653,13 @@ def run_oproj(B: int, hidden: int, qdim: int, steps: int, warmup: int, cpu: bool
     flops = 2.0 * B * hidden * qdim
     nbytes = hidden * qdim * 2.0 + B * qdim * att_size + 2.0 * B * hidden * 4.0
     if gemv:
-        roof = {"bound": "hbm", "kernel": "oproj_gemv_kernel<1,%d>" % (1 if B == 1 else 8),
+        roof = {"bound": "hbm", "kernel": "oproj_gemv_kernel" if B <= 2 else "oproj_gemv_kernel or oproj_rows_kernel",
                 "achieved": nbytes / (kern_ms * 1e-3) / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                 "frac": nbytes / (kern_ms * 1e-3) / HBM_PEAK, "bytes_per_launch": nbytes, "launch_ms": kern_ms,
                 "traffic": traffic_of(f"oproj{B}")}
         value, unit = nbytes / (ms * 1e-3) / 1e9, "GB/s"
     else:
-        roof = {"bound": "mfma", "kernel": "oproj_gemm_kernel<4,4>" if B > 64 else "oproj_rows_kernel<4>",
+        roof = {"bound": "mfma", "kernel": "oproj_gemm_kernel" if B > 64 else "oproj_rows_kernel",
                 "achieved": flops / (kern_ms * 1e-3) / 1e12, "peak": MFMA_F16_PEAK / 1e12, "unit": "TFLOP/s",
                 "frac": flops / (kern_ms * 1e-3) / MFMA_F16_PEAK, "flops_per_launch": flops, "launch_ms": kern_ms,
                 "traffic": traffic_of(f"oproj{B}")}
