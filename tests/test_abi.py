@@ -320,14 +320,24 @@ def test_building_and_binding_need_no_torch(hiplib):
     assert r.returncode == 0 and "gfx950" in r.stdout, r.stderr
 
 
-def test_host_workspace_never_reaches_the_gpu(hiplib, monkeypatch):
-    """A workspace in host memory, too short for the sizes the call is planned
-    for but long enough for the call itself, is replaced like any short one."""
+@pytest.mark.parametrize("where", ["host", "other_gpu"])
+def test_workspace_elsewhere_never_reaches_the_gpu(hiplib, monkeypatch, where):
+    """A workspace in host memory or on another GPU, too short for the sizes
+    the call is planned for but long enough for the call itself, is replaced
+    like any short one."""
     import torch
 
     from yllm_amd import attention as A
 
     host = torch.empty(4096, dtype=torch.uint8)
+    if where == "other_gpu":  # host memory in the place of another device's
+        class Other:
+            is_cuda, device = True, torch.device("cuda", 1)
+            numel, element_size, data_ptr = host.numel, host.element_size, host.data_ptr
+
+        ws = Other()
+    else:
+        ws = host
     seen = []
 
     def fn(ws, have, stream):
@@ -335,5 +345,5 @@ def test_host_workspace_never_reaches_the_gpu(hiplib, monkeypatch):
         return 0 if have >= 1024 else -28  # the call needs 1024 bytes, the bound is 8192
 
     monkeypatch.setattr(A, "_stream", lambda: 0)
-    A._with_workspace(fn, (), host, lambda: 8192, torch.device("cpu"))
+    A._with_workspace(fn, (), ws, lambda: 8192, torch.device("cpu"))
     assert seen and host.data_ptr() not in seen

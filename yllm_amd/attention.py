@@ -211,10 +211,10 @@ def _with_workspace(fn, args: tuple, workspace: torch.Tensor | None, need, devic
     """fn(*args, workspace, its bytes, stream).  A caller's workspace is tried
     as it is, which spares the separate planning call: the library refuses one
     that is too short before it launches anything, and then, as without one,
-    `need()` bytes are allocated.  (One in host memory is not tried: the
-    library cannot tell, and a call may need less than `need()`, which serves
-    every call up to this one's sizes.)"""
-    if workspace is not None and workspace.is_cuda and workspace.numel():
+    `need()` bytes are allocated.  (One in host memory or on another GPU is
+    not tried: the library cannot tell, and a call may need less than
+    `need()`, which serves every call up to this one's sizes.)"""
+    if workspace is not None and workspace.is_cuda and workspace.device == device and workspace.numel():
         have = workspace.numel() * workspace.element_size()
         rc = fn(*args, workspace.data_ptr(), have, _stream())
         if rc != ENOSPC or have >= need():
