@@ -237,8 +237,9 @@ int yhip_rope_kv_store(void* q_out, uint32_t q_out_dtype, uint32_t q_out_stride,
  * f32 (no workspace).  More: f16 MFMA products with f32 accumulation and the
  * residual add fused (f32 att, and f32 weights, enter as f16 hi + lo parts
  * whose products accumulate together: about 22 bits of each operand).  Such
- * calls take yhip_o_proj_workspace bytes (0 for f16 att), room for the parts;
- * the kernels split in registers and leave it untouched.  qdim must be a
+ * calls take yhip_o_proj_workspace bytes (0 for f16 att), used only where f32
+ * att or f32 weights overlap x (x += W_o . x): read from a copy there.  f16
+ * operands, and all of up to 8 tokens, must not overlap x.  qdim must be a
  * multiple of 8; w and att 16-byte aligned with att_stride a multiple of 8
  * elements; hidden * qdim below 2^30. */
 size_t yhip_o_proj_workspace(uint32_t B, uint32_t hidden, uint32_t qdim, uint32_t w_dtype, uint32_t att_dtype);

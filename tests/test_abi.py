@@ -347,3 +347,33 @@ def test_workspace_elsewhere_never_reaches_the_gpu(hiplib, monkeypatch, where):
     monkeypatch.setattr(A, "_stream", lambda: 0)
     A._with_workspace(fn, (), ws, lambda: 8192, torch.device("cpu"))
     assert seen and host.data_ptr() not in seen
+
+
+def test_rows_overlap_against_their_bytes(hiplib):
+    """The test that decides whether o_proj reads an operand from a copy, on
+    random row layouts, against the sets of bytes: never a miss, and exact for
+    column ranges of one matrix of equal heights."""
+    class Rows(ctypes.Structure):
+        _fields_ = [("p", ctypes.c_void_p), ("step", ctypes.c_uint64), ("bytes", ctypes.c_uint64), ("n", ctypes.c_uint64)]
+
+    fn = hiplib._ZN4yhip12rows_overlapERKNS_4RowsES2_
+    fn.restype = ctypes.c_bool
+    rng = np.random.default_rng(3)
+    found = {True: 0, False: 0}
+    for i in range(4000):
+        step, n = int(rng.integers(1, 12)), int(rng.integers(1, 6))
+        a = (64, step, int(rng.integers(1, step + 1)), n)
+        if i % 2:  # columns of the same matrix
+            at = int(rng.integers(0, step))
+            b = (64 + at, step, int(rng.integers(1, step - at + 1)), n)
+        else:
+            step = step if i % 4 else int(rng.integers(1, 12))
+            b = (int(rng.integers(1, 140)), step, int(rng.integers(1, step + 1)), int(rng.integers(1, 6)))
+        sets = [{p + r * st + j for r in range(m) for j in range(w)} for p, st, w, m in (a, b)]
+        meet = bool(sets[0] & sets[1])
+        for x, y in ((a, b), (b, a)):
+            got = fn(ctypes.byref(Rows(*x)), ctypes.byref(Rows(*y)))
+            assert got or not meet, (x, y)
+            assert got == meet or not i % 2, (x, y)
+        found[meet] += 1
+    assert min(found.values()) > 500

@@ -264,3 +264,46 @@ def test_o_proj_after_gated_decode(cuda, oracle):
     err = rel_l2(xt.cpu().numpy(), want)
     print(f"gated decode + o_proj: rel_l2 {err:.2e}")
     assert err <= 1e-3
+
+
+@pytest.mark.parametrize("B", [9, 64, 300])
+@pytest.mark.parametrize("wdt", ["f16", "f32"])
+@pytest.mark.parametrize("how", ["same", "rows", "columns", "beside"])
+def test_o_proj_reads_att_that_overlaps_x(cuda, B, wdt, how):
+    """f32 att that shares memory with x, more than 8 tokens (fewer never
+    allowed it): all of att is read before x changes, so x += W x is what it
+    says.  Same rows, x one row further on, overlapping columns, and columns
+    side by side in one matrix, which share no element.  Bound as in the tile
+    tests: att is split (and f32 w), sums in fp32."""
+    from yllm_amd.attention import o_proj
+
+    n = 520
+    g = torch.Generator(device="cuda").manual_seed(B)
+    w = torch.randn(n, n, generator=g, device=cuda) * n ** -0.5
+    w = w.half() if wdt == "f16" else w
+    m = torch.randn(B + 1, 2 * n, generator=g, device=cuda)
+    att, x = {"same": (m[:B, :n], m[:B, :n]), "rows": (m[:B, :n], m[1:, :n]), "columns": (m[:B, :n], m[:B, 13:n + 13]),
+              "beside": (m[:B, :n], m[:B, n:])}[how]
+    m0, a64, x64 = m.clone(), att.double(), x.double()
+    o_proj(x, att, w)
+    want = x64 + a64 @ w.double().t()
+    bound = (3 * n * 2.0 ** -24 + 3 * 2.0 ** -22) * (a64.abs() @ w.double().abs().t()) + 2.0 ** -23 * (want.abs() + x64.abs())
+    assert ((x.double() - want).abs() <= bound).all()
+    x.copy_(x64)  # nothing else changed
+    assert torch.equal(m, m0)
+
+
+def test_o_proj_reads_weights_that_overlap_x(cuda):
+    """f32 weights that share memory with x: all of them are read before x changes."""
+    from yllm_amd.attention import o_proj
+
+    B, hidden, qdim = 40, 72, 80
+    g = torch.Generator(device="cuda").manual_seed(1)
+    m = torch.randn(64 * 128, generator=g, device=cuda)
+    w, x = m[:hidden * qdim].view(hidden, qdim), m[2048:2048 + B * hidden].view(B, hidden)
+    att = torch.randn(B, qdim, generator=g, device=cuda)
+    w64, x64 = w.double(), x.double()
+    o_proj(x, att, w)
+    want = x64 + att.double() @ w64.t()
+    bound = (3 * qdim * 2.0 ** -24 + 3 * 2.0 ** -22) * (att.double().abs() @ w64.abs().t()) + 2.0 ** -23 * (want.abs() + x64.abs())
+    assert ((x.double() - want).abs() <= bound).all()

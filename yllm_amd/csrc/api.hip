@@ -534,7 +534,7 @@ int yhip_o_proj(float* x, uint32_t x_stride, const void* att, uint32_t att_dtype
     a.qdim = qdim;
     a.w_f16 = w_dtype == YHIP_F16;
     a.att_f16 = att_dtype == YHIP_F16;
-    const char* msg = yhip::launch_oproj(a, (hipStream_t)stream);
+    const char* msg = yhip::launch_oproj(a, need ? workspace : nullptr, (hipStream_t)stream);
     if (msg) return fail(YHIP_EDEVICE, "%s: %s", fn, msg);
     return done(hipSuccess, "");
 }

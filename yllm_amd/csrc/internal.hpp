@@ -139,10 +139,15 @@ struct OProjArgs {
     uint32_t x_stride, att_stride, B, hidden, qdim, w_f16, att_f16;
 };
 constexpr uint32_t kGemvRows = 8;  // up to this many tokens: f32 products, no workspace asked for
-// bytes yhip_o_proj asks its callers for; no kernel uses them
+// n rows of `bytes` bytes, `step` bytes apart (step >= bytes, n >= 1)
+struct Rows {
+    const void* p;
+    uint64_t step, bytes, n;
+};
+bool rows_overlap(const Rows& a, const Rows& b);
 size_t oproj_workspace(uint32_t B, uint32_t qdim, uint32_t w_f16, uint32_t att_f16, uint32_t hidden);
 // null on success, else a message
-const char* launch_oproj(const OProjArgs& a, hipStream_t st);
+const char* launch_oproj(const OProjArgs& a, void* ws, hipStream_t st);
 
 // ---- gdn_conv.hip ----
 struct GdnConvArgs {

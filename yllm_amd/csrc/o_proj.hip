@@ -699,19 +699,68 @@ uint32_t rows_from(uint32_t hidden, uint32_t qdim, bool att_f16)
 
 size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
+// f32 rows of 4 cols4 elements, `stride` elements apart, to a contiguous matrix
+__global__ __launch_bounds__(256) void oproj_copy_kernel(f32x4* dst, const float* src, uint32_t stride, uint32_t cols4,
+                                                         uint64_t n)
+{
+    const uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x;
+    if (i >= n) return;
+    dst[i] = *reinterpret_cast<const f32x4*>(src + i / cols4 * stride + i % cols4 * 4u);
+}
+
+hipError_t copy_rows(void* dst, const void* src, uint32_t stride, uint32_t rows, uint32_t cols, hipStream_t st)
+{
+    const uint64_t n = (uint64_t)rows * (cols / 4);
+    hipLaunchKernelGGL(oproj_copy_kernel, dim3((uint32_t)((n + 255) / 256)), dim3(256), 0, st,
+                       reinterpret_cast<f32x4*>(dst), reinterpret_cast<const float*>(src), stride, cols / 4, n);
+    return hipGetLastError();
+}
+
 }  // namespace
+
+// whether some byte lies both in a row of a and in a row of b
+bool rows_overlap(const Rows& a, const Rows& b)
+{
+    const uint64_t pa = (uint64_t)(uintptr_t)a.p, pb = (uint64_t)(uintptr_t)b.p;
+    if (pa + (a.n - 1) * a.step + a.bytes <= pb || pb + (b.n - 1) * b.step + b.bytes <= pa) return false;
+    if (a.step != b.step) return true;  // (or taken to)
+    // column ranges of one matrix: where b's rows start within a's step
+    const uint64_t d = pb >= pa ? (pb - pa) % a.step : (a.step - (pa - pb) % a.step) % a.step;
+    return d < a.bytes || d + b.bytes > a.step;
+}
 
 size_t oproj_workspace(uint32_t B, uint32_t qdim, uint32_t w_f16, uint32_t att_f16, uint32_t hidden)
 {
     if (B <= kGemvRows || att_f16) return 0;
-    // What callers have had to bring for f32 operands (once their f16 parts); no kernel uses it any more.
+    // Room for a copy of each f32 operand, which a call whose operands overlap x needs (launch_oproj).
     return 2 * align256((size_t)B * qdim * 2) + (w_f16 ? 0 : 2 * align256((size_t)hidden * qdim * 2));
 }
 
-const char* launch_oproj(const OProjArgs& a, hipStream_t st)
+const char* launch_oproj(const OProjArgs& in, void* ws, hipStream_t st)
 {
+    OProjArgs a = in;
     // the MFMA kernels address a tile's rows with 32-bit byte offsets
-    const bool near = 256ull * 4 * (a.att_stride > a.qdim ? a.att_stride : a.qdim) < 0xf0000000ull;
+    auto reach = [&] { return 256ull * 4 * (a.att_stride > a.qdim ? a.att_stride : a.qdim) < 0xf0000000ull; };
+    bool near = reach();
+    // The MFMA kernels read an operand in many workgroups while others already update x.  An f32 operand that
+    // overlaps x (x += W x) is read from a copy; so are rows too far apart, which would take the one-pass kernel.
+    if (a.B > kGemvRows && !a.att_f16 && ws) {
+        const Rows x = {a.x, a.x_stride * 4ull, a.hidden * 4ull, a.B}, row = {a.att, a.att_stride * 4ull, a.qdim * 4ull, a.B},
+                   w = {a.w, a.qdim * 4ull, a.qdim * 4ull, a.hidden};
+        hipError_t e = hipSuccess;
+        if (!a.w_f16 && rows_overlap(x, w)) {
+            char* dst = reinterpret_cast<char*>(ws) + 2 * align256((size_t)a.B * a.qdim * 2);
+            e = copy_rows(dst, a.w, a.qdim, a.hidden, a.qdim, st);
+            a.w = dst;
+        }
+        if (e == hipSuccess && (!near || rows_overlap(x, row))) {
+            e = copy_rows(ws, a.att, a.att_stride, a.B, a.qdim, st);
+            a.att = ws;
+            a.att_stride = a.qdim;
+            near = reach();
+        }
+        if (e != hipSuccess) return hipGetErrorString(e);
+    }
     if (a.B <= kGemvRows) {
         hipError_t e;
         if (a.w_f16 && a.B >= rows_from(a.hidden, a.qdim, a.att_f16) && near) {
@@ -734,7 +783,7 @@ const char* launch_oproj(const OProjArgs& a, hipStream_t st)
             p.B = a.B - b0 < kGemvRows ? a.B - b0 : kGemvRows;
             p.x = a.x + (size_t)b0 * a.x_stride;
             p.att = reinterpret_cast<const char*>(a.att) + (size_t)b0 * a.att_stride * (a.att_f16 ? 2 : 4);
-            if (const char* msg = launch_oproj(p, st)) return msg;
+            if (const char* msg = launch_oproj(p, nullptr, st)) return msg;
         }
         return nullptr;
     }
