@@ -309,6 +309,36 @@ def test_prefill_plan_fits_its_workspace(hiplib):
     assert n > 1000
 
 
+@pytest.mark.parametrize("nh,nkv,d,B,start,dt,splits", [
+    # unsplit, a gate is applied in the few workgroups' epilogues: these are faster in two ranges with one
+    (24, 4, 256, 33, 100, 2, (False, True)),
+    (8, 8, 256, 133, 11, 0, (False, True)),
+    (16, 2, 256, 256, 0, 2, (False, True)),
+    (24, 4, 256, 128, 11, 0, (False, True)),
+    (28, 4, 128, 192, 100, 0, (False, True)),
+    (64, 8, 64, 8, 300, 0, (False, True)),
+    (16, 2, 256, 64, 0, 2, (False, False)),   # too few keys
+    (28, 4, 128, 1000, 0, 0, (False, False)),  # the partials would cost more
+    (28, 4, 128, 64, 1984, 0, (True, True)),
+])
+def test_prefill_plan_counts_the_gate(hiplib, nh, nkv, d, B, start, dt, splits):
+    """Which calls split their keys without and with a gate: one that does
+    refuses a workspace of no bytes.  The bound holds for both."""
+    import torch
+
+    if torch.cuda.is_available():
+        pytest.skip("a GPU would run the launch")
+    p, row = 1 << 20, nh * d
+    ws = hiplib.yhip_attn_prefill_workspace(B, start + B, nh, nkv, d)
+    for gated in (False, True):
+        def call(nbytes):
+            return hiplib.yhip_attn_prefill(p, 1, row, p, dt, row, p, p, start, B, nh, nkv, d, 65536,
+                                            p if gated else None, row, p, nbytes, None)
+
+        assert (call(0) == -28) == splits[gated]
+        assert call(ws) == -5
+
+
 def test_building_and_binding_need_no_torch(hiplib):
     """The C library builds and binds where torch is not installed."""
     import subprocess

@@ -689,6 +689,12 @@ def _prefill_f64(q, cache, start, nh, gate=None):
     (40, 5, 64, 1100, 3, "f32", "f32", True),
     # 16-bit d 256: packed rows that do not fill a workgroup, in ranges of eight tiles
     (8, 8, 256, 33, 4000, "bf16", "f32", True),
+    # gated calls that split for the gate's sake
+    (24, 4, 256, 33, 100, "bf16", "bf16", True),
+    (8, 8, 256, 133, 11, "f16", "f32", True),
+    (24, 4, 256, 128, 11, "f32", "f32", True),
+    (28, 4, 128, 192, 100, "f16", "f16", True),
+    (64, 8, 64, 8, 300, "bf16", "f32", True),
     (15, 3, 128, 140, 900, "bf16", "f32", False),
     (5, 5, 64, 70, 800, "f16", "f32", True),
 ])

@@ -1672,15 +1672,23 @@ size_t prefill_plan(PrefillArgs& a)
     // unsplit, 34.4 in two; f32 38 and 55, 400 tokens at 2000 49 in four, 42 in
     // two; 64 tokens at 1984 16 us in eight; 2 tokens at 300 11.8 unsplit, 9.7
     // in two; 16 / 2 heads of 256, f32: 256 tokens at 512 30.1 in four, 28.0 in six).
+    // An unsplit launch applies the gate in its few workgroups' epilogues (2.9, 5.7
+    // and 5.4 us at head_dim 64, 128 and 256), a split one in the merge's many
+    // (0.2 to 2): what fits the 16-bit walks beside the merge's estimate is 1.3, 2.6
+    // and 3 us (f16, gated, unsplit / in two: 24 / 4 heads of 256, 33 tokens at 100
+    // 22.6 / 15.5; 8 / 8, 133 at 11 22.0 / 16.3; 28 / 4 of 128, 192 at 100 18.3 /
+    // 14.6), for fp32 queries the same 3 at 256 and nothing below, where the walk
+    // is estimated long.
     const bool f32q = a.q_dtype == kF32;
     const float per64 = !f32q ? 0.35f + (float)a.D / 160.0f : a.D > 128 ? 3.5f : 1.6f * (0.35f + (float)a.D / 160.0f);
     const float round2 = f32q && a.D == 128 ? 2.0f : 1.5f;
     const float rows_us = (float)a.n_heads * a.B * a.D * 8.0f / 5.0e6f;
+    const float gate_us = !a.gate || (f32q && a.D <= 128) ? 0.0f : fminf((float)a.D / 50.0f, 3.0f);
     uint64_t S = 1;
     float best = 0.0f;
     for (uint64_t n = 1; n <= most; ++n) {
         const float walk = (float)((ntiles + n - 1) / n * bn_of((int)a.D)) / 64.0f * per64;
-        const float cost = walk * (base * n > (uint64_t)n_cus() ? round2 : 1.0f) + (n > 1 ? 1.4f + rows_us * n : 0.0f);
+        const float cost = walk * (base * n > (uint64_t)n_cus() ? round2 : 1.0f) + (n > 1 ? 1.4f + rows_us * n : gate_us);
         if (n == 1 || cost < best) {
             best = cost;
             S = n;
