@@ -689,6 +689,11 @@ def _prefill_f64(q, cache, start, nh, gate=None):
     (40, 5, 64, 1100, 3, "f32", "f32", True),
     # 16-bit d 256: packed rows that do not fill a workgroup, in ranges of eight tiles
     (8, 8, 256, 33, 4000, "bf16", "f32", True),
+    # 16-bit d 256 in one range of five, seven and eight tiles (packed and not)
+    (24, 4, 256, 133, 11, "f16", "f16", False),
+    (24, 4, 256, 192, 11, "bf16", "f32", False),
+    (32, 4, 256, 192, 50, "f16", "f32", False),
+    (32, 4, 256, 100, 100, "bf16", "bf16", False),
     # gated calls that split for the gate's sake
     (24, 4, 256, 33, 100, "bf16", "bf16", True),
     (8, 8, 256, 133, 11, "f16", "f32", True),

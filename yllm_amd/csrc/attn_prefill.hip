@@ -1507,17 +1507,19 @@ hipError_t launch_prefill_d(PrefillArgs a, hipStream_t st)
 }
 
 // The split mode at head_dim 256 with 16-bit queries: walks of up to four
-// 32-key tiles (eight where packed rows do not fill a workgroup, so that idle
-// waves leave the other kernel's shorter steps uncovered) stay with
-// prefill_kernel, whose first scores need half the bytes and MFMAs (16 / 2
-// heads, us with it / with prefill_halves_kernel: 64 tokens at 0 12.0 / 14.2,
-// 33 at 100 15.6 / 18.5, four tiles each at 1984 23.0 / 23.2; 8 / 8 heads, 33
-// tokens at 4000 in eight 18.4 / 19.8); longer ones are shorter in the other
-// (64 tokens at 4000 in eight 27.6 / 26.1, at 16000 54 / 45, 1000 at 4000 215 /
-// 98).
+// 32-key tiles (seven in one range; eight where packed rows do not fill a
+// workgroup, so that idle waves leave the other kernel's shorter steps
+// uncovered) stay with prefill_kernel, whose first scores need half the bytes
+// and MFMAs and which walks an odd tile alone (16 / 2 heads, us with it / with
+// prefill_halves_kernel: 64 tokens at 0 12.0 / 14.2, 33 at 100 15.6 / 18.5, four
+// tiles each at 1984 23.0 / 23.2; 24 / 4 heads in one range of five tiles, 133
+// at 11 15.8 / 16.9; 8 / 8 heads, 33 tokens at 4000 in eight 18.4 / 19.8); longer
+// ones are shorter in the other (64 tokens at 4000 in eight 27.6 / 26.1, at 16000
+// 54 / 45, 1000 at 4000 215 / 98; 24 / 4 heads in one range of eight, 133 at 100
+// 19.2 / 18.4).  n_split is set.
 bool split_halves(const PrefillArgs& a)
 {
-    const uint32_t most = a.pack && a.gmax * a.B < (uint32_t)BM ? 8u : 4u;
+    const uint32_t most = a.pack && a.gmax * a.B < (uint32_t)BM ? 8u : a.n_split == 1 ? 7u : 4u;
     return a.D > 128 && a.q_dtype != kF32 && a.split_tiles > most;
 }
 
@@ -1702,9 +1704,12 @@ size_t prefill_plan(PrefillArgs& a)
         return 0;
     }
     a.split_tiles = (ntiles + (uint32_t)S - 1) / (uint32_t)S;
-    // prefill_halves_kernel walks pairs of 32-key tiles
-    if (split_halves(a)) a.split_tiles += a.split_tiles & 1u;
     a.n_split = (ntiles + a.split_tiles - 1) / a.split_tiles;
+    // prefill_halves_kernel walks pairs of 32-key tiles (of two ranges or more of five tiles at least, so two remain)
+    if (split_halves(a)) {
+        a.split_tiles += a.split_tiles & 1u;
+        a.n_split = (ntiles + a.split_tiles - 1) / a.split_tiles;
+    }
     return split_bytes(a.n_split, a.B, a.n_heads, a.D);
 }
 
