@@ -184,8 +184,9 @@ def test_o_proj_few_large_tokens(cuda, att16):
 
 @pytest.mark.parametrize("att16", [False, True], ids=["f32att", "f16att"])
 def test_o_proj_rows_too_far_apart_for_a_tile(cuda, att16):
-    """att rows 2^22 elements apart: a tile's 32-bit offsets do not reach, the
-    one-pass kernel takes the tokens eight at a time."""
+    """att rows 2^22 elements apart: a tile's 32-bit offsets do not reach.  f32
+    rows are made contiguous in the workspace, f16 rows (which bring none) go
+    through the one-pass kernel eight tokens at a time."""
     from yllm_amd.attention import o_proj
 
     B, hidden, qdim, stride = 11, 72, 64, 1 << 22
